@@ -233,12 +233,20 @@ class HipDense:
         return matmul(self, other)
 
 
+def _sorted(A):
+    """A with sorted column indices; the caller's matrix keeps its order
+    (csr_matrix(A) shares A's arrays, and a stacked time-dependent generator
+    names its entries' elements by position)."""
+    if A.has_sorted_indices:
+        return A
+    return A.sorted_indices()
+
+
 class HipCSR:
     """CSR matrix in HBM (int32 indices, complex128 or complex64 values)."""
 
     def __init__(self, A, fp32=False):
-        A = sp.csr_matrix(A, dtype=np.complex128)
-        A.sort_indices()
+        A = _sorted(sp.csr_matrix(A, dtype=np.complex128))
         self.shape = A.shape
         self.nnz = int(A.nnz)
         self.fp32 = bool(fp32)
@@ -303,8 +311,7 @@ def sell_arrays(A, lanes=1):
     the column of their own row (clipped to the column count)."""
     if lanes not in (1, 2, 4, 8):
         raise ValueError("lanes must be 1, 2, 4 or 8")
-    A = sp.csr_matrix(A)
-    A.sort_indices()
+    A = _sorted(sp.csr_matrix(A))
     n = A.shape[0]
     C = 64 // lanes
     ns = (n + C - 1) // C
@@ -427,8 +434,7 @@ def sell_coded_arrays(A, lanes=1, fp32=False, uniform="auto", elem=None):
     if lanes not in (1, 2, 4, 8):
         raise ValueError("lanes must be 1, 2, 4 or 8")
     if elem is None:
-        A = sp.csr_matrix(A)
-        A.sort_indices()
+        A = _sorted(sp.csr_matrix(A))
     n = A.shape[0]
     dic = code_dictionary(A, fp32, elem)
     if dic is None:

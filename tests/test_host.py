@@ -384,3 +384,22 @@ def test_stacked_elements_code_ranges():
     for k, m in enumerate(mats):
         vals = set(np.round(vtab[vstart[k]:vstart[k + 1]], 12)) - {0}
         assert vals == set(np.round(m.data, 12)) - {0}
+
+
+def test_operator_layouts_leave_the_matrix_as_it_is():
+    """A stacked time-dependent generator lists its entries element by
+    element; building a layout of it (the lane tuner does, before the engine)
+    must not sort the caller's arrays, whose order the element list follows."""
+    rng = np.random.default_rng(4)
+    mats = [sp.random(40, 40, 0.1, random_state=k, format="csr").astype(complex)
+            for k in range(3)]
+    A, elem = qdata.stacked_elements(mats)
+    before = A.indices.copy(), A.data.copy()
+    assert not A.has_sorted_indices
+    qdata.sell_arrays(A, 2)
+    qdata.sell_coded_arrays(A, 2)
+    assert np.array_equal(A.indices, before[0]) and np.array_equal(A.data, before[1])
+    x = rng.standard_normal(40)
+    for e, M in enumerate(mats):
+        part = sp.csr_matrix((np.where(elem == e, A.data, 0), A.indices, A.indptr), A.shape)
+        assert np.allclose(part @ x, M @ x, atol=1e-14)
