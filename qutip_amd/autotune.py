@@ -1,6 +1,9 @@
 """Autotuners: the SELL-C spmv of the RK stage kernels and the tile shape of
 the matrix-form MFMA kernels.
 
+Operators that the resident step loop takes get their lane count from a rule
+instead (resident_lanes).
+
 The tile shape is the number of lanes per row L (1, 2, 4, 8; C = 64 / L
 rows per wavefront).  Few lanes per row keep the padding low, more lanes per
 row give more wavefronts in flight (latency hiding for the column gathers).
@@ -78,9 +81,39 @@ def measure(A, fp32=False, candidates=CANDIDATES, reps=8, rounds=4, coded=False)
     return best
 
 
+# Lanes the resident step loop takes: 512 threads on each of 256 compute
+# units, and the entries a lane keeps in registers (kResKept).
+RESIDENT_LANES = 512 * 256
+RESIDENT_ENTRIES = 16
+
+
+def resident_lanes(A, coded=False):
+    """Lanes per row for the resident step loop (csrc/rk_resident.hip), or
+    None when A has no shape for it: the fewest that leave at most 16 entries
+    a lane, which it then keeps in registers, and two above 32768 rows, where
+    one would leave half of the lanes unused.  Measured, us per right-hand
+    side at 1 / 2 / 4 lanes: 4096 rows of 13-18 entries 3.3 / 2.6 / 3.1,
+    16384 of 15-21 5.0 / 3.9 / 4.0, 6400 of 7 2.4 / 2.5 / 3.6, 8192 of 14
+    2.6 / 3.0 / 3.8, 65536 of 17 5.4 / 4.7 / -."""
+    if any(os.environ.get(k, "")[:1] == "0" for k in ("QUTIP_AMD_RESIDENT", "QUTIP_AMD_GRAPH")):
+        return None
+    n = A.shape[0]
+    width = int(np.diff(A.indptr).max()) if A.nnz else 0
+    for L in CANDIDATES:
+        per = -(-width // L)
+        if coded:
+            per = -(-per // 4) * 4
+        if n * L <= RESIDENT_LANES and per <= RESIDENT_ENTRIES:
+            return 2 if L == 1 and 32768 < n <= RESIDENT_LANES // 2 else L
+    return None
+
+
 def lanes_for(A, fp32=False, coded=False):
     n = A.shape[0]
     nnz_row = A.nnz / max(n, 1)
+    L = resident_lanes(A, coded)
+    if L is not None:
+        return L
     if n < MIN_TUNE_ROWS or os.environ.get("QUTIP_AMD_NO_TUNE"):
         return heuristic_lanes(nnz_row)
     if not _CACHE:

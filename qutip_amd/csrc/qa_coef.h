@@ -286,7 +286,7 @@ __device__ __forceinline__ void coef_scale_table(const CoefSet &S, double t, dou
     for (int i = v0 + (int)threadIdx.x; i < v1; i += (int)blockDim.x) {
         int e = 0;
         while (e + 1 < S.ncoef && i >= S.vstart[e + 1]) ++e;
-        vt[i] = cmul(vt[i], cf[e]);
+        vt[i] = cmul_fixed(vt[i], cf[e]);
     }
     __syncthreads();
 }

@@ -17,6 +17,10 @@ namespace qa {
 __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
     return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
+// a b with its rounding spelled out, where several kernels must agree
+__device__ __forceinline__ double2 cmul_fixed(double2 a, double2 b) {
+    return make_double2(fma(-a.y, b.y, a.x * b.x), fma(a.y, b.x, a.x * b.y));
+}
 __device__ __forceinline__ double2 cadd(double2 a, double2 b) {
     return make_double2(a.x + b.x, a.y + b.y);
 }
@@ -35,7 +39,8 @@ __device__ __forceinline__ void raxpy(double2 &acc, double s, double2 v) {
     acc.x = fma(s, v.x, acc.x);
     acc.y = fma(s, v.y, acc.y);
 }
-__device__ __forceinline__ double cabs2(double2 a) { return a.x * a.x + a.y * a.y; }
+// (an explicit fma: every kernel that forms an error norm rounds it alike)
+__device__ __forceinline__ double cabs2(double2 a) { return fma(a.x, a.x, a.y * a.y); }
 
 // Value loads: operator values may be stored in complex64 (float2) and are
 // widened to FP64 for accumulation.
@@ -134,14 +139,14 @@ __device__ __forceinline__ void sell_chunk(const int *__restrict__ col, const V 
 constexpr int kRowChunk = 24;  // entries of a lane per chunk (sell_row_dot)
 static_assert(kRowChunk % 2 == 0, "chunks must start at even steps");
 
-template <int L, typename V>
+template <int L, typename V, int CH = kRowChunk>
 __device__ __forceinline__ double2 sell_row_dot(const int *__restrict__ col,
                                                 const V *__restrict__ vals,
                                                 const double2 *__restrict__ x, int base,
                                                 int steps, int lane) {
     // Every lane of a slice makes the same number of steps (the slice width
     // divided by L), so the code below is not divergent.  A lane's entries
-    // go in chunks of up to kRowChunk; the last chunk (a wave-uniform count)
+    // go in chunks of up to CH (kRowChunk); the last chunk (a wave-uniform count)
     // is dispatched once to a fully unrolled body of exactly that length, so
     // no load is predicated and none waits for another.  A row that fits one
     // chunk costs two dependent round trips (columns and values, then the
@@ -150,12 +155,12 @@ __device__ __forceinline__ double2 sell_row_dot(const int *__restrict__ col,
     const int p0 = base + lane;
     double2 a0 = make_double2(0.0, 0.0), a1 = make_double2(0.0, 0.0);
     int k = 0;
-    for (; k + kRowChunk < steps; k += kRowChunk)
-        sell_chunk<kRowChunk>(col, vals, x, p0 + k * QA_WAVE, a0, a1);
+    for (; k + CH < steps; k += CH) sell_chunk<CH>(col, vals, x, p0 + k * QA_WAVE, a0, a1);
     const int p = p0 + k * QA_WAVE;
+    static_assert(CH % 2 == 0 && CH <= kRowChunk, "chunks start at even steps");
     switch (steps - k) {
 #define QA_SELL_CASE(m) \
-        case m: sell_chunk<m>(col, vals, x, p, a0, a1); break;
+        case m: sell_chunk<(m <= CH ? m : 1)>(col, vals, x, p, a0, a1); break;
         QA_SELL_CASE(24) QA_SELL_CASE(23) QA_SELL_CASE(22) QA_SELL_CASE(21) QA_SELL_CASE(20)
         QA_SELL_CASE(19) QA_SELL_CASE(18) QA_SELL_CASE(17) QA_SELL_CASE(16) QA_SELL_CASE(15)
         QA_SELL_CASE(14) QA_SELL_CASE(13) QA_SELL_CASE(12) QA_SELL_CASE(11) QA_SELL_CASE(10)

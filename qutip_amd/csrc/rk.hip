@@ -20,6 +20,12 @@
 // * one loop iteration (all of the above) is captured once into a hipGraph
 //   and replayed; kernels whose phase does not match return immediately.
 //
+// Sparse and banded engines of up to 131072 lanes run whole chunks of
+// attempts in one launch instead (rk_resident.hip), with the same bits; the
+// launched loop is theirs for single steps, while another engine of the
+// process holds the device's resident slot, and where a resident launch
+// gives up.
+//
 // Device state lives in an RKCtl block in HBM.  Vectors are complex128,
 // padded to a multiple of 64 rows.  Operator values are complex128 or
 // complex64 (widened to FP64 in registers; accumulation is always FP64).
@@ -27,168 +33,19 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <new>
 #include <vector>
 
 #include "qa_api_internal.h"
 #include "qa_coef.h"
 #include "qa_common.h"
+#include "qa_rk.h"
+#include "rk_resident.h"
 
 using namespace qa;
 
 namespace {
-
-enum Phase { PH_IDLE = 0, PH_STEP = 1, PH_DENSE = 2, PH_OUTPUT = 3, PH_DONE = 4, PH_ERROR = 5 };
-// integrator status codes: qutip/solver/integrator/explicit_rk.pxd:5-12
-enum Status {
-    ST_AT_FRONT = 2,
-    ST_INTERPOLATED = 1,
-    ST_NORMAL = 0,
-    ST_TOO_MUCH_WORK = -1,
-    ST_DT_UNDERFLOW = -2,
-    ST_OUTSIDE_RANGE = -3,
-    ST_NOT_INITIATED = -4
-};
-
-constexpr int kMaxStages = 16;
-constexpr int kMaxPending = 4;     // output times handled per output launch
-constexpr int kOutChunk = 16;      // functional entries per output workgroup
-constexpr int kOutThreads = 64;    // one wavefront per output workgroup
-constexpr int kStepBlocks = 256;   // threads per stage workgroup
-constexpr int kMaxChunk = 64;      // loop iterations per host chunk
-constexpr int kGraphBatch = 8;     // loop iterations per batch graph
-constexpr int kBatchAfter = 128;   // iterations an engine runs before it batches
-
-struct RKCtl {
-    double t_prev, t_front, dt_safe, dt_int, dt_try, err, t_last;
-    double rtol, atol, min_step, max_step;
-    double *times;  // mutable copy of the requested output times
-    double2 *fun_out;
-    double2 *states_out;
-    int ntimes, phase, cur, out_idx, nsteps_left, nsteps_call, dense_ready, status;
-    int order, max_numsteps, interpolate, adaptive, single_step, nfun;
-    long long n_attempts, n_accepted, n_dense, n_outputs;
-};
-
-// ---- step control (executed by one thread) ---------------------------------
-__device__ double get_timestep(const RKCtl *c, double t) {
-    // explicit_rk.pyx:439-449
-    const double dt_needed = t - c->t_prev;
-    if (!c->adaptive) return dt_needed;
-    if (c->interpolate) return c->dt_safe;
-    if (dt_needed <= c->dt_safe) return dt_needed;
-    return dt_needed / (double)((long long)(dt_needed / c->dt_safe) + 1);
-}
-
-__device__ void recompute_safe_step(RKCtl *c, double err, double dt) {
-    // explicit_rk.pyx:451-467
-    if (!c->adaptive) return;
-    double factor;
-    if (err == 0.0) {
-        factor = 10.0;
-    } else {
-        factor = 0.9 * pow(err, -1.0 / (c->order + 1));
-        factor = fmin(10.0, factor);
-        factor = fmax(0.2, factor);
-    }
-    c->dt_safe = dt * factor;
-    if (c->max_step != 0.0) c->dt_safe = fmin(c->max_step, c->dt_safe);
-    if (c->min_step != 0.0) c->dt_safe = fmax(c->min_step, c->dt_safe);
-}
-
-// y_prev <- y_front, t_prev <- t_front, then a fresh _step_in_err
-// (explicit_rk.pyx:312-316).
-__device__ void start_step(RKCtl *c, double target) {
-    c->cur ^= 1;
-    c->t_prev = c->t_front;
-    c->dense_ready = 0;
-    c->nsteps_call = 0;
-    c->dt_try = get_timestep(c, target);
-    c->phase = PH_STEP;
-}
-
-// Decide what the next output time needs (explicit_rk.pyx:288-331).
-__device__ void route(RKCtl *c) {
-    if (c->out_idx >= c->ntimes) {
-        c->phase = PH_DONE;
-        return;
-    }
-    double target = c->times[c->out_idx];
-    if (target < c->t_prev) {
-        c->status = ST_OUTSIDE_RANGE;
-        c->phase = PH_ERROR;
-        return;
-    }
-    if (target < c->t_front) {
-        if (!c->interpolate) {
-            c->status = ST_OUTSIDE_RANGE;
-            c->phase = PH_ERROR;
-            return;
-        }
-        c->phase = c->dense_ready ? PH_OUTPUT : PH_DENSE;
-        return;
-    }
-    if (c->single_step && c->t_last < c->t_front && target > c->t_front) {
-        // integrate(t, step=True) clamps to the front (explicit_rk.pyx:309-311)
-        c->times[c->out_idx] = c->t_front;
-        target = c->t_front;
-    }
-    if (target == c->t_front) {
-        c->phase = PH_OUTPUT;
-        return;
-    }
-    c->nsteps_left = c->max_numsteps;
-    c->status = ST_NORMAL;
-    start_step(c, target);
-}
-
-// After one attempt of _compute_step (explicit_rk.pyx:333-356).
-__device__ void after_attempt(RKCtl *c, double err) {
-    const double dt = c->dt_try;
-    c->err = err;
-    c->n_attempts++;
-    c->dt_int = dt;
-    recompute_safe_step(c, err, dt);
-    if (dt == c->min_step && err > 1.0) {
-        c->status = ST_DT_UNDERFLOW;
-        c->phase = PH_ERROR;
-        return;
-    }
-    c->nsteps_call++;
-    if (c->nsteps_call > c->nsteps_left) {
-        c->status = ST_TOO_MUCH_WORK;
-        c->phase = PH_ERROR;
-        return;
-    }
-    double target = c->times[c->out_idx];
-    if (err >= 1.0) {
-        c->dt_try = get_timestep(c, target);
-        c->phase = PH_STEP;
-        return;
-    }
-    c->t_front = c->t_prev + dt;
-    c->nsteps_left -= c->nsteps_call;
-    c->nsteps_call = 0;
-    c->n_accepted++;
-    c->dense_ready = 0;
-    if (c->single_step && c->t_front < target) {
-        // integrate(t, step=True) stops after one step at the front
-        c->times[c->out_idx] = c->t_front;
-        target = c->t_front;
-    }
-    if (c->t_front < target) {
-        start_step(c, target);
-    } else if (c->t_front > target) {
-        if (c->interpolate) {
-            c->phase = PH_DENSE;
-        } else {
-            c->status = ST_OUTSIDE_RANGE;
-            c->phase = PH_ERROR;
-        }
-    } else {
-        c->phase = PH_OUTPUT;
-    }
-}
 
 // ---- kernels -----------------------------------------------------------------
 enum Input { IN_YPREV = 0, IN_YFRONT = 1, IN_X = 2 };
@@ -229,9 +86,6 @@ struct StageArgs : EpiArgs {
     // coefficient programs and their value-table ranges
     CoefSet td;
 };
-
-// Operator forms of rk_stage_kernel.
-enum StageForm { FORM_PLAIN = 0, FORM_CODED = 1, FORM_CODED_UNIFORM = 2 };
 
 // The vectors a stage reads and writes, resolved from the control block.
 struct StageVecs {
@@ -400,7 +254,7 @@ __global__ __launch_bounds__(256) void coef_table_kernel(CoefSet S, double t,
         if (i >= S.vstart[0] && i < S.vstart[S.ncoef]) {
             int e = 0;
             while (e + 1 < S.ncoef && i >= S.vstart[e + 1]) ++e;
-            v = cmul(v, cf[e]);
+            v = cmul_fixed(v, cf[e]);
         }
         vt_out[i] = v;
     }
@@ -415,72 +269,6 @@ __global__ __launch_bounds__(256) void coef_eval_kernel(CoefSet S, int ntimes,
     if (i >= (int64_t)S.ncoef * ntimes) return;
     const int e = (int)(i / ntimes), k = (int)(i % ntimes);
     out[i] = coef_eval(S, e, times[k]);
-}
-
-// ---- banded (DIA) Lindblad right-hand side ----------------------------------
-// The matrix-form RHS k = Hm X + X Hp + sum_c C_c X Cd_c (Hm = -i H_nh,
-// Hp = i H_nh^dag, Cd_c = C_c^dag) for banded operators, as LindbladMatrix-
-// Form computes it with Dia products (lindblad_matrix_form.pyx:105-203 over
-// matmul_dia_dense_dense, matmul.pyx:429-507), in FP64.  Every product is a
-// list of terms acc += A[i, i+o] x[i+o, j-p] B[j-p, j]: a diagonal of Hm
-// (B = 1), of Hp (A = 1), or a pair of diagonals of C_c and Cd_c.  Values
-// are rows of `val` (row d: the diagonal's entries by row index; the last
-// row all ones).  One thread per element (i, j) of the column-major N x N
-// state, i fastest: the x and A loads of a wavefront are coalesced and its
-// B load is one value.  Terms go in chunks of at most eight, each a body of
-// exactly its length, so a chunk's loads are issued together; out-of-range
-// neighbours are clamped and their terms dropped by a select.
-constexpr int kDiaMaxTerms = 96;
-
-struct DiaTerm {
-    int o, p, a, b;
-};
-
-struct DiaOp {
-    int N, nterms;
-    const double2 *val;  // [rows][N]
-    DiaTerm t[kDiaMaxTerms];
-};
-
-template <int M>
-__device__ __forceinline__ void dia_terms(const DiaOp &D, const double2 *__restrict__ x, int i,
-                                          int j, int t0, double2 &acc) {
-    const int N = D.N;
-    double2 av[M], bv[M], xv[M];
-    bool ok[M];
-#pragma unroll
-    for (int u = 0; u < M; ++u) {
-        const DiaTerm T = D.t[t0 + u];
-        const int ii = i + T.o, jj = j - T.p;
-        ok[u] = (unsigned)ii < (unsigned)N && (unsigned)jj < (unsigned)N;
-        const int iic = ok[u] ? ii : i, jjc = ok[u] ? jj : j;
-        av[u] = D.val[(int64_t)T.a * N + i];
-        bv[u] = D.val[(int64_t)T.b * N + jjc];
-        xv[u] = x[(int64_t)jjc * N + iic];
-    }
-#pragma unroll
-    for (int u = 0; u < M; ++u) {
-        const double2 t = cmul(cmul(av[u], xv[u]), bv[u]);
-        if (ok[u]) acc = cadd(acc, t);
-    }
-}
-
-__device__ __forceinline__ double2 dia_rhs_at(const DiaOp &D, const double2 *__restrict__ x,
-                                              int i, int j) {
-    double2 acc = make_double2(0.0, 0.0);
-    int t = 0;
-    for (; t + 8 <= D.nterms; t += 8) dia_terms<8>(D, x, i, j, t, acc);
-    switch (D.nterms - t) {
-        case 7: dia_terms<7>(D, x, i, j, t, acc); break;
-        case 6: dia_terms<6>(D, x, i, j, t, acc); break;
-        case 5: dia_terms<5>(D, x, i, j, t, acc); break;
-        case 4: dia_terms<4>(D, x, i, j, t, acc); break;
-        case 3: dia_terms<3>(D, x, i, j, t, acc); break;
-        case 2: dia_terms<2>(D, x, i, j, t, acc); break;
-        case 1: dia_terms<1>(D, x, i, j, t, acc); break;
-        default: break;
-    }
-    return acc;
 }
 
 // One RK stage of the banded matrix form: the product for element r plus
@@ -1415,7 +1203,6 @@ __global__ __launch_bounds__(256) void rk_combine_kernel(RKCtl *ctl, int64_t npa
     }
 }
 
-constexpr int kMaxDenseOrder = 8;
 
 struct OutArgs {
     RKCtl *ctl;
@@ -1571,26 +1358,6 @@ __global__ __launch_bounds__(256) void rk_store_kernel(OutArgs A) {
     }
 }
 
-// Completion of an output (thread 0 of one workgroup): the time and status
-// of the last output, the counters, and the next phase (route).
-__device__ void finish_outputs(RKCtl *c, int ph, int nq, const int *front) {
-    if (nq == 0) {
-        // a non-finite step left no output time inside [t_prev, t_front]
-        c->status = ST_OUTSIDE_RANGE;
-        c->phase = PH_ERROR;
-        return;
-    }
-    if (ph == PH_DENSE) {
-        c->dense_ready = 1;
-        c->n_dense++;
-    }
-    c->t_last = c->times[c->out_idx + nq - 1];
-    c->status = front[nq - 1] ? ST_AT_FRONT : ST_INTERPOLATED;
-    c->n_outputs += nq;
-    c->out_idx += nq;
-    route(c);
-}
-
 // Functionals of the pending output states: linear f = sum w y[col] (a
 // vectorised density matrix: tr(O rho), tr(rho)) or quadratic
 // f = sum w conj(y[row]) y[col] (a ket: <psi|O|psi>, ||psi||^2).  Grid
@@ -1643,11 +1410,10 @@ __global__ __launch_bounds__(kOutThreads) void rk_output_kernel(OutArgs A) {
         if (q >= nq) break;  // uniform
         double2 v = make_double2(0.0, 0.0);
         if (has) {
-            v = cmul(fw, interp(A, kc, pc, fc, w[q], front[q]));
-            if (quad) {
-                const double2 l = interp(A, kr, pr, fr, w[q], front[q]);
-                v = cmul(make_double2(l.x, -l.y), v);
-            }
+            const double2 y = interp(A, kc, pc, fc, w[q], front[q]);
+            double2 l = y;
+            if (quad) l = interp(A, kr, pr, fr, w[q], front[q]);
+            v = fun_term(fw, y, quad, l);
         }
         const double re = wave_sum(v.x), im = wave_sum(v.y);
         if (lane == 0 && f < A.nfun) {
@@ -1864,11 +1630,26 @@ struct qa_rk_solver {
     // previous chunk's step-only head and starting time
     std::vector<double> times_host;
     bool run_single = false;
+    // the resident loop (rk_resident.hip): -1 not planned yet, 0 not for this
+    // engine (QUTIP_AMD_RESIDENT=0, or a shape it does not take), 1 planned.
+    // res_dev: the device whose resident slot this engine holds while a
+    // launch is in flight, or -1.
+    int res = -1, res_form = 0, res_dev = -1;
+    ResArgs rp = {};
+    void *res_block = nullptr;
+    // the rows the functionals read, and the entries by their slots
+    int nneed = 0, fnnz = 0;
+    int *need_dev = nullptr, *fslot_dev = nullptr;  // [npad]; [2][entries]: rows, columns
+    double2 *yout_dev = nullptr;
+    int64_t yout_cap = 0;  // states of nneed rows
     int ramp = 8, last_head = 0;
     double last_front = 0.0;
 };
 
 namespace {
+
+void res_give(qa_rk_solver *S);
+int res_prepare(qa_rk_solver *S);
 
 void fill_epi(EpiArgs &P, qa_rk_solver *S, int i) {
     P.nrows = S->n;
@@ -2276,7 +2057,7 @@ void free_all(qa_rk_solver *S) {
     if (S->event) (void)hipEventDestroy(S->event);
     void *ptrs[] = {S->block, S->dense_block, S->ctl, S->bi_dev, S->times_dev, S->fun_out_dev, S->fptr_dev,
                     S->fkind_dev, S->frow_dev, S->fcol_dev, S->fw_dev, S->fpart_dev, S->td_block,
-                    S->vtab_t, S->arrivals};
+                    S->vtab_t, S->arrivals, S->res_block, S->need_dev, S->fslot_dev, S->yout_dev};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (void *p : S->retired) (void)hipFree(p);
@@ -2311,6 +2092,8 @@ int rk_finish_create(qa_rk_solver *S, int order, int rk_step, int rk_extra, int 
         S->use_graph = !(g && g[0] == '0');
         const char *so = getenv("QUTIP_AMD_STEP_ONLY");
         S->step_only = !(so && so[0] == '0');
+        const char *rs = getenv("QUTIP_AMD_RESIDENT");
+        if (!S->use_graph || (rs && rs[0] == '0')) S->res = 0;
     }
     if (bi) S->bi.assign(bi, bi + (size_t)rk_extra * dorder);
     S->rtol = rtol;
@@ -2769,6 +2552,11 @@ int qa_rk_set_coefficients(qa_rk_solver *S, int ncoef, const int *start, const i
     S->td = T;
     S->td_on = 1;
     S->graph_dirty = true;
+    if (S->res == 1) {  // planned for the generator before
+        S->retired.push_back(S->res_block);
+        S->res_block = nullptr;
+        S->res = -1;
+    }
     return QA_OK;
 }
 
@@ -2795,6 +2583,7 @@ int qa_coef_eval(int ncoef, const int *start, int ncode, const int *code, int nc
 int qa_rk_destroy(qa_rk_solver *S) {
     if (!S) return QA_OK;
     (void)hipStreamSynchronize(S->stream);
+    res_give(S);
     free_all(S);
     delete S;
     return QA_OK;
@@ -2880,13 +2669,18 @@ int qa_rk_set_functionals(qa_rk_solver *S, int nfun, const int *kinds, const int
     int maxlen = 0;
     for (int f = 0; f < nfun; ++f) maxlen = std::max(maxlen, fptr[f + 1] - fptr[f]);
     QA_HIP(hipStreamSynchronize(S->stream));
-    void *olds[] = {S->fptr_dev, S->fkind_dev, S->frow_dev, S->fcol_dev, S->fw_dev, S->fpart_dev};
+    void *olds[] = {S->fptr_dev, S->fkind_dev, S->frow_dev, S->fcol_dev, S->fw_dev, S->fpart_dev,
+                    S->need_dev, S->fslot_dev, S->yout_dev};
     QA_HIP(hipStreamSynchronize(S->stream));  // no launch of this engine still reads them
     for (void *p : olds)
         if (p) S->retired.push_back(p);
     QA_CHECK(release_retired(S));
     S->fptr_dev = S->fkind_dev = S->frow_dev = S->fcol_dev = nullptr;
     S->fw_dev = S->fpart_dev = nullptr;
+    S->need_dev = S->fslot_dev = nullptr;
+    S->yout_dev = nullptr;
+    S->yout_cap = 0;
+    S->nneed = 0;
     S->nfun = nfun;
     S->nchunks = std::max(1, (maxlen + kOutChunk - 1) / kOutChunk);
     const int nf1 = std::max(nfun, 1);
@@ -2910,6 +2704,31 @@ int qa_rk_set_functionals(qa_rk_solver *S, int nfun, const int *kinds, const int
         QA_HIP(hipMemcpy(S->fcol_dev, cols, sizeof(int) * nnz, hipMemcpyHostToDevice));
         QA_HIP(hipMemcpy(S->fw_dev, w, sizeof(double2) * nnz, hipMemcpyHostToDevice));
     }
+    if (nnz > 0 && S->res != 0 && S->kind != 1) {
+        // the slots of the rows the entries read, in row order
+        std::vector<int> need((size_t)S->npad, -1), slot(2 * (size_t)nnz, 0);
+        for (int f = 0; f < nfun; ++f)
+            for (int p = fptr[f]; p < fptr[f + 1]; ++p) {
+                need[cols[p]] = 0;
+                if (kinds[f]) need[rows[p]] = 0;
+            }
+        int k = 0;
+        for (int &v : need)
+            if (v == 0) v = k++;
+        for (int f = 0; f < nfun; ++f)
+            for (int p = fptr[f]; p < fptr[f + 1]; ++p) {
+                slot[nnz + p] = need[cols[p]];
+                slot[p] = kinds[f] ? need[rows[p]] : 0;
+            }
+        S->nneed = k;
+        QA_HIP(hipMalloc((void **)&S->need_dev, sizeof(int) * need.size()));
+        QA_HIP(hipMalloc((void **)&S->fslot_dev, sizeof(int) * slot.size()));
+        QA_HIP(hipMemcpy(S->need_dev, need.data(), sizeof(int) * need.size(),
+                         hipMemcpyHostToDevice));
+        QA_HIP(hipMemcpy(S->fslot_dev, slot.data(), sizeof(int) * slot.size(),
+                         hipMemcpyHostToDevice));
+    }
+    S->fnnz = nnz;
     S->graph_dirty = true;
     return QA_OK;
 }
@@ -2984,6 +2803,8 @@ int qa_rk_begin(qa_rk_solver *S, int ntimes, const double *times, int single_ste
     hipStream_t s = S->stream;
     // the previous run may still be draining its last chunk
     QA_HIP(hipStreamSynchronize(s));
+    res_give(S);
+    if (S->res < 0) QA_CHECK(res_prepare(S));
     if (ntimes > S->times_cap) {
         if (S->times_dev) S->retired.push_back(S->times_dev);
         QA_CHECK(release_retired(S));
@@ -3015,7 +2836,10 @@ int qa_rk_begin(qa_rk_solver *S, int ntimes, const double *times, int single_ste
     // the sources above are pageable host memory: complete the copies here
     QA_HIP(hipStreamSynchronize(s));
     S->run_store = states_out != nullptr;
-    if (S->use_graph && (S->graph_dirty || S->graph_store != S->run_store)) {
+    // an engine with a resident loop captures its graphs when it first needs
+    // them (qa_rk_advance)
+    if (S->use_graph && (S->res != 1 || single_step) &&
+        (S->graph_dirty || S->graph_store != S->run_store)) {
         int rc = rebuild_graph(S);
         if (rc) return rc;
     }
@@ -3038,6 +2862,186 @@ int qa_rk_begin(qa_rk_solver *S, int ntimes, const double *times, int single_ste
 }
 
 namespace {
+
+// ---- the resident loop ------------------------------------------------------
+// One resident launch at a time per device and process: two of them could
+// each hold compute units that the other waits for.  An engine that does not
+// get the slot runs the launched loop for that chunk (the same bits).
+std::atomic<int> g_res_slot[64];
+constexpr int kResAttempts = 1024;             // attempts a launch
+constexpr int64_t kResOutBytes = 64LL << 20;   // states kept for the functionals
+
+bool res_take(qa_rk_solver *S) {
+    int dev = 0, none = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+    if (!g_res_slot[dev].compare_exchange_strong(none, 1)) return false;
+    S->res_dev = dev;
+    return true;
+}
+
+void res_give(qa_rk_solver *S) {
+    if (S->res_dev >= 0) g_res_slot[S->res_dev].store(0);
+    S->res_dev = -1;
+}
+
+// The launch shape, buffers and combine lists of an engine's resident loop;
+// S->res becomes 1 when it has one, else 0.
+int res_prepare(qa_rk_solver *S) {
+    S->res = 0;
+    if (S->kind == 1 || S->c.empty() || S->c[0] != 0.0) return QA_OK;
+    const int nk = S->interpolate ? S->rk_extra : S->rk_step;
+    const bool dense = S->interpolate && S->rk_extra > S->rk_step;
+    // the product of y_front serves both the next k_0 and the first dense
+    // stage when that stage is at the step's end
+    if (dense && S->first_dense_from_front && S->c[S->rk_step] != 1.0) return QA_OK;
+    const bool td = S->td_on != 0;
+    const int lanes = S->kind == 2 ? 1 : S->lanes;
+    const int64_t total = S->kind == 2 ? (int64_t)S->n : (int64_t)S->nslices * QA_WAVE;
+    if (S->kind == 2) {
+        S->res_form = RES_DIA;
+    } else {
+        // the longest slice: entries (coded: words of four) a lane
+        std::vector<int> sp((size_t)S->nslices + 1);
+        QA_HIP(hipMemcpy(sp.data(), S->slice_ptr, sizeof(int) * sp.size(), hipMemcpyDeviceToHost));
+        int w = 0;
+        for (int k = 0; k < S->nslices; ++k) w = std::max(w, (sp[k + 1] - sp[k]) / QA_WAVE);
+        if (!td && (S->coded ? 4 * w : w) <= kResKept)
+            S->res_form = RES_KEPT;
+        else if (S->coded)
+            S->res_form = td ? RES_CODED_TD : RES_CODED;
+        else
+            S->res_form = S->vals_fp32 ? RES_SELL_F32 : RES_SELL;
+    }
+    ResArgs &P = S->rp;
+    if (!res_plan(S->res_form, lanes, total, nk, S->vbits, &P)) return QA_OK;
+    P.n = S->n;
+    P.nslices = S->nslices;
+    P.nblk = S->nparts;
+    P.npad = S->npad;
+    P.rk_step = S->rk_step;
+    P.nk = nk;
+    P.dorder = S->dorder;
+    P.has_bi = S->interpolate ? 1 : 0;
+    P.dense = dense;
+    P.first_front = S->first_dense_from_front;
+    P.slice_ptr = S->slice_ptr;
+    P.col = S->col;
+    P.vals = S->vals;
+    P.code = (const uint2 *)S->code;
+    P.vtab = S->vtab;
+    P.otab = S->otab;
+    P.vbits = S->vbits;
+    P.fp32 = S->vals_fp32;
+    P.td = S->td;
+    P.ctl = S->ctl;
+    P.y0 = S->y0;
+    P.y1 = S->y1;
+    P.K = S->K;
+    P.y_last = S->y_last;
+    P.max_attempts = kResAttempts;
+    ResTab T;
+    memset(&T, 0, sizeof(T));
+    for (int i = 0; i <= kMaxStages; ++i) {
+        if (i < nk) {
+            EpiArgs E;
+            fill_epi(E, S, i);
+            T.nt[i] = E.nt;
+            for (int t = 0; t < E.nt; ++t) {
+                T.tj[i][t] = E.tj[t];
+                T.tc[i][t] = E.tc[t];
+                if (i == S->rk_step - 1) T.te[t] = E.te[t];
+            }
+            T.cs[i] = E.coef_self;
+            if (i == S->rk_step - 1) T.ce = E.ecoef_self;
+            T.c[i] = S->c[i];
+        } else if (i == kMaxStages && dense) {
+            for (int j = 0; j < S->rk_step; ++j) {
+                const double a = S->a[(size_t)S->rk_step * S->rk_extra + j];
+                if (a == 0.0) continue;
+                T.tj[i][T.nt[i]] = j;
+                T.tc[i][T.nt[i]++] = a;
+            }
+            if (T.nt[i] > kMaxStages - 1) return QA_OK;
+        }
+    }
+    if (S->interpolate)
+        for (int i = 0; i < nk; ++i)
+            for (int j = 0; j < S->dorder && j < kMaxDenseOrder; ++j)
+                T.bi[i][j] = S->bi[(size_t)i * S->dorder + j];
+    // ring, control words, tableau, partials
+    const size_t ring = sizeof(double2) * (size_t)S->npad * kResRing;
+    const size_t sync = sizeof(unsigned) * kResSyncWords;
+    const size_t tab = (sizeof(ResTab) + 255) / 256 * 256;
+    if (hipMalloc(&S->res_block, ring + sync + tab + sizeof(double) * 2 * (size_t)S->nparts) !=
+        hipSuccess) {
+        (void)hipGetLastError();  // no room: the launched loop needs less
+        S->res_block = nullptr;
+        return QA_OK;
+    }
+    char *p = (char *)S->res_block;
+    P.ring = (double2 *)p; p += ring;
+    P.sync = (unsigned *)p; p += sync;
+    P.tab = (const ResTab *)p; p += tab;
+    P.parts = (double *)p;
+    QA_HIP(hipMemcpyAsync((void *)P.tab, &T, sizeof(T), hipMemcpyHostToDevice, S->stream));
+    QA_HIP(hipStreamSynchronize(S->stream));
+    S->res = 1;
+    return QA_OK;
+}
+
+// A resident launch from output out_base on, and the functionals of the
+// outputs it reaches; false when it cannot run now.
+int res_chunk(qa_rk_solver *S, int out_base, bool *ran) {
+    *ran = false;
+    const int left = S->run_ntimes - out_base;
+    int64_t cap = left;
+    if (S->nneed > 0)
+        cap = std::min<int64_t>(left, std::max<int64_t>(kMaxPending, kResOutBytes / (16LL * S->nneed)));
+    if (S->nneed > 0 && cap * S->nneed > S->yout_cap) {
+        if (S->yout_dev) S->retired.push_back(S->yout_dev);
+        S->yout_dev = nullptr;
+        S->yout_cap = 0;
+        if (hipMalloc((void **)&S->yout_dev, sizeof(double2) * (size_t)(cap * S->nneed)) !=
+            hipSuccess) {
+            (void)hipGetLastError();
+            S->res = 0;
+            return QA_OK;
+        }
+        S->yout_cap = cap * S->nneed;
+    }
+    if (!res_take(S)) return QA_OK;
+    ResArgs P = S->rp;
+    P.need = S->nneed > 0 ? S->need_dev : nullptr;
+    P.yout = S->yout_dev;
+    P.nneed = S->nneed;
+    P.out_base = out_base;
+    P.out_cap = (int)std::max<int64_t>(cap, kMaxPending);
+    int rc = res_launch(S->res_form, P, S->dia, S->stream);
+    if (rc) {
+        res_give(S);
+        S->res = 0;
+        return rc;
+    }
+    ResFunArgs A;
+    A.ctl = S->ctl;
+    A.yout = S->yout_dev;
+    A.nneed = S->nneed;
+    A.out_base = out_base;
+    A.nfun = S->nfun;
+    A.fptr = S->fptr_dev;
+    A.fkind = S->fkind_dev;
+    A.frow = S->fslot_dev;
+    A.fcol = S->fslot_dev + S->fnnz;
+    A.fw = S->fw_dev;
+    A.fun_out = S->fun_out_dev;
+    rc = res_functionals(A, (int)cap, S->stream);
+    if (rc) {
+        res_give(S);
+        return rc;
+    }
+    *ran = true;
+    return QA_OK;
+}
 
 // The next chunk after the control block mirror `h`: its first *head
 // iterations step-only, the rest full; returns the chunk length (`chunk`,
@@ -3102,14 +3106,26 @@ int qa_rk_advance(qa_rk_solver *S, int *done) {
     hipStream_t s = S->stream;
     int head = 0;        // step-only iterations at the start of the next chunk
     bool idle = false;   // the stream has no work left (the last chunk completed)
+    int out_base = 0;
     if (S->in_flight) {
         const hipError_t q = hipEventQuery(S->event);
         if (q == hipErrorNotReady) return QA_OK;
         QA_HIP(q);
         S->in_flight = false;
         const RKCtl &h = *S->ctl_host;
+        const bool resident = S->res_dev >= 0;
+        res_give(S);
+        if (resident && h.resident != RES_DONE) {
+            // its workgroups did not all become resident: the state is as it
+            // was, and the launched loop takes over for good
+            S->res = 0;
+        } else if (resident) {
+            S->run_iters += h.n_attempts - std::max(S->last_attempts, 0LL);
+            S->graph_launches += h.n_attempts - std::max(S->last_attempts, 0LL);
+        }
+        out_base = h.out_idx;
         if (h.phase == PH_DONE || h.phase == PH_IDLE) {
-            if (!S->run_store) {  // y_last, which rk_store_kernel did not write
+            if (!S->run_store && !resident) {  // y_last, which rk_store_kernel did not write
                 OutArgs A = out_args(S);
                 const unsigned blocks = (unsigned)std::min<int64_t>((S->npad + 255) / 256, 2048);
                 hipLaunchKernelGGL(rk_final_state_kernel, dim3(blocks), dim3(256), 0, s, A);
@@ -3124,7 +3140,8 @@ int qa_rk_advance(qa_rk_solver *S, int *done) {
             *done = -1;
             return QA_OK;
         }
-        if (h.n_attempts == S->last_attempts && h.n_outputs == S->last_outputs) {
+        if (!(resident && S->res == 0) && h.n_attempts == S->last_attempts &&
+            h.n_outputs == S->last_outputs) {
             S->run_state = 3;
             qa::set_error("device loop made no progress (phase %d, output %d)", h.phase, h.out_idx);
             return QA_ERR_STATE;
@@ -3139,6 +3156,21 @@ int qa_rk_advance(qa_rk_solver *S, int *done) {
         S->chunk = plan_chunk(S, h, attempts_before, S->last_front, S->chunk, &head);
         S->last_front = h.t_front;
         idle = true;
+    }
+    if (S->res == 1 && !S->run_single) {
+        bool ran = false;
+        QA_CHECK(res_chunk(S, out_base, &ran));
+        if (ran) {
+            S->last_head = 0;
+            QA_HIP(hipMemcpyAsync(S->ctl_host, S->ctl, sizeof(RKCtl), hipMemcpyDeviceToHost, s));
+            QA_HIP(hipEventRecord(S->event, s));
+            S->in_flight = true;
+            return QA_OK;
+        }
+    }
+    if (S->use_graph && (S->graph_dirty || S->graph_store != S->run_store)) {
+        if (!idle) QA_HIP(hipStreamSynchronize(s));
+        QA_CHECK(rebuild_graph(S));
     }
     S->last_head = head;
     // An engine that has run kBatchAfter iterations captures the batch graph
