@@ -56,7 +56,7 @@ namespace qa {
 namespace {
 
 constexpr int kResThreads = 512;      // at most; two waves per SIMD
-constexpr int kResPoll = 1 << 17;     // polls of a wait (0.5 us or more each)
+constexpr int kResPoll = 1 << 20;     // polls of a wait (0.4 us or more each)
 constexpr int kResChunk = 12;         // entries of a longer plain row in flight (registers)
 constexpr int kResTimes = 256;        // output times kept in LDS
 constexpr size_t kResLdsMax = 160 * 1024 - 8 * 1024;  // beside the static part
@@ -650,7 +650,7 @@ __global__ __launch_bounds__(kResThreads) void rk_resident_kernel(ResArgs P, Dia
         unsigned d;
         d = 0;
         if (alive && W.wg != 0)
-            for (int k = 0; k < 16 * kResPoll && d == 0; ++k) d = ld_agent(P.sync + kSyCommit);
+            for (int k = 0; k < 4 * kResPoll && d == 0; ++k) d = ld_agent(P.sync + kSyCommit);
         if (d == 0) {
             // workgroup 0 past the last barrier, or a wait that ran out: the
             // first to set the word decides for all.  (Write back can only
