@@ -413,6 +413,40 @@ int qa_mc_run(int d, int ntraj, int ntimes, const double *times_dev, const void 
               double *col_times_dev, int *col_which_dev, int max_jumps, int *info_dev,
               int grid, void *stream);
 
+/* A d x d operator (d <= 2^cbits) in packed form, for the trajectory and
+ * whole-solve kernels: its diagonal (d complex values) apart, and up to
+ * `width` (even, at most 16) off-diagonal entries a row as 16-bit codes,
+ * entry u of row r at code[u d + r]: the column in the low cbits bits, an
+ * index into `table` above them.  table[0] is 0; shorter rows are filled
+ * with their own row and index 0.  ntab <= min(256, 2^(16 - cbits)).  imag != 0:
+ * every off-diagonal value is purely imaginary and `table` holds the ntab
+ * imaginary parts (real numbers), else ntab complex ones.  Values are
+ * complex64 / float when the run's fp32 is set.  The kernels that read it
+ * are compiled for one tableau shape: rk_step and rk_extra state the run's
+ * (10 and 16, adaptive, with dense output, the last stage not that of the
+ * new state).  Device pointers; a plain host struct.  No reference
+ * counterpart (storage form). */
+typedef struct {
+    const void *code, *diag, *table;
+    int width, cbits, ntab, imag, rk_step, rk_extra;
+} qa_packed_op;
+
+/* qa_mc_run with H_eff also given in packed form (NULL: none).  The kernel
+ * then keeps the codes and the diagonal in registers and the values in LDS
+ * instead of reading the ELL every stage, where the table fits the LDS
+ * beside the shape's vectors. */
+int qa_mc_run_packed(const qa_packed_op *packed, int d, int ntraj, int ntimes,
+              const double *times_dev, const void *psi0_dev, int h_width,
+              const int *h_col, const void *h_vals, int nchan,
+              const int *c_rowptr, const int *c_col, const void *c_vals, int neops,
+              const int *e_rowptr, const int *e_col, const void *e_vals,
+              const void *tableau_dev, const double *draws_dev, int max_draws,
+              double rtol, double atol, int nsteps, double first_step, double min_step,
+              double max_step, int norm_steps, double norm_t_tol, double norm_tol,
+              double norm_min_step, double mc_corr_eps, int fp32, void *expect_out_dev,
+              double *col_times_dev, int *col_which_dev, int max_jumps, int *info_dev,
+              int grid, void *stream);
+
 /* ---- whole solves of small systems ----------------------------------------
  * Replaces, for a constant generator with n <= 1024, the output loop of
  * Solver.run (qutip/solver/solver_base.py:81-157) around
@@ -439,6 +473,17 @@ int qa_functionals_check(int n, int nfun, const int *kinds, const int *fptr, con
 
 int qa_rk_small_run(int n, int nsys, double t0, int ntimes, const double *times_dev,
                     const void *y0_dev, int h_width, const int *h_col, const void *h_vals,
+                    long long h_stride, int nfun, const int *fkind, const int *fptr,
+                    const int *frows, const int *fcols, const void *fw, const void *tableau_dev,
+                    double rtol, double atol, int nsteps, double first_step, double min_step,
+                    double max_step, int fp32, void *fun_out_dev, void *y_final_dev,
+                    int *info_dev, int grid, void *stream);
+
+/* qa_rk_small_run with the operator also in packed form (NULL: none; one
+ * operator for every system, h_stride 0). */
+int qa_rk_small_run_packed(const qa_packed_op *packed, int n, int nsys, double t0, int ntimes,
+                    const double *times_dev, const void *y0_dev, int h_width, const int *h_col,
+                    const void *h_vals,
                     long long h_stride, int nfun, const int *fkind, const int *fptr,
                     const int *frows, const int *fcols, const void *fw, const void *tableau_dev,
                     double rtol, double atol, int nsteps, double first_step, double min_step,

@@ -20,16 +20,29 @@
 // streamed in; a trajectory that uses up its draws stops with a status the
 // host acts on.
 //
-// Layout: each thread owns one or two rows of the state (d <= 1024).  The
-// RK stage vectors stay on the chip for the whole trajectory: all sixteen in
-// LDS when they take at most half of it (two workgroups per CU), else
-// k_0..k_9 in registers and k_10..k_15 in LDS.  The vector an RHS product
-// reads is staged in LDS.  H_eff is
-// a column-major ELL in HBM (entry u of row r at u d + r), so the 64 lanes of
-// a wave, which own 64 consecutive rows, load 64 consecutive columns and
-// values per instruction; c_ops and e_ops (used at jumps and outputs only)
-// are CSR.  All operators are shared by all trajectories and served from L2.  Norms, error norms and expectation values accumulate in FP64;
-// with the complex64 variant the state, stages and RHS products are FP32.
+// Layout: each thread owns one row of the state (d <= 1024).  The RK stage
+// vectors stay on the chip for the whole trajectory, k_0..k_9 in registers
+// and k_10..k_15 in LDS.  The vector an RHS product reads is staged in LDS.
+// A vern7 run on an operator of few entries a row and few distinct values has
+// it packed: 16-bit codes in registers, values in LDS, so a stage touches no
+// other memory.  Else H_eff is a column-major ELL (entry u of row r at
+// u d + r), so the 64 lanes of a wave, which own 64 consecutive rows, load 64
+// consecutive columns and values per instruction, from L2; c_ops and e_ops
+// (used at jumps and outputs only) are CSR.  Norms, error norms and
+// expectation values accumulate in FP64; with the complex64 variant the
+// state, stages and RHS products are FP32.
+//
+// What bounds it: a stage is a chain (sum of stages, LDS write, barrier,
+// gathers, multiply-adds) of some 1700 clocks with one workgroup a CU, and
+// with 16 waves a CU the instructions and the LDS bytes of the gathers.
+// Measured against the ELL form with two rows a thread and a run-time
+// tableau, Ising chains with vern7, kernel time: L = 10, 2048 trajectories:
+// complex128 140 -> 53 ms, complex64 104 -> 52; L = 8, 500 of them: 4.2 ->
+// 1.9 ms and 3.8 -> 1.9; L = 8, 8192: 62 -> 16 ms; whole solve of a 400-row
+// Liouvillian: 5.5 -> 2.9 ms.  What gave it, for L = 10: no ELL in the
+// stages, one row a thread and stages in registers (the spills gone from the
+// stage loop) 140 -> 104, compile-time stage loops with step and dense output
+// apart 104 -> 53.
 #include <algorithm>
 #include <math.h>
 #include <string.h>
@@ -45,7 +58,7 @@ constexpr int kMcStages = 16;
 constexpr int kMcOrder = 8;
 constexpr int kMcMaxChan = 32;
 constexpr int kMcMaxEops = 8;
-constexpr int kMcThreads = 512;  // 2 waves per SIMD: 256 VGPRs per lane
+constexpr int kMcThreads = 1024; // threads of a workgroup at most
 
 // trajectory status codes (beside the RK codes of explicit_rk.pxd:5-12)
 enum McStatus {
@@ -100,6 +113,38 @@ struct McArgs {
     double2 *y_final;  // [nsys][d] or null
     int fun_lds;       // LDS bytes reserved for the functionals and times (0: none)
     int x2;            // a second LDS copy of the product's input vector is reserved
+    // packed operator (OP_PACKED, OP_PACKED_IM), or pk_width 0: the diagonal
+    // [d], and up to kMcPack off-diagonal entries a row as 16-bit codes,
+    // entry u of row r at u d + r: column | value index << pk_cbits; index 0
+    // is the value 0
+    const unsigned short *pk_code;
+    const void *pk_diag, *pk_tab;
+    int pk_width, pk_cbits, pk_ntab, pk_imag;
+};
+
+// Forms of the shared operator.  OP_ELL: columns and values from global
+// memory (or LDS, rk_small_kernel's HL); OP_PACKED: codes and the diagonal
+// in registers, the distinct values in LDS; OP_PACKED_IM: the same with
+// purely imaginary off-diagonal values (-i H of a real H).
+enum OpForm { OP_ELL = 0, OP_PACKED = 1, OP_PACKED_IM = 2 };
+constexpr int kMcPack = 16;     // packed entries a row
+constexpr int kMcPackTab = 256; // distinct packed values
+constexpr int kPackStep = 10;   // stages of a step, and with the dense output,
+constexpr int kPackExtra = 16;  // of the tableau that goes with a packed operator
+
+// A double that every thread of the workgroup holds alike, kept in scalar
+// registers: assignments go through lane 0.  The trajectory's times and
+// norms would take some forty vector registers otherwise, and comparisons of
+// them would mask lanes instead of branching.
+__device__ __forceinline__ double uni(double v) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+struct Uni {
+    double v;
+    __device__ __forceinline__ Uni() : v(0.0) {}
+    __device__ __forceinline__ Uni(double x) : v(uni(x)) {}
+    __device__ __forceinline__ operator double() const { return v; }
 };
 
 template <typename R>
@@ -140,12 +185,10 @@ __device__ __forceinline__ double nrm2(C2<R> v) {
     return (double)v.x * (double)v.x + (double)v.y * (double)v.y;
 }
 
-// RS (a template parameter): stages k_0..k_{RS-1} live in registers, the
-// rest in LDS.  RS = 10 keeps the step stages of vern7 in registers (512
-// threads, up to 256 VGPRs each); RS = 0 keeps every stage in LDS, which
-// frees the registers for 1024-thread workgroups (more waves in flight) when
-// the LDS holds all 18 vectors.
-constexpr int kRegStagesMax = 10;
+// Stages k_0 .. k_9 (the step stages of vern7) live in registers, the rest in
+// LDS: from LDS the sums over stages moved more bytes than the products, and
+// with two rows a thread the registers spilled.
+constexpr int kRegStages = 10;
 
 // Per-workgroup LDS (dynamic): the vector an RHS product reads, the stage
 // vectors k_10.. (the dense-output stages of vern7) and the FSAL slot, one
@@ -154,85 +197,94 @@ template <typename R>
 struct McLds {
     C2<R> *x;      // [npad]
     C2<R> *xalt;   // [npad] the other input buffer, or null (one buffer)
-    C2<R> *kd;     // [kMcStages - RS][npad]
-    C2<R> *kfsal;  // [npad]
+    C2<R> *kd;     // [npad][kDenseSlots]: a row's stages, then its FSAL slot
     double *red;   // [2 * kFunGroup * threads / 64]
     double *probs; // [kMcMaxChan]
     double *bfs;   // [2][kMcStages] dense-output weights (two buffers, alternating)
     int bsel;      // the buffer the next interpolation writes
     double *rsum;  // [2][2 * threads / 64] block-sum partials (two buffers, alternating)
     int rsel;      // the buffer the next block sum writes
+    const void *vt;  // packed operator: the table of values
     int npad;
 };
+
+// Slots of a row in kd: an odd number, so the 16-byte accesses of 16 lanes
+// fall into different banks, with one address register for all of them.
+constexpr int kDenseSlots = kMcStages - kRegStages + 1;
 
 // Functionals summed per block reduction (one pair of barriers for each
 // group) by the whole-solve kernel.
 constexpr int kFunGroup = 4;
 
 template <typename R>
-inline size_t mc_lds_bytes(int npad, int threads, int RS) {
-    return sizeof(C2<R>) * (size_t)npad * (2 + kMcStages - RS) +
+inline size_t mc_lds_bytes(int threads) {
+    return sizeof(C2<R>) * (size_t)threads * (1 + kDenseSlots) +
            sizeof(double) * ((2 * kFunGroup + 4) * (threads / 64) + kMcMaxChan + 2 * kMcStages) +
            64;
 }
 
-// A per-row value: each thread owns NR rows (r = threadIdx.x + q * blockDim.x).
-template <typename R, int NR>
-struct V {
-    C2<R> v[NR];
-};
-
-template <typename R, int NR>
-__device__ __forceinline__ V<R, NR> vzero() {
-    V<R, NR> o;
-#pragma unroll
-    for (int q = 0; q < NR; ++q) o.v[q] = mk<R>(0, 0);
-    return o;
-}
-
 // Per-trajectory integrator state.  Vectors are per thread; scalars are
 // uniform (every thread holds the same value).
-template <typename R, int NR, int RS>
+template <typename R>
 struct Traj {
-    V<R, NR> k[RS > 0 ? RS : 1];
-    V<R, NR> yprev, yfront, y;
-    double t, t_prev, t_front, dt_safe, dt_int;
+    C2<R> k[kRegStages];
+    C2<R> yprev, yfront, y;
+    Uni t, t_prev, t_front, dt_safe, dt_int;
     int status;    // trajectory status (McStatus)
     int rk_state;  // last RK status (INTERPOLATED marks a prepared dense output)
     long long attempts;
     int ndense;  // dense-output preparations
 };
 
-template <typename R, int NR, int RS>
+template <typename R, int NT, int FM>
 struct Ctx {
     const McArgs &A;
     McLds<R> &S;
-    const McTableau &T;
-    int row[NR];
-    bool act[NR];
-    int rowc[NR];  // the row clamped into [0, d) for the ELL loads
+    const double (*bi)[kMcOrder];  // the dense-output weights' polynomials, in LDS
+    int wave0;          // the first row of this wave, uniform
+    bool act;
+    int rowc;  // the row clamped into [0, d) for the ELL loads
     const int *hcol;    // this system's H_eff ELL
     const void *hval;
+    unsigned pk[FM == OP_ELL ? 1 : kMcPack / 2];  // this thread's codes, two a word
+    C2<R> dg;                                     // and diagonal entries
+    int n_step, n_extra, is_fsal, is_adaptive, is_interp;  // of the tableau, uniform
+    const __attribute__((address_space(4))) McTableau *tab;
+    // Packed operators come with a tableau of vern7's shape (packed_args), so
+    // the loops over stages have compile-time bounds: with run-time ones a
+    // branch stood between any two stages of every sum, and the compiler
+    // spilled the stage vectors.
+    static constexpr bool kFix = FM != OP_ELL;
+    __device__ __forceinline__ int rk_step() const { return kFix ? kPackStep : n_step; }
+    __device__ __forceinline__ int rk_extra() const { return kFix ? kPackExtra : n_extra; }
+    __device__ __forceinline__ bool fsal() const { return kFix ? false : is_fsal != 0; }
+    __device__ __forceinline__ bool adaptive() const { return kFix ? true : is_adaptive != 0; }
+    __device__ __forceinline__ bool interp() const { return kFix ? true : is_interp != 0; }
 };
+
+// This thread's row, formed anew at each use from the lane
+// number: kept in a register across the trajectory loop it was spilled, and
+// a scratch load (some 700 clocks) sat before every write to the LDS.
+template <typename R, int NT, int FM>
+__device__ __forceinline__ int row_of(const Ctx<R, NT, FM> &c) {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return c.wave0 + l;
+}
 
 // Stage vector j; j is a compile-time constant after unrolling, so the
 // register / LDS choice costs nothing.
-template <typename R, int NR, int RS>
-__device__ __forceinline__ V<R, NR> kget(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s, int j) {
-    if (j < RS) return s.k[j < RS ? j : 0];
-    V<R, NR> o;
-#pragma unroll
-    for (int q = 0; q < NR; ++q)
-        o.v[q] = c.S.kd[(size_t)(j - RS) * c.S.npad + c.row[q]];
-    return o;
+template <typename R, int NT, int FM>
+__device__ __forceinline__ C2<R> kget(Ctx<R, NT, FM> &c, Traj<R> &s, int j) {
+    if (j < kRegStages) return s.k[j < kRegStages ? j : 0];
+    return c.S.kd[row_of(c) * kDenseSlots + (j - kRegStages)];
 }
-template <typename R, int NR, int RS>
-__device__ __forceinline__ void kset(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s, int j, const V<R, NR> &x) {
-    if (j < RS) {
-        s.k[j < RS ? j : 0] = x;
+template <typename R, int NT, int FM>
+__device__ __forceinline__ void kset(Ctx<R, NT, FM> &c, Traj<R> &s, int j, const C2<R> &x) {
+    if (j < kRegStages) {
+        s.k[j < kRegStages ? j : 0] = x;
     } else {
-#pragma unroll
-        for (int q = 0; q < NR; ++q) c.S.kd[(size_t)(j - RS) * c.S.npad + c.row[q]] = x.v[q];
+        c.S.kd[row_of(c) * kDenseSlots + (j - kRegStages)] = x;
     }
 }
 
@@ -240,8 +292,8 @@ __device__ __forceinline__ void kset(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s, int 
 // so one barrier per sum suffices: a buffer is written again only after the
 // barrier of the sum in between, which every thread passes after its reads
 // of it (the buffers serve nothing else).
-template <typename R, int NR, int RS>
-__device__ __forceinline__ double bsum(Ctx<R, NR, RS> &c, double v) {
+template <typename R, int NT, int FM>
+__device__ __forceinline__ double bsum(Ctx<R, NT, FM> &c, double v) {
     const int lane = threadIdx.x & (QA_WAVE - 1), wid = threadIdx.x / QA_WAVE;
     const int nw = blockDim.x / QA_WAVE;
     double *rb = c.S.rsum + 2 * nw * c.S.rsel;
@@ -251,13 +303,13 @@ __device__ __forceinline__ double bsum(Ctx<R, NR, RS> &c, double v) {
     __syncthreads();
     double t = 0.0;
     for (int w = 0; w < nw; ++w) t += rb[w];
-    return t;
+    return uni(t);
 }
 
 // Two block sums with one pair of barriers; each component is summed in
 // the order bsum uses, so the results are bsum's bits.
-template <typename R, int NR, int RS>
-__device__ __forceinline__ double2 bsum2(Ctx<R, NR, RS> &c, double a, double b) {
+template <typename R, int NT, int FM>
+__device__ __forceinline__ double2 bsum2(Ctx<R, NT, FM> &c, double a, double b) {
     const int lane = threadIdx.x & (QA_WAVE - 1), wid = threadIdx.x / QA_WAVE;
     const int nw = blockDim.x / QA_WAVE;
     double *rb = c.S.rsum + 2 * nw * c.S.rsel;
@@ -274,7 +326,7 @@ __device__ __forceinline__ double2 bsum2(Ctx<R, NR, RS> &c, double a, double b) 
         ta += rb[w];
         tb += rb[nw + w];
     }
-    return make_double2(ta, tb);
+    return make_double2(uni(ta), uni(tb));
 }
 
 // The input of a product (or of the functionals) into LDS, for every thread
@@ -283,8 +335,8 @@ __device__ __forceinline__ double2 bsum2(Ctx<R, NR, RS> &c, double a, double b) 
 // the other buffer has not reached that barrier, and every read of a
 // buffer lies between the barrier after its writes and the barrier after
 // the next input's, before the buffer is written again.
-template <typename R, int NR, int RS>
-__device__ __forceinline__ void stage_in(Ctx<R, NR, RS> &c, const V<R, NR> &x) {
+template <typename R, int NT, int FM>
+__device__ __forceinline__ void stage_in(Ctx<R, NT, FM> &c, const C2<R> &x) {
     if (c.S.xalt) {  // uniform
         C2<R> *t = c.S.x;
         c.S.x = c.S.xalt;
@@ -292,140 +344,209 @@ __device__ __forceinline__ void stage_in(Ctx<R, NR, RS> &c, const V<R, NR> &x) {
     } else {
         __syncthreads();
     }
-#pragma unroll
-    for (int q = 0; q < NR; ++q) c.S.x[c.row[q]] = x.v[q];
+    c.S.x[row_of(c)] = x;
     __syncthreads();
 }
 
 // M ELL entries (u0 .. u0 + M - 1) of this thread's rows: all column and
 // value loads first, then the LDS gathers and multiply-adds.
-template <int M, typename R, int NR, int RS>
-__device__ __forceinline__ void ell_chunk(Ctx<R, NR, RS> &c, int u0, V<R, NR> &acc) {
+template <int M, typename R, int NT, int FM>
+__device__ __forceinline__ void ell_chunk(Ctx<R, NT, FM> &c, int u0, C2<R> &acc) {
     const C2<R> *hv = (const C2<R> *)c.hval;
     const size_t d = (size_t)c.A.d;
-    int cc[NR][M];
-    C2<R> vv[NR][M];
+    int cc[M];
+    C2<R> vv[M];
 #pragma unroll
-    for (int q = 0; q < NR; ++q)
+    for (int w = 0; w < M; ++w) cc[w] = c.hcol[(size_t)(u0 + w) * d + c.rowc];
 #pragma unroll
-        for (int w = 0; w < M; ++w) cc[q][w] = c.hcol[(size_t)(u0 + w) * d + c.rowc[q]];
+    for (int w = 0; w < M; ++w) vv[w] = hv[(size_t)(u0 + w) * d + c.rowc];
 #pragma unroll
-    for (int q = 0; q < NR; ++q)
-#pragma unroll
-        for (int w = 0; w < M; ++w) vv[q][w] = hv[(size_t)(u0 + w) * d + c.rowc[q]];
-#pragma unroll
-    for (int q = 0; q < NR; ++q)
-#pragma unroll
-        for (int w = 0; w < M; ++w) cfmaR<R>(acc.v[q], vv[q][w], c.S.x[cc[q][w]]);
+    for (int w = 0; w < M; ++w) cfmaR<R>(acc, vv[w], c.S.x[cc[w]]);
 }
 
-// k = H_eff x for this thread's rows; x is staged in LDS first.  The ELL
-// width is a multiple of 4 (the host pads it), so entries go in chunks of 8
-// (4 for two complex128 rows per thread, which leaves room for the stage
-// vectors in registers) and at most one chunk of 4; no load is predicated.
-template <typename R, int NR, int RS>
-__device__ __forceinline__ V<R, NR> rhs(Ctx<R, NR, RS> &c, const V<R, NR> &x) {
-    constexpr int K = (NR == 2 && sizeof(R) == 8) ? 4 : 8;
-    stage_in(c, x);
-    V<R, NR> acc = vzero<R, NR>();
-    const int W = c.A.h_width;
-    int u = 0;
-    for (; u + K <= W; u += K) ell_chunk<K>(c, u, acc);
-    if (K == 8 && u < W) ell_chunk<4>(c, u, acc);
+// M packed entries u0 .. u0 + M - 1 of this thread's rows: the gathers and
+// the values (LDS, no other memory) together, then the multiply-adds.
+template <int M, int U0, typename R, int NT, int FM>
+__device__ __forceinline__ void packed_chunk(Ctx<R, NT, FM> &c, C2<R> &acc) {
+    const unsigned cm = (1u << c.A.pk_cbits) - 1u;
+    C2<R> xv[M], vv[M];
 #pragma unroll
-    for (int q = 0; q < NR; ++q)
-        if (!c.act[q]) acc.v[q] = mk<R>(0, 0);  // padding rows stay zero
+    for (int w = 0; w < M; ++w) {
+        const unsigned h = (c.pk[(U0 + w) / 2] >> (16 * ((U0 + w) & 1))) & 0xffffu;
+        xv[w] = c.S.x[h & cm];
+        if constexpr (FM == OP_PACKED_IM)
+            vv[w].y = ((const R *)c.S.vt)[h >> c.A.pk_cbits];
+        else
+            vv[w] = ((const C2<R> *)c.S.vt)[h >> c.A.pk_cbits];
+    }
+#pragma unroll
+    for (int w = 0; w < M; ++w) {
+        if constexpr (FM == OP_PACKED_IM) {
+            acc.x = fma(-vv[w].y, xv[w].y, acc.x);
+            acc.y = fma(vv[w].y, xv[w].x, acc.y);
+        } else {
+            cfmaR<R>(acc, vv[w], xv[w]);
+        }
+    }
+}
+
+template <int K, int U0, typename R, int NT, int FM>
+__device__ __forceinline__ void packed_from(Ctx<R, NT, FM> &c, C2<R> &acc) {
+    if constexpr (U0 < kMcPack) {
+        const int left = c.A.pk_width - U0;  // uniform, even
+        if constexpr (K >= 8 && U0 + 8 <= kMcPack) {
+            if (left >= 8) {
+                packed_chunk<8, U0>(c, acc);
+                packed_from<K, U0 + 8>(c, acc);
+                return;
+            }
+        }
+        if constexpr (U0 + 4 <= kMcPack) {
+            if (left >= 4) {
+                packed_chunk<4, U0>(c, acc);
+                packed_from<4, U0 + 4>(c, acc);
+                return;
+            }
+        }
+        if (left == 2) packed_chunk<2, U0>(c, acc);
+    }
+}
+
+// k = H_eff x for this thread's rows; x is staged in LDS first.  ELL: the
+// width is a multiple of 4 (the host pads it), so entries go in chunks of 8
+// (4 in 1024 threads with complex128 stages in registers, which leaves room
+// for those) and at most one chunk of 4; no load is predicated.
+// Packed: the diagonal, then the entries in eights or fours and a last two.
+template <typename R, int NT, int FM>
+__device__ __forceinline__ C2<R> rhs(Ctx<R, NT, FM> &c, const C2<R> &x) {
+    stage_in(c, x);
+    C2<R> acc = mk<R>(0, 0);
+    constexpr int K = (NT > kMcThreads / 2 && sizeof(R) == 8) ? 4 : 8;
+    if constexpr (FM == OP_ELL) {
+        const int W = c.A.h_width;
+        int u = 0;
+        for (; u + K <= W; u += K) ell_chunk<K>(c, u, acc);
+        if (K == 8 && u < W) ell_chunk<4>(c, u, acc);
+    } else {
+        // opaque here, or every slot's decoded addresses are kept in
+        // registers for the whole kernel
+#pragma unroll
+        for (int w = 0; w < kMcPack / 2; ++w) asm volatile("" : "+v"(c.pk[w]));
+        cfmaR<R>(acc, c.dg, x);
+        packed_from<K, 0>(c, acc);
+    }
+    if constexpr (FM == OP_ELL) {
+        if (!c.act) acc = mk<R>(0, 0);  // padding rows stay zero
+    }
     return acc;
 }
 
 // (O x)_r for a CSR operator (c_ops / e_ops block); x already in LDS.
-template <typename R, int NR, int RS>
-__device__ __forceinline__ V<R, NR> op_rows(Ctx<R, NR, RS> &c, const int *rowptr, const int *col,
+template <typename R, int NT, int FM>
+__device__ __forceinline__ C2<R> op_rows(Ctx<R, NT, FM> &c, const int *rowptr, const int *col,
                                             const void *vals) {
-    V<R, NR> acc = vzero<R, NR>();
+    C2<R> acc = mk<R>(0, 0);
     const C2<R> *v = (const C2<R> *)vals;
-#pragma unroll
-    for (int q = 0; q < NR; ++q)
-        if (c.act[q])
-            for (int p = rowptr[c.row[q]]; p < rowptr[c.row[q] + 1]; ++p)
-                cfmaR<R>(acc.v[q], v[p], c.S.x[col[p]]);
+    if (c.act)
+        for (int p = rowptr[row_of(c)]; p < rowptr[row_of(c) + 1]; ++p)
+            cfmaR<R>(acc, v[p], c.S.x[col[p]]);
     return acc;
 }
 
-template <typename R, int NR, int RS>
-__device__ __forceinline__ double norm2(Ctx<R, NR, RS> &c, const V<R, NR> &x) {
+template <typename R, int NT, int FM>
+__device__ __forceinline__ double norm2(Ctx<R, NT, FM> &c, const C2<R> &x) {
     double s = 0.0;
-#pragma unroll
-    for (int q = 0; q < NR; ++q) s += nrm2<R>(x.v[q]);  // inactive rows hold zeros
+    s += nrm2<R>(x);  // inactive rows hold zeros
     return bsum(c, s);
 }
 
-// base + dt * sum_{j < n} coef[j] k_j (zero terms skipped like iadd_data)
-template <typename R, int NR, int RS>
-__device__ __forceinline__ V<R, NR> combine(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s, const V<R, NR> &base,
-                                            const double *coef, int n, double dt) {
-    V<R, NR> o = base;
+// The tableau's rows come through the constant address space: scalar loads
+// into scalar registers (from LDS they took two vector registers each and
+// spilled the stage vectors).
+typedef const __attribute__((address_space(4))) McTableau McConstTab;
+typedef const __attribute__((address_space(4))) double McCoef;
+
+// The weight of a stage in dt sum_j coef_j k_j.  complex128 sums with the
+// bare coefficient and multiplies by dt once; complex64 rounds the product
+// for every stage (with rounded coefficients the sums of a row's weights are
+// off by the same 1e-7 in every step, which adds up: the mean of 500
+// trajectories moved by 1e-4).
+__device__ __forceinline__ double weight(double coef, double, double) { return coef; }
+__device__ __forceinline__ float weight(double coef, double dt, float) { return (float)(coef * dt); }
+
+// yprev + dt sum_{j < n} coef[j] k_j (a zero coefficient adds nothing).
+template <typename R, int NT, int FM>
+__device__ __forceinline__ C2<R> combine(Ctx<R, NT, FM> &c, Traj<R> &s, McCoef *coef,
+                                            int n, double dt) {
+    constexpr bool once = sizeof(R) == 8;
+    C2<R> o = once ? mk<R>(0, 0) : s.yprev;
 #pragma unroll
     for (int j = 0; j < kMcStages; ++j) {
         if (j < n) {
-            const double f = dt * coef[j];
-            if (f != 0.0) {
-                const V<R, NR> kj = kget(c, s, j);
-#pragma unroll
-                for (int q = 0; q < NR; ++q) raxpyR<R>(o.v[q], (R)f, kj.v[q]);
-            }
+            const C2<R> kj = kget(c, s, j);
+            const R fj = weight(coef[j], dt, R());
+            raxpyR<R>(o, fj, kj);
         }
     }
-    return o;
+    if constexpr (!once) return o;
+    C2<R> r = s.yprev;
+    raxpyR<R>(r, (R)dt, o);
+    return r;
 }
 
-// _compute_step (explicit_rk.pyx:358-389) + _error (:391-397)
-template <typename R, int NR, int RS>
-__device__ __forceinline__ double compute_step(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s, double dt) {
-    const McTableau &T = c.T;
-    s.attempts++;
-    if (T.fsal) {
-        V<R, NR> k0;
+// The stages I0 <= i < I1, of which i0 <= i < i1 are formed.
+template <int I0, int I1, typename R, int NT, int FM>
+__device__ __forceinline__ void stages(Ctx<R, NT, FM> &c, Traj<R> &s, int i0, int i1,
+                                       double dt) {
 #pragma unroll
-        for (int q = 0; q < NR; ++q) k0.v[q] = c.S.kfsal[c.row[q]];
-        kset(c, s, 0, k0);
-    } else {
-        kset(c, s, 0, rhs(c, s.yprev));
-    }
-#pragma unroll
-    for (int i = 1; i < kMcStages; ++i) {
-        if (i < T.rk_step) {
-            const V<R, NR> x = combine(c, s, s.yprev, T.a[i], i, dt);
+    for (int i = I0; i < I1; ++i) {
+        if (FM != OP_ELL || (i >= i0 && i < i1)) {
+            const C2<R> x = combine(c, s, c.tab->a[i], i, dt);
             kset(c, s, i, rhs(c, x));
         }
     }
-    s.yfront = combine(c, s, s.yprev, T.b, T.rk_step, dt);
-    s.t_front = s.t_prev + dt;
-    if (!T.adaptive) return 0.0;
-    const V<R, NR> ev = combine(c, s, vzero<R, NR>(), T.e, T.rk_step, dt);
-    double qsum = 0.0;
+}
+
+// The stages of _compute_step (explicit_rk.pyx:358-389) and those of the
+// dense output (:399-410).
+template <typename R, int NT, int FM>
+__device__ __forceinline__ void step_stages(Ctx<R, NT, FM> &c, Traj<R> &s, double dt) {
+    stages<0, FM != OP_ELL ? kPackStep : kMcStages>(c, s, c.fsal() ? 1 : 0, c.rk_step(), dt);
+}
+template <typename R, int NT, int FM>
+__device__ __forceinline__ void dense_stages(Ctx<R, NT, FM> &c, Traj<R> &s) {
+    stages<FM != OP_ELL ? kPackStep : 1, kMcStages>(c, s, c.rk_step(), c.rk_extra(), s.dt_int);
+}
+
+// The end of _compute_step: y_front and the error norm (:391-397), one pass
+// over the stages for both sums.
+template <typename R, int NT, int FM>
+__device__ __forceinline__ double step_end(Ctx<R, NT, FM> &c, Traj<R> &s, double dt) {
+    constexpr bool once = sizeof(R) == 8;
+    McCoef *cb = c.tab->b, *ce = c.tab->e;
+    C2<R> o = once ? mk<R>(0, 0) : s.yprev, ev = mk<R>(0, 0);
 #pragma unroll
-    for (int q = 0; q < NR; ++q) {
-        if (c.act[q]) {
-            const double ratio = sqrt(nrm2<R>(ev.v[q])) /
-                                 (c.A.atol + c.A.rtol * sqrt(nrm2<R>(s.yfront.v[q])));
-            qsum += ratio * ratio;
+    for (int j = 0; j < kMcStages; ++j) {
+        if (j < c.rk_step()) {
+            const C2<R> kj = kget(c, s, j);
+            const R fb = weight(cb[j], dt, R()), fe = weight(ce[j], dt, R());
+            raxpyR<R>(o, fb, kj);
+            raxpyR<R>(ev, fe, kj);
         }
+    }
+    s.yfront = once ? s.yprev : o;
+    if constexpr (once) {
+        raxpyR<R>(s.yfront, (R)dt, o);
+    }
+    s.t_front = s.t_prev + dt;
+    if (!c.adaptive()) return 0.0;
+    double qsum = 0.0;
+    if (row_of(c) < c.A.d) {
+        const double tol = c.A.atol + c.A.rtol * sqrt(nrm2<R>(s.yfront));
+        const double ratio = (once ? dt : 1.0) * sqrt(nrm2<R>(ev)) / tol;
+        qsum += ratio * ratio;
     }
     return sqrt(bsum(c, qsum) / (double)c.A.d);
-}
-
-template <typename R, int NR, int RS>
-__device__ __forceinline__ void prep_dense_out(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s) {
-    const McTableau &T = c.T;
-    s.ndense++;
-#pragma unroll
-    for (int i = 0; i < kMcStages; ++i) {
-        if (i >= T.rk_step && i < T.rk_extra) {
-            const V<R, NR> x = combine(c, s, s.yprev, T.a[i], i, s.dt_int);
-            kset(c, s, i, rhs(c, x));
-        }
-    }
 }
 
 // The weights b_i(tau) (explicit_rk.pyx:412-430) are formed by threads
@@ -435,9 +556,8 @@ __device__ __forceinline__ void prep_dense_out(Ctx<R, NR, RS> &c, Traj<R, NR, RS
 // interpolation suffices: a buffer is written again only after the barrier
 // of the interpolation in between, which every thread passes after its
 // reads of it.
-template <typename R, int NR, int RS>
-__device__ __forceinline__ V<R, NR> interpolate(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s, double t) {
-    const McTableau &T = c.T;
+template <typename R, int NT, int FM>
+__device__ __forceinline__ C2<R> interpolate(Ctx<R, NT, FM> &c, Traj<R> &s, double t) {
     double *bw = c.S.bfs + kMcStages * c.S.bsel;
     c.S.bsel ^= 1;
     const int i = threadIdx.x;
@@ -445,38 +565,43 @@ __device__ __forceinline__ V<R, NR> interpolate(Ctx<R, NR, RS> &c, Traj<R, NR, R
         const double tau = (t - s.t_prev) / s.dt_int;
         double bv[kMcOrder];
 #pragma unroll
-        for (int j = 0; j < kMcOrder; ++j) bv[j] = T.bi[i][j];
+        for (int j = 0; j < kMcOrder; ++j) bv[j] = c.bi[i][j];
         double v = 0.0;
-        if (i < T.rk_extra) {
+        if (i < c.rk_extra()) {
 #pragma unroll
             for (int j = kMcOrder - 1; j >= 0; --j)
-                if (j < T.dorder) {  // Horner from j = dorder - 1 down
+                if (j < c.tab->dorder) {  // Horner from j = dorder - 1 down
                     v += bv[j];
                     v *= tau;
                 }
         }
-        bw[i] = v;
+        bw[i] = s.dt_int * v;
     }
     __syncthreads();
-    double bf[kMcStages];
+    C2<R> o = s.yprev;
 #pragma unroll
-    for (int k = 0; k < kMcStages; ++k) bf[k] = bw[k];
-    return combine(c, s, s.yprev, bf, T.rk_extra, s.dt_int);
+    for (int j = 0; j < kMcStages; ++j) {
+        if (j < c.rk_extra()) {
+            const C2<R> kj = kget(c, s, j);
+            const R fj = (R)bw[j];
+            raxpyR<R>(o, fj, kj);
+        }
+    }
+    return o;
 }
 
-template <typename R, int NR, int RS>
-__device__ __forceinline__ double estimate_first_step(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s,
-                                                      const V<R, NR> &y0) {
-    const McTableau &T = c.T;
-    if (!T.adaptive) return 0.0;
+template <typename R, int NT, int FM>
+__device__ __forceinline__ double estimate_first_step(Ctx<R, NT, FM> &c, Traj<R> &s,
+                                                      const C2<R> &y0) {
+    McConstTab &T = *c.tab;
+    if (!c.adaptive()) return 0.0;
     double norm = sqrt(norm2(c, y0));
     const double tol = c.A.atol + norm * c.A.rtol;
     // f(y0) and f(y0 + dt1/100 f(y0)) are local temporaries (the reference
     // borrows k[0] and k[1] for them; the next step overwrites both anyway)
-    V<R, NR> f0;
-    if (T.fsal) {
-#pragma unroll
-        for (int q = 0; q < NR; ++q) f0.v[q] = c.S.kfsal[c.row[q]];
+    C2<R> f0;
+    if (c.fsal()) {
+        f0 = c.S.kd[row_of(c) * kDenseSlots + (kDenseSlots - 1)];
     } else {
         f0 = rhs(c, y0);
     }
@@ -489,10 +614,9 @@ __device__ __forceinline__ double estimate_first_step(Ctx<R, NR, RS> &c, Traj<R,
         dt1 = pow(tol * factorial * pow(norm, T.order), 1.0 / (T.order + 1)) / tmp;
     else
         dt1 = pow(tol * factorial, 1.0 / (T.order + 1)) * norm * 0.5;
-    V<R, NR> yt = y0;
-#pragma unroll
-    for (int q = 0; q < NR; ++q) raxpyR<R>(yt.v[q], (R)(dt1 / 100), f0.v[q]);
-    const V<R, NR> f1 = rhs(c, yt);
+    C2<R> yt = y0;
+    raxpyR<R>(yt, (R)(dt1 / 100), f0);
+    const C2<R> f1 = rhs(c, yt);
     tmp = sqrt(norm2(c, f1));
     if (tmp >= c.A.atol * 1e-6)
         dt2 = pow(tol * factorial * pow(norm, T.order), 1.0 / (T.order + 1)) / tmp;
@@ -504,33 +628,47 @@ __device__ __forceinline__ double estimate_first_step(Ctx<R, NR, RS> &c, Traj<R,
     return dt;
 }
 
+// The stages in registers hold nothing from here on (no instruction): their
+// registers are free until the next stages fill them.
+template <typename R>
+__device__ __forceinline__ void drop_stages(Traj<R> &s) {
+#pragma unroll
+    for (int j = 0; j < kRegStages; ++j)
+        asm volatile("" : "=v"(s.k[j].x), "=v"(s.k[j].y));
+}
+
 // set_initial_value (explicit_rk.pyx:204-230)
-template <typename R, int NR, int RS>
-__device__ __forceinline__ void set_initial_value(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s,
-                                                  const V<R, NR> &y0, double t0) {
-    s.t = s.t_prev = s.t_front = t0;
+template <typename R, int NT, int FM>
+__device__ __forceinline__ void set_initial_value(Ctx<R, NT, FM> &c, Traj<R> &s,
+                                                  const C2<R> &y0, double t0) {
+    s.t = t0;
+    s.t_prev = s.t;
+    s.t_front = s.t;
     s.dt_int = 0.0;
     s.y = y0;
     s.yfront = y0;
     s.yprev = y0;
     s.rk_state = RK_NORMAL;
-    if (c.T.fsal) {
-        const V<R, NR> kf = rhs(c, y0);
-#pragma unroll
-        for (int q = 0; q < NR; ++q) c.S.kfsal[c.row[q]] = kf.v[q];
+    drop_stages(s);
+    if (c.fsal()) {
+        const C2<R> kf = rhs(c, y0);
+        c.S.kd[row_of(c) * kDenseSlots + (kDenseSlots - 1)] = kf;
     }
     s.dt_safe = c.A.first_step != 0.0 ? c.A.first_step : estimate_first_step(c, s, y0);
 }
 
-template <typename R, int NR, int RS>
-__device__ __forceinline__ void recompute_safe_step(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s, double err,
+template <typename R, int NT, int FM>
+__device__ __forceinline__ void recompute_safe_step(Ctx<R, NT, FM> &c, Traj<R> &s, double err,
                                                     double dt) {
-    if (!c.T.adaptive) return;
+    if (!c.adaptive()) return;
     double f;
     if (err == 0.0) {
         f = 10.0;
     } else {
-        f = 0.9 * pow(err, -1.0 / (c.T.order + 1));
+        // three square roots for vern7's eighth root: pow, which every wave
+        // computes, took 3800 clocks of a step in one wave and 13000 in 16
+        f = c.tab->order == 7 ? 0.9 / sqrt(sqrt(sqrt(err)))
+                              : 0.9 * pow(err, -1.0 / (c.tab->order + 1));
         f = fmin(10.0, f);
         f = fmax(0.2, f);
     }
@@ -539,83 +677,97 @@ __device__ __forceinline__ void recompute_safe_step(Ctx<R, NR, RS> &c, Traj<R, N
     if (c.A.min_step != 0.0) s.dt_safe = fmax(c.A.min_step, s.dt_safe);
 }
 
-template <typename R, int NR, int RS>
-__device__ __forceinline__ double get_timestep(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s, double t) {
+template <typename R, int NT, int FM>
+__device__ __forceinline__ double get_timestep(Ctx<R, NT, FM> &c, Traj<R> &s, double t) {
     const double dt_needed = t - s.t_prev;
-    if (!c.T.adaptive) return dt_needed;
-    if (c.T.interpolate) return s.dt_safe;
+    if (!c.adaptive()) return dt_needed;
+    if (c.interp()) return s.dt_safe;
     if (dt_needed <= s.dt_safe) return dt_needed;
     return dt_needed / (double)((long long)(dt_needed / s.dt_safe) + 1);
 }
 
-// _step_in_err (explicit_rk.pyx:333-356); returns attempts, sets status
-template <typename R, int NR, int RS>
-__device__ __forceinline__ int step_in_err(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s, double t, int max_step) {
-    double error = 1.0;
-    int n = 0;
-    while (error >= 1.0) {
-        const double dt = get_timestep(c, s, t);
-        error = compute_step(c, s, dt);
-        s.dt_int = dt;
-        recompute_safe_step(c, s, error, dt);
-        if (dt == c.A.min_step && error > 1.0) {
-            s.status = MC_DT_UNDERFLOW;
-            break;
-        }
-        n++;
-        if (n > max_step) {
-            s.status = MC_TOO_MUCH_WORK;
-            break;
-        }
-    }
-    if (c.T.fsal) {
-#pragma unroll
-        for (int j = 0; j < kMcStages; ++j) {
-            if (j == c.T.rk_step - 1) {
-                const V<R, NR> kl = kget(c, s, j);
-#pragma unroll
-                for (int q = 0; q < NR; ++q) c.S.kfsal[c.row[q]] = kl.v[q];
-            }
-        }
-    }
-    return n;
-}
-
-// integrate(t, step=True): explicit_rk.pyx:278-331 with step=True.
-template <typename R, int NR, int RS>
-__device__ __forceinline__ void mcstep(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s, double t) {
-    int nsteps_left = c.A.nsteps;
+// integrate(t, step) (explicit_rk.pyx:278-331) with _step_in_err (:333-356):
+// single: one accepted step at most (mcstep), else steps until t_front
+// reaches t within one budget of nsteps attempts; then the state at t, by
+// interpolation or y_front.
+template <typename R, int NT, int FM>
+__device__ __forceinline__ void advance(Ctx<R, NT, FM> &c, Traj<R> &s, double t,
+                                        bool single) {
     if (t == s.t) return;
     if (t < s.t_prev) {
         s.status = MC_OUTSIDE_RANGE;
         return;
     }
-    if (c.T.interpolate && t < s.t_front) {
-        if (s.rk_state != RK_INTERPOLATED) {
-            prep_dense_out(c, s);
-            s.rk_state = RK_INTERPOLATED;
+    bool stepping = false, dense = false, interp = false;
+    if (c.interp() && t < s.t_front) {
+        dense = s.rk_state != RK_INTERPOLATED;
+        interp = true;
+    } else {
+        s.rk_state = RK_NORMAL;
+        if (single && s.t < s.t_front && t > s.t_front) t = s.t_front;
+        stepping = s.t_front < t;
+        if (!stepping) {
+            s.rk_state = RK_AT_FRONT;
+            s.t = s.t_front;
+            s.y = s.yfront;
+            return;
         }
-        s.y = interpolate(c, s, t);
-        s.t = t;
-        return;
-    }
-    s.rk_state = RK_NORMAL;
-    if (s.t < s.t_front && t > s.t_front) t = s.t_front;
-    if (s.t_front < t) {
         s.yprev = s.yfront;
         s.t_prev = s.t_front;
-        nsteps_left -= step_in_err(c, s, t, nsteps_left);
     }
-    if (s.status < 0) return;
-    if (s.t_front > t) {
-        prep_dense_out(c, s);
+    int nsteps_left = c.A.nsteps, n = 0;
+    while (stepping) {
+        drop_stages(s);
+        const double dt = get_timestep(c, s, t);
+        s.attempts++;
+        if (c.fsal()) {
+            C2<R> k0;
+            k0 = c.S.kd[row_of(c) * kDenseSlots + (kDenseSlots - 1)];
+            kset(c, s, 0, k0);
+        }
+        step_stages(c, s, dt);
+        const double error = step_end(c, s, dt);
+        s.dt_int = dt;
+        recompute_safe_step(c, s, error, dt);
+        n++;
+        if (dt == c.A.min_step && error > 1.0)
+            s.status = MC_DT_UNDERFLOW;
+        else if (n > nsteps_left)
+            s.status = MC_TOO_MUCH_WORK;
+        if (error >= 1.0 && s.status >= 0) continue;
+        if (c.fsal()) {
+#pragma unroll
+            for (int j = 0; j < kMcStages; ++j) {
+                if (j == c.rk_step() - 1) {
+                    const C2<R> kl = kget(c, s, j);
+                    c.S.kd[row_of(c) * kDenseSlots + (kDenseSlots - 1)] = kl;
+                }
+            }
+        }
+        if (s.status < 0) return;
+        nsteps_left -= n;
+        n = 0;
+        if (!single && s.t_front < t) {
+            s.yprev = s.yfront;
+            s.t_prev = s.t_front;
+            continue;
+        }
+        stepping = false;
+        interp = dense = s.t_front > t;
+        if (!interp) {
+            s.rk_state = RK_AT_FRONT;
+            s.t = s.t_front;
+            s.y = s.yfront;
+        }
+    }
+    if (dense) {
+        s.ndense++;
+        dense_stages(c, s);
         s.rk_state = RK_INTERPOLATED;
-        s.t = t;
+    }
+    if (interp) {
         s.y = interpolate(c, s, t);
-    } else {
-        s.rk_state = RK_AT_FRONT;
-        s.t = s.t_front;
-        s.y = s.yfront;
+        s.t = t;
     }
 }
 
@@ -624,117 +776,27 @@ struct Rng {
     int n, used;
 };
 
-__device__ __forceinline__ bool draw(Rng &g, double &u) {
+template <typename D>
+__device__ __forceinline__ bool draw(Rng &g, D &u) {
     if (g.used >= g.n) return false;
     u = g.d[g.used++];
     return true;
 }
 
-template <typename R, int NR, int RS>
-__device__ __forceinline__ void write_expect(Ctx<R, NR, RS> &c, const V<R, NR> &y, int traj, int k) {
-    const double n2 = norm2(c, y);
+template <typename R, int NT, int FM>
+__device__ __forceinline__ void write_expect(Ctx<R, NT, FM> &c, const C2<R> &y, double n2,
+                                             int traj, int k) {
     stage_in(c, y);
     for (int e = 0; e < c.A.neops; ++e) {
         const int *rp = c.A.e_rowptr + (size_t)e * (c.A.d + 1);
-        const V<R, NR> oy = op_rows(c, rp, c.A.e_col, c.A.e_vals);
+        const C2<R> oy = op_rows(c, rp, c.A.e_col, c.A.e_vals);
         double re = 0.0, im = 0.0;  // conj(y_r) (O y)_r in FP64
-#pragma unroll
-        for (int q = 0; q < NR; ++q) {
-            re += (double)y.v[q].x * oy.v[q].x + (double)y.v[q].y * oy.v[q].y;
-            im += (double)y.v[q].x * oy.v[q].y - (double)y.v[q].y * oy.v[q].x;
-        }
+        re += (double)y.x * oy.x + (double)y.y * oy.y;
+        im += (double)y.x * oy.y - (double)y.y * oy.x;
         const double2 r = bsum2(c, re, im);
         if (threadIdx.x == 0)
             c.A.expect_out[((size_t)traj * c.A.ntimes + k) * c.A.neops + e] =
                 make_double2(r.x / n2, r.y / n2);
-    }
-}
-
-// LDS carving, tableau copy and zeroing shared by the kernels of this file.
-template <typename R, int NR, int RS>
-__device__ __forceinline__ void kernel_prologue(const McArgs &A, unsigned char *lds,
-                                                McTableau &T, McLds<R> &S) {
-    const int nt = blockDim.x;
-    const int npad = nt * NR;
-    {
-        unsigned char *p = lds;
-        S.npad = npad;
-        S.x = (C2<R> *)p;
-        p += sizeof(C2<R>) * npad;
-        S.kd = (C2<R> *)p;
-        p += sizeof(C2<R>) * npad * (kMcStages - RS);
-        S.kfsal = (C2<R> *)p;
-        p += sizeof(C2<R>) * npad;
-        S.red = (double *)p;
-        p += sizeof(double) * 2 * kFunGroup * (nt / QA_WAVE);
-        S.probs = (double *)p;
-        p += sizeof(double) * kMcMaxChan;
-        S.bfs = (double *)p;
-        S.bsel = 0;
-        p += sizeof(double) * 2 * kMcStages;
-        S.rsum = (double *)p;
-        S.rsel = 0;
-        S.xalt = nullptr;
-    }
-    {
-        const double *src = (const double *)A.tab;
-        double *dst = (double *)&T;
-        const int nd = (int)(sizeof(McTableau) / sizeof(double));
-        for (int i = threadIdx.x; i < nd; i += nt) dst[i] = src[i];
-    }
-    for (int i = threadIdx.x; i < (kMcStages - RS + 2) * npad; i += nt)
-        S.x[i] = mk<R>(0, 0);  // x, the LDS stages and the FSAL slot start at zero
-    __syncthreads();
-}
-
-template <typename R, int NR, int RS>
-__device__ __forceinline__ void ctx_rows(Ctx<R, NR, RS> &c, const int *hcol, const void *hval) {
-    c.hcol = hcol;
-    c.hval = hval;
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-        c.row[q] = threadIdx.x + q * blockDim.x;
-        c.act[q] = c.row[q] < c.A.d;
-        c.rowc[q] = c.act[q] ? c.row[q] : 0;
-    }
-}
-
-// integrate(t, step=False) (explicit_rk.pyx:278-331): steps until t_front
-// reaches t within one budget of nsteps attempts, then interpolates (or
-// takes y_front).
-template <typename R, int NR, int RS>
-__device__ __forceinline__ void integrate_to(Ctx<R, NR, RS> &c, Traj<R, NR, RS> &s, double t) {
-    int nsteps_left = c.A.nsteps;
-    if (t == s.t) return;
-    if (t < s.t_prev) {
-        s.status = MC_OUTSIDE_RANGE;
-        return;
-    }
-    if (c.T.interpolate && t < s.t_front) {
-        if (s.rk_state != RK_INTERPOLATED) {
-            prep_dense_out(c, s);
-            s.rk_state = RK_INTERPOLATED;
-        }
-        s.y = interpolate(c, s, t);
-        s.t = t;
-        return;
-    }
-    s.rk_state = RK_NORMAL;
-    while (s.t_front < t && s.status >= 0) {
-        s.yprev = s.yfront;
-        s.t_prev = s.t_front;
-        nsteps_left -= step_in_err(c, s, t, nsteps_left);
-    }
-    if (s.status < 0) return;
-    if (s.t_front > t) {
-        prep_dense_out(c, s);
-        s.rk_state = RK_INTERPOLATED;
-        s.t = t;
-        s.y = interpolate(c, s, t);
-    } else {
-        s.rk_state = RK_AT_FRONT;
-        s.t = s.t_front;
-        s.y = s.yfront;
     }
 }
 
@@ -748,6 +810,80 @@ __device__ __forceinline__ unsigned char *align16(T *p) {
     return b + ((16 - ((uintptr_t)b & 15)) & 15);
 }
 
+// LDS carving, tableau copy and zeroing shared by the kernels of this file;
+// returns the first free byte, aligned to 16.
+template <typename R, int NT, int FM>
+__device__ __forceinline__ unsigned char *kernel_prologue(const McArgs &A, unsigned char *lds,
+                                                          double (*bi)[kMcOrder], McLds<R> &S) {
+    const int nt = blockDim.x;
+    const int npad = nt;
+    unsigned char *p = lds;
+    S.npad = npad;
+    S.x = (C2<R> *)p;
+    p += sizeof(C2<R>) * npad;
+    S.kd = (C2<R> *)p;
+    p += sizeof(C2<R>) * npad * kDenseSlots;
+    S.red = (double *)p;
+    p += sizeof(double) * 2 * kFunGroup * (nt / QA_WAVE);
+    S.probs = (double *)p;
+    p += sizeof(double) * kMcMaxChan;
+    S.bfs = (double *)p;
+    S.bsel = 0;
+    p += sizeof(double) * 2 * kMcStages;
+    S.rsum = (double *)p;
+    S.rsel = 0;
+    unsigned char *tail = align16(S.rsum + 4 * (nt / QA_WAVE));
+    S.vt = tail;
+    if constexpr (FM != OP_ELL) {  // the packed operator's values
+        const int words = A.pk_ntab * (int)(sizeof(R) * (FM == OP_PACKED_IM ? 1 : 2) / 4);
+        for (int i = threadIdx.x; i < words; i += nt) ((int *)tail)[i] = ((const int *)A.pk_tab)[i];
+        tail = align16((int *)tail + words);
+    }
+    S.xalt = nullptr;
+    if (A.x2) {  // the second input buffer, when the launcher reserved it
+        S.xalt = (C2<R> *)tail;
+        tail += sizeof(C2<R>) * (size_t)npad;
+    }
+    for (int i = threadIdx.x; i < kMcStages * kMcOrder; i += nt)
+        (&bi[0][0])[i] = (&A.tab->bi[0][0])[i];
+    for (int i = threadIdx.x; i < (1 + kDenseSlots) * npad; i += nt)
+        S.x[i] = mk<R>(0, 0);  // x, the LDS stages and the FSAL slot start at zero
+    __syncthreads();
+    return tail;
+}
+
+// The rows of this thread, the operator it multiplies with, and the
+// tableau's sizes as scalars.
+template <typename R, int NT, int FM>
+__device__ __forceinline__ void ctx_rows(Ctx<R, NT, FM> &c, const int *hcol, const void *hval) {
+    c.hcol = hcol;
+    c.hval = hval;
+    c.wave0 = __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~(QA_WAVE - 1));
+    c.tab = (McConstTab *)c.A.tab;
+    c.n_step = c.tab->rk_step;
+    c.n_extra = c.tab->rk_extra;
+    c.is_fsal = c.tab->fsal;
+    c.is_adaptive = c.tab->adaptive;
+    c.is_interp = c.tab->interpolate;
+    const int row = row_of(c);
+    c.act = row < c.A.d;
+    c.rowc = c.act ? row : 0;
+    if constexpr (FM != OP_ELL) {
+        // padding rows: a zero diagonal and value 0 in every slot
+        c.dg = c.act ? ((const C2<R> *)c.A.pk_diag)[c.rowc] : mk<R>(0, 0);
+#pragma unroll
+        for (int u = 0; u < kMcPack; ++u) {
+            const unsigned h = u < c.A.pk_width && c.act
+                                   ? c.A.pk_code[(size_t)u * c.A.d + c.rowc]
+                                   : 0u;
+            if (u & 1)
+                c.pk[u / 2] |= h << 16;
+            else
+                c.pk[u / 2] = h;
+        }
+    }
+}
+
 // The functionals as the whole-solve kernel reads them: kind, CSR-style
 // entry pointer, rows, columns and weights, in LDS when they were staged
 // there, else in global memory.
@@ -759,8 +895,8 @@ struct FunView {
 // Functionals of the state y (linear: sum w y[col]; quadratic:
 // sum w conj(y[row]) y[col]), accumulated in FP64 in a fixed order, into
 // out[0 .. nfun-1] (thread 0 writes).
-template <typename R, int NR, int RS>
-__device__ __forceinline__ void write_functionals(Ctx<R, NR, RS> &c, const V<R, NR> &y,
+template <typename R, int NT, int FM>
+__device__ __forceinline__ void write_functionals(Ctx<R, NT, FM> &c, const C2<R> &y,
                                                   const FunView &fv, double2 *out) {
     stage_in(c, y);
     const int lane = threadIdx.x & (QA_WAVE - 1), wid = threadIdx.x / QA_WAVE;
@@ -814,183 +950,165 @@ __device__ __forceinline__ void write_functionals(Ctx<R, NR, RS> &c, const V<R, 
     }
 }
 
-template <typename R, int NR, int RS>
-__global__ __launch_bounds__(RS == 0 ? 2 * kMcThreads : kMcThreads) void mc_traj_kernel(McArgs A) {
+// One trajectory after another (grid-stride).  The loop holds one copy of
+// each part: a start (of the trajectory, or after a jump), one advance (to
+// the next output time, or to a guess of the collapse time), the search and
+// the jump, the outputs.
+template <typename R, int NT, int FM>
+__global__ __launch_bounds__(NT) void mc_traj_kernel(McArgs A) {
     extern __shared__ __align__(16) unsigned char mc_dyn_lds[];
-    __shared__ McTableau T;
+    __shared__ double bi[kMcStages][kMcOrder];
     McLds<R> S;
-    const int nt = blockDim.x;
-    const int npad = nt * NR;
-    {
-        unsigned char *p = mc_dyn_lds;
-        S.npad = npad;
-        S.x = (C2<R> *)p;
-        p += sizeof(C2<R>) * npad;
-        S.kd = (C2<R> *)p;
-        p += sizeof(C2<R>) * npad * (kMcStages - RS);
-        S.kfsal = (C2<R> *)p;
-        p += sizeof(C2<R>) * npad;
-        S.red = (double *)p;
-        p += sizeof(double) * 2 * kFunGroup * (nt / QA_WAVE);
-        S.probs = (double *)p;
-        p += sizeof(double) * kMcMaxChan;
-        S.bfs = (double *)p;
-        S.bsel = 0;
-        p += sizeof(double) * 2 * kMcStages;
-        S.rsum = (double *)p;
-        S.rsel = 0;
-        // the second input buffer, when the launcher reserved it
-        S.xalt = A.x2 ? (C2<R> *)align16(S.rsum + 4 * (nt / QA_WAVE)) : nullptr;
-    }
-    {
-        const double *src = (const double *)A.tab;
-        double *dst = (double *)&T;
-        const int nd = (int)(sizeof(McTableau) / sizeof(double));
-        for (int i = threadIdx.x; i < nd; i += nt) dst[i] = src[i];
-    }
-    for (int i = threadIdx.x; i < (kMcStages - RS + 2) * npad; i += nt)
-        S.x[i] = mk<R>(0, 0);  // x, the LDS stages and the FSAL slot start at zero
-    __syncthreads();
-    // (written out here rather than through kernel_prologue / ctx_rows: the
-    // shared helpers cost this kernel 100 B/lane more register spill)
-    Ctx<R, NR, RS> c{A, S, T};
-    c.hcol = A.h_col;
-    c.hval = A.h_vals;
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-        c.row[q] = threadIdx.x + q * nt;
-        c.act[q] = c.row[q] < A.d;
-        c.rowc[q] = c.act[q] ? c.row[q] : 0;
-    }
+    kernel_prologue<R, NT, FM>(A, mc_dyn_lds, bi, S);
+    Ctx<R, NT, FM> c{A, S, bi};
+    ctx_rows(c, A.h_col, A.h_vals);
 
     for (int traj = blockIdx.x; traj < A.ntraj; traj += gridDim.x) {
-        Traj<R, NR, RS> s;
+        Traj<R> s;
         s.status = MC_OK;
         s.attempts = 0;
         s.ndense = 0;
+#pragma unroll
+        for (int j = 0; j < kRegStages; ++j) s.k[j] = mk<R>(0, 0);
         Rng g{A.draws + (size_t)traj * A.max_draws, A.max_draws, 0};
         int jumps = 0;
-        double target = 0.0;
-        V<R, NR> y0;
-#pragma unroll
-        for (int q = 0; q < NR; ++q) {
-            const double2 p0 = c.act[q] ? A.psi0[c.row[q]] : make_double2(0.0, 0.0);
-            y0.v[q] = mk<R>((R)p0.x, (R)p0.y);
-        }
+        Uni target;
+        // s.y: the state of the next start
+        const double2 p0 = c.act ? A.psi0[row_of(c)] : make_double2(0.0, 0.0);
+        s.y = mk<R>((R)p0.x, (R)p0.y);
         if (!draw(g, target)) s.status = MC_DRAWS_EXHAUSTED;
-        if (s.status == MC_OK) set_initial_value(c, s, y0, A.times[0]);
-        if (s.status == MC_OK) write_expect(c, y0, traj, 0);
-        for (int k = 1; k < A.ntimes && s.status == MC_OK; ++k) {
-            const double tk = A.times[k];
-            // MCIntegrator.integrate (mcsolve.py:286-302)
-            // (the state at t_old is always s.y: every path below that moves
-            // t_old also moves s.y there)
-            double t_old = s.t;
-            double norm_old = norm2(c, s.y);
-            long long guard = 0;
-            while (t_old < tk && s.status == MC_OK) {
+        int k = 0;          // the next output
+        int guard = 0;      // advances since the last output
+        bool start = true, search = false;
+        int tries = 0;
+        Uni t_out = A.times[0];  // output k
+        Uni t_start = t_out, t_old = t_start, norm_old = 1.0;
+        Uni tp, tf, nold, nrm, t_guess;
+        while (s.status == MC_OK) {
+            // MCIntegrator.integrate (mcsolve.py:286-302); the state at t_old
+            // is s.y outside of the search
+            Uni n2 = -1.0;  // the norm of s.y once it is known
+            bool found = false;
+            if (start) {
+                set_initial_value(c, s, s.y, t_start);
+                start = false;
+                t_old = s.t;
+                norm_old = 1.0;  // after a jump (an output below sets it again)
+            } else {
                 if (++guard > 100000) {
                     s.status = MC_NO_PROGRESS;
                     break;
                 }
-                mcstep(c, s, tk);
+                advance(c, s, search ? (double)t_guess : (double)t_out, true);
                 if (s.status < 0) break;
-                const double t_step = s.t;
-                double nrm = norm2(c, s.y);
-                if (nrm <= target) {
-                    // _find_collapse_time (mcsolve.py:321-369)
-                    int tries = 0;
-                    double tp = t_old, tf = t_step, nold = norm_old, t_guess = tf;
-                    while (tries < A.norm_steps) {
-                        tries++;
-                        if (tf - tp < A.norm_t_tol) {
-                            t_guess = tf;
-                            break;
-                        }
+                n2 = norm2(c, s.y);
+                if (search) {
+                    if (fabs(target - n2) < A.norm_tol * target) {
+                        found = true;
+                    } else if (n2 < target) {
+                        tf = t_guess;
+                        nrm = n2;
+                    } else {
+                        tp = t_guess;
+                        nold = n2;
+                    }
+                } else if (n2 <= target) {
+                    search = true;
+                    tries = 0;
+                    tp = t_old;
+                    tf = s.t;
+                    nold = norm_old;
+                    nrm = n2;
+                    t_guess = tf;
+                } else {
+                    t_old = s.t;
+                    norm_old = n2;
+                }
+            }
+            if (search) {
+                // _find_collapse_time (mcsolve.py:321-369)
+                if (!found) {
+                    if (tries >= A.norm_steps) {
+                        s.status = MC_COLLAPSE_NOT_FOUND;
+                        break;
+                    }
+                    tries++;
+                    if (tf - tp < A.norm_t_tol) {
+                        t_guess = tf;
+                        found = true;
+                    } else {
                         const double dtc = tf - tp;
                         double ratio = log(nold / target) / log(nold / nrm);
                         if (ratio < A.norm_min_step) ratio = A.norm_min_step;
                         if (ratio > 1.0 - A.norm_min_step) ratio = 1.0 - A.norm_min_step;
                         t_guess = tp + dtc * ratio;
                         if (t_guess - tp < A.norm_t_tol) t_guess = tp + A.norm_t_tol;
-                        mcstep(c, s, t_guess);
-                        if (s.status < 0) break;
-                        const double n2g = norm2(c, s.y);
-                        if (fabs(target - n2g) < A.norm_tol * target) {
-                            break;
-                        } else if (n2g < target) {
-                            tf = t_guess;
-                            nrm = n2g;
-                        } else {
-                            tp = t_guess;
-                            nold = n2g;
-                        }
+                        continue;
                     }
-                    if (s.status < 0) break;
-                    if (tries >= A.norm_steps) {
-                        s.status = MC_COLLAPSE_NOT_FOUND;
+                }
+                if (tries >= A.norm_steps) {
+                    s.status = MC_COLLAPSE_NOT_FOUND;
+                    break;
+                }
+                // _do_collapse (mcsolve.py:371-406); the state is s.y
+                search = false;
+                const C2<R> psi = s.y;
+                stage_in(c, psi);
+                int which = 0;
+                if (A.nchan > 1) {
+                    double tot = 0.0;
+                    for (int ch = 0; ch < A.nchan; ++ch) {
+                        const int *rp = A.c_rowptr + (size_t)ch * (A.d + 1);
+                        const double pr = norm2(c, op_rows(c, rp, A.c_col, A.c_vals));
+                        if (threadIdx.x == 0) S.probs[ch] = pr;
+                        tot += pr;
+                    }
+                    __syncthreads();
+                    Uni u;
+                    if (!draw(g, u)) {
+                        s.status = MC_DRAWS_EXHAUSTED;
                         break;
                     }
-                    // _do_collapse (mcsolve.py:371-406); the state is s.y
-                    const V<R, NR> psi = s.y;
-                    stage_in(c, psi);
-                    int which = 0;
-                    if (A.nchan > 1) {
-                        double tot = 0.0;
-                        for (int ch = 0; ch < A.nchan; ++ch) {
-                            const int *rp = A.c_rowptr + (size_t)ch * (A.d + 1);
-                            const double pr = norm2(c, op_rows(c, rp, A.c_col, A.c_vals));
-                            if (threadIdx.x == 0) S.probs[ch] = pr;
-                            tot += pr;
-                        }
-                        __syncthreads();
-                        double u;
-                        if (!draw(g, u)) {
-                            s.status = MC_DRAWS_EXHAUSTED;
-                            break;
-                        }
-                        double tg = tot * u - S.probs[0];
-                        while (tg > 0.0 && which < A.nchan - 1) {
-                            which++;
-                            tg -= S.probs[which];
-                        }
+                    double tg = tot * u - S.probs[0];
+                    while (tg > 0.0 && which < A.nchan - 1) {
+                        which++;
+                        tg -= S.probs[which];
                     }
-                    const int *rp = A.c_rowptr + (size_t)which * (A.d + 1);
-                    V<R, NR> ynew = op_rows(c, rp, A.c_col, A.c_vals);
-                    const double nn = sqrt(norm2(c, ynew));
-                    if (nn < A.mc_corr_eps) {
-                        const double np = sqrt(norm2(c, psi));
-#pragma unroll
-                        for (int q = 0; q < NR; ++q) {
-                            ynew.v[q].x = (R)(psi.v[q].x / np);
-                            ynew.v[q].y = (R)(psi.v[q].y / np);
-                        }
-                    } else {
-#pragma unroll
-                        for (int q = 0; q < NR; ++q) {
-                            ynew.v[q].x = (R)(ynew.v[q].x / nn);
-                            ynew.v[q].y = (R)(ynew.v[q].y / nn);
-                        }
-                        if (threadIdx.x == 0 && jumps < A.max_jumps) {
-                            A.col_times[(size_t)traj * A.max_jumps + jumps] = t_guess;
-                            A.col_which[(size_t)traj * A.max_jumps + jumps] = which;
-                        }
-                        jumps++;
-                        if (!draw(g, target)) {
-                            s.status = MC_DRAWS_EXHAUSTED;
-                            break;
-                        }
-                    }
-                    set_initial_value(c, s, ynew, t_guess);
-                    t_old = s.t;
-                    norm_old = 1.0;
-                } else {
-                    t_old = t_step;
-                    norm_old = nrm;
                 }
+                const int *rp = A.c_rowptr + (size_t)which * (A.d + 1);
+                C2<R> ynew = op_rows(c, rp, A.c_col, A.c_vals);
+                const double nn = sqrt(norm2(c, ynew));
+                if (nn < A.mc_corr_eps) {
+                    const double np = sqrt(norm2(c, psi));
+                    ynew.x = (R)(psi.x / np);
+                    ynew.y = (R)(psi.y / np);
+                } else {
+                    ynew.x = (R)(ynew.x / nn);
+                    ynew.y = (R)(ynew.y / nn);
+                    if (threadIdx.x == 0 && jumps < A.max_jumps) {
+                        A.col_times[(size_t)traj * A.max_jumps + jumps] = t_guess;
+                        A.col_which[(size_t)traj * A.max_jumps + jumps] = which;
+                    }
+                    jumps++;
+                    if (!draw(g, target)) {
+                        s.status = MC_DRAWS_EXHAUSTED;
+                        break;
+                    }
+                }
+                s.y = ynew;
+                start = true;
+                t_start = t_guess;
+                continue;
             }
-            if (s.status != MC_OK) break;
-            write_expect(c, s.y, traj, k);
+            // the outputs reached (the first one at the start)
+            while (k < A.ntimes && (k == 0 || !(t_old < t_out))) {
+                if (n2 < 0.0) n2 = norm2(c, s.y);
+                write_expect(c, s.y, n2, traj, k);
+                norm_old = n2;
+                guard = 0;
+                if (++k < A.ntimes) t_out = A.times[k];
+            }
+            if (k >= A.ntimes) break;
         }
         if (threadIdx.x == 0) {
             A.info[(size_t)traj * 4 + 0] = s.status;
@@ -1011,20 +1129,15 @@ __global__ __launch_bounds__(RS == 0 ? 2 * kMcThreads : kMcThreads) void mc_traj
 // 0) is copied into LDS after the other arrays once per workgroup, so the
 // RHS products read it there instead of from L2 (the launcher picks this
 // when it fits the configuration's LDS budget).
-template <typename R, int NR, int RS, bool HL>
-__global__ __launch_bounds__(RS == 0 ? 2 * kMcThreads : kMcThreads) void rk_small_kernel(McArgs A) {
+template <typename R, int NT, int FM, bool HL>
+__global__ __launch_bounds__(NT) void rk_small_kernel(McArgs A) {
     extern __shared__ __align__(16) unsigned char mc_dyn_lds[];
-    __shared__ McTableau T;
+    __shared__ double bi[kMcStages][kMcOrder];
     McLds<R> S;
-    kernel_prologue<R, NR, RS>(A, mc_dyn_lds, T, S);
-    Ctx<R, NR, RS> c{A, S, T};
+    unsigned char *tail = kernel_prologue<R, NT, FM>(A, mc_dyn_lds, bi, S);
+    Ctx<R, NT, FM> c{A, S, bi};
     const int *lcol = nullptr;
     const C2<R> *lval = nullptr;
-    unsigned char *tail = align16(S.rsum + 4 * (blockDim.x / QA_WAVE));
-    if (A.x2) {  // the launcher reserved the second input buffer here
-        S.xalt = (C2<R> *)tail;
-        tail += sizeof(C2<R>) * (size_t)S.npad;
-    }
     if constexpr (HL) {
         const int nent = A.h_width * A.d;
         C2<R> *v = (C2<R> *)tail;
@@ -1081,30 +1194,27 @@ __global__ __launch_bounds__(RS == 0 ? 2 * kMcThreads : kMcThreads) void rk_smal
             ctx_rows(c, lcol, (const void *)lval);
         else
             ctx_rows(c, A.h_col + hoff, (const void *)((const C2<R> *)A.h_vals + hoff));
-        Traj<R, NR, RS> s;
+        Traj<R> s;
         s.status = MC_OK;
         s.attempts = 0;
         s.ndense = 0;
-        V<R, NR> y0;
 #pragma unroll
-        for (int q = 0; q < NR; ++q) {
-            const double2 p0 =
-                c.act[q] ? A.psi0[(size_t)sys * A.d + c.row[q]] : make_double2(0.0, 0.0);
-            y0.v[q] = mk<R>((R)p0.x, (R)p0.y);
-        }
+        for (int j = 0; j < kRegStages; ++j) s.k[j] = mk<R>(0, 0);
+        C2<R> y0;
+        const double2 p0 =
+            c.act ? A.psi0[(size_t)sys * A.d + row_of(c)] : make_double2(0.0, 0.0);
+        y0 = mk<R>((R)p0.x, (R)p0.y);
         set_initial_value(c, s, y0, A.t0);
         int k = 0;
         for (; k < A.ntimes && s.status >= 0; ++k) {
-            integrate_to(c, s, times[k]);
+            advance(c, s, times[k], false);
             if (s.status < 0) break;
             write_functionals(c, s.y, fv, A.fun_out + ((size_t)sys * A.ntimes + k) * A.nfun);
         }
         if (A.y_final) {
-#pragma unroll
-            for (int q = 0; q < NR; ++q)
-                if (c.act[q])
-                    A.y_final[(size_t)sys * A.d + c.row[q]] =
-                        make_double2((double)s.y.v[q].x, (double)s.y.v[q].y);
+            if (c.act)
+                A.y_final[(size_t)sys * A.d + row_of(c)] =
+                    make_double2((double)s.y.x, (double)s.y.y);
         }
         if (threadIdx.x == 0) {
             A.info[(size_t)sys * 4 + 0] = s.status;
@@ -1117,13 +1227,14 @@ __global__ __launch_bounds__(RS == 0 ? 2 * kMcThreads : kMcThreads) void rk_smal
 }
 
 constexpr size_t kLdsBudget = 160 * 1024;  // LDS of one gfx950 CU
+constexpr int kChipCUs = 256;
 
 constexpr size_t kFunLdsMax = 16 * 1024;  // LDS for the functionals and times
 
-// Static LDS of both kernels (the `__shared__ McTableau T`), rounded up to
+// Static LDS of both kernels (the dense-output polynomials), rounded up to
 // the 16-byte granule the dynamic part starts on.  Every budget below counts
 // it: a workgroup's LDS is the static part plus the dynamic bytes.
-constexpr size_t kLdsStatic = (sizeof(McTableau) + 15) & ~(size_t)15;
+constexpr size_t kLdsStatic = (sizeof(double) * kMcStages * kMcOrder + 15) & ~(size_t)15;
 
 // The LDS plan of one launch: dynamic bytes, the operator in LDS (HL), and
 // the bytes reserved for functionals and times.
@@ -1132,26 +1243,32 @@ struct McPlan {
     bool hl;      // the shared ELL operator is staged in LDS
     int fun_lds;  // bytes for the functionals and times (0: none)
     bool x2;      // a second input buffer (one barrier per product instead of two)
+    bool pk;      // the packed operator is used (its values in LDS)
 };
 
-// RS == 0 runs two workgroups per CU, so each gets half of the CU's LDS,
-// its static part included.
-inline size_t mc_lds_cap(int RS) {
-    return (RS == 0 ? kLdsBudget / 2 : kLdsBudget) - kLdsStatic;
-}
+inline size_t mc_lds_cap() { return kLdsBudget - kLdsStatic; }
 
 template <typename R>
-McPlan plan_mc(const McArgs &A, int threads, int NR, int RS, bool small) {
+McPlan plan_mc(const McArgs &A, int threads, bool small) {
     McPlan P;
-    P.lds = mc_lds_bytes<R>(threads * NR, threads, RS);
+    P.lds = mc_lds_bytes<R>(threads);
     P.hl = false;
     P.fun_lds = 0;
     P.x2 = false;
-    const size_t cap = mc_lds_cap(RS);
-    if (small && A.h_stride == 0 && A.h_width > 0) {
-        // the shared operator in LDS when it fits the budget of this shape
+    const size_t cap = mc_lds_cap();
+    P.pk = false;
+    if (A.pk_code) {
+        const size_t tab = 16 + 2 * sizeof(R) * (size_t)A.pk_ntab;
+        if (P.lds + tab <= cap) {
+            P.lds += tab;
+            P.pk = true;
+        }
+    }
+    if (small && !P.pk && A.h_stride == 0 && A.h_width > 0) {
+        // the shared operator in LDS when it fits, beside a second workgroup
+        // where the systems are more than the CUs
         const size_t ell = (size_t)A.h_width * A.d * (sizeof(C2<R>) + sizeof(int));
-        if (P.lds + ell <= cap) {
+        if (P.lds + ell <= (A.ntraj > kChipCUs ? kLdsBudget / 2 - kLdsStatic : cap)) {
             P.lds += ell;
             P.hl = true;
         }
@@ -1159,7 +1276,7 @@ McPlan plan_mc(const McArgs &A, int threads, int NR, int RS, bool small) {
     {
         // the second input buffer (with 16 bytes for its alignment) when it
         // fits and keeps the number of workgroups an LDS-limited CU holds
-        const size_t xb = 16 + sizeof(C2<R>) * (size_t)threads * NR;
+        const size_t xb = 16 + sizeof(C2<R>) * (size_t)threads;
         if (P.lds + xb <= cap &&
             kLdsBudget / (P.lds + xb + kLdsStatic) == kLdsBudget / (P.lds + kLdsStatic)) {
             P.lds += xb;
@@ -1183,72 +1300,63 @@ McPlan plan_mc(const McArgs &A, int threads, int NR, int RS, bool small) {
     return P;
 }
 
-template <typename R, int NR, int RS, bool SMALL>
+template <typename R, int NT, bool SMALL>
 int launch_mc_cfg(const McArgs &A0, int threads, int blocks, hipStream_t s) {
     McArgs A = A0;
-    const McPlan P = plan_mc<R>(A, threads, NR, RS, SMALL);
-    if (P.lds > mc_lds_cap(RS)) {
+    const McPlan P = plan_mc<R>(A, threads, SMALL);
+    if (P.lds > mc_lds_cap()) {
         qa::set_error("trajectory kernel: %zu B of dynamic LDS exceed the %zu B budget", P.lds,
-                      mc_lds_cap(RS));
+                      mc_lds_cap());
         return QA_ERR_ARG;
     }
     A.fun_lds = P.fun_lds;
     A.x2 = P.x2 ? 1 : 0;
     const size_t lds = P.lds;
     const bool hl = P.hl;
-    const void *fn = !SMALL ? (const void *)mc_traj_kernel<R, NR, RS>
-                     : hl   ? (const void *)rk_small_kernel<R, NR, RS, true>
-                            : (const void *)rk_small_kernel<R, NR, RS, false>;
-    QA_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    if (!SMALL)
-        hipLaunchKernelGGL((mc_traj_kernel<R, NR, RS>), dim3(blocks), dim3(threads), lds, s, A);
-    else if (hl)
-        hipLaunchKernelGGL((rk_small_kernel<R, NR, RS, true>), dim3(blocks), dim3(threads), lds,
-                           s, A);
+    const int fm = !P.pk ? OP_ELL : A.pk_imag ? OP_PACKED_IM : OP_PACKED;
+    const void *fn;
+    if constexpr (!SMALL)
+        fn = fm == OP_PACKED_IM ? (const void *)mc_traj_kernel<R, NT, OP_PACKED_IM>
+             : fm == OP_PACKED  ? (const void *)mc_traj_kernel<R, NT, OP_PACKED>
+                                : (const void *)mc_traj_kernel<R, NT, OP_ELL>;
     else
-        hipLaunchKernelGGL((rk_small_kernel<R, NR, RS, false>), dim3(blocks), dim3(threads), lds,
-                           s, A);
+        fn = fm == OP_PACKED_IM ? (const void *)rk_small_kernel<R, NT, OP_PACKED_IM, false>
+             : fm == OP_PACKED  ? (const void *)rk_small_kernel<R, NT, OP_PACKED, false>
+             : hl               ? (const void *)rk_small_kernel<R, NT, OP_ELL, true>
+                                : (const void *)rk_small_kernel<R, NT, OP_ELL, false>;
+    QA_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    void *args[] = {(void *)&A};
+    QA_HIP(hipLaunchKernel(fn, dim3(blocks), dim3(threads), args, lds, s));
     QA_CHECK_LAUNCH();
     return QA_OK;
 }
 
-// Launch shape (measured on the TFIM trajectories at d = 512 and 1024):
-// (threads, rows per thread NR, register stages RS) for d rows, false when
-// d does not fit.  Every stage in LDS, one row per thread, when the 18
-// vectors take at most half of the LDS: two workgroups then share a CU,
-// which beats keeping the step stages in registers.  Otherwise the step
-// stages stay in registers, one row per thread up to 512 rows and two rows
-// per thread above.
+// Threads for d rows, one row each; false when d does not fit.
 template <typename R>
-bool shape_mc(int d, int *threads, int *NR, int *RS) {
-    const int t1 = ((d + QA_WAVE - 1) / QA_WAVE) * QA_WAVE;
-    if (t1 <= 2 * kMcThreads && mc_lds_bytes<R>(t1, t1, 0) <= mc_lds_cap(0)) {
-        *threads = t1, *NR = 1, *RS = 0;
-        return true;
-    }
-    if (t1 <= kMcThreads && mc_lds_bytes<R>(t1, t1, kRegStagesMax) <= mc_lds_cap(kRegStagesMax)) {
-        *threads = t1, *NR = 1, *RS = kRegStagesMax;
-        return true;
-    }
-    const int rows = (d + 1) / 2;
-    const int t2 = ((rows + QA_WAVE - 1) / QA_WAVE) * QA_WAVE;
-    if (t2 > kMcThreads ||
-        mc_lds_bytes<R>(2 * t2, t2, kRegStagesMax) > mc_lds_cap(kRegStagesMax))
-        return false;
-    *threads = t2, *NR = 2, *RS = kRegStagesMax;
-    return true;
+bool shape_mc(int d, int *threads) {
+    const int t = ((d + QA_WAVE - 1) / QA_WAVE) * QA_WAVE;
+    if (t > kMcThreads) return false;
+    *threads = t;
+    return mc_lds_bytes<R>(t) <= mc_lds_cap();
 }
 
+// The kernels are compiled for up to 1024 threads (128 vector registers each,
+// so 16 waves a CU), and the whole-solve kernel also for up to 512 (256
+// registers, 8 waves a CU, nothing spilled): that form is the faster one
+// where no CU gets a second workgroup (400 rows, one system: 2.96 ms against
+// 3.23).  Trajectories come in numbers: 512 of 512 rows 3.3 ms with 1024, 4.2
+// with 512, and 8192 of 256 rows 16 against 24 ms; 500 of them are equal.
 template <typename R, bool SMALL = false>
 int launch_mc(const McArgs &A, int blocks, hipStream_t s) {
-    int threads, NR, RS;
-    if (!shape_mc<R>(A.d, &threads, &NR, &RS)) {
+    int threads;
+    if (!shape_mc<R>(A.d, &threads)) {
         qa::set_error("qa_mc_run: d = %d does not fit the trajectory kernel", A.d);
         return QA_ERR_ARG;
     }
-    if (NR == 1 && RS == 0) return launch_mc_cfg<R, 1, 0, SMALL>(A, threads, blocks, s);
-    if (NR == 1) return launch_mc_cfg<R, 1, kRegStagesMax, SMALL>(A, threads, blocks, s);
-    return launch_mc_cfg<R, 2, kRegStagesMax, SMALL>(A, threads, blocks, s);
+    if constexpr (SMALL)
+        if (threads <= kMcThreads / 2 && blocks <= kChipCUs)
+            return launch_mc_cfg<R, kMcThreads / 2, SMALL>(A, threads, blocks, s);
+    return launch_mc_cfg<R, kMcThreads, SMALL>(A, threads, blocks, s);
 }
 
 }  // namespace
@@ -1267,23 +1375,22 @@ int qa_mc_lds_plan(int d, int h_width, int nfun, int ntimes, int fp32, int small
     A.h_width = h_width;
     A.nfun = nfun;
     A.ntimes = ntimes;
-    int threads, NR, RS;
-    const bool ok = fp32 ? shape_mc<float>(d, &threads, &NR, &RS)
-                         : shape_mc<double>(d, &threads, &NR, &RS);
+    int threads;
+    const bool ok = fp32 ? shape_mc<float>(d, &threads) : shape_mc<double>(d, &threads);
     if (!ok) {
         qa::set_error("qa_mc_lds_plan: d = %d does not fit the trajectory kernel", d);
         return QA_ERR_ARG;
     }
-    const McPlan P = fp32 ? plan_mc<float>(A, threads, NR, RS, small != 0)
-                          : plan_mc<double>(A, threads, NR, RS, small != 0);
+    const McPlan P = fp32 ? plan_mc<float>(A, threads, small != 0)
+                          : plan_mc<double>(A, threads, small != 0);
     out[0] = threads;
-    out[1] = NR;
-    out[2] = RS;
+    out[1] = 1;  // rows per thread
+    out[2] = kRegStages;
     out[3] = (long long)P.lds;
     out[4] = (long long)kLdsStatic;
     out[5] = P.hl ? 1 : 0;
     out[6] = P.fun_lds;
-    out[7] = (long long)mc_lds_cap(RS);
+    out[7] = (long long)mc_lds_cap();
     return QA_OK;
 }
 
@@ -1324,6 +1431,31 @@ int qa_mc_pack_tableau(void *out, int order, int rk_step, int rk_extra, int dord
     return QA_OK;
 }
 
+static int packed_args(McArgs &A, const qa_packed_op *op) {
+    A.pk_code = nullptr;
+    A.pk_diag = A.pk_tab = nullptr;
+    A.pk_width = A.pk_cbits = A.pk_ntab = A.pk_imag = 0;
+    if (!op) return QA_OK;
+    QA_REQUIRE(op->code && op->diag && op->table, "packed operator: null pointer");
+    QA_REQUIRE(op->width >= 0 && op->width <= kMcPack && op->width % 2 == 0,
+               "packed operator: width must be even, at most %d", kMcPack);
+    QA_REQUIRE(op->cbits >= 1 && op->cbits <= 15 && A.d <= (1 << op->cbits),
+               "packed operator: columns must fit cbits");
+    QA_REQUIRE(op->ntab >= 1 && op->ntab <= kMcPackTab && op->ntab <= (1 << (16 - op->cbits)),
+               "packed operator: 1 <= ntab <= %d", kMcPackTab);
+    QA_REQUIRE(op->rk_step == kPackStep && op->rk_extra == kPackExtra,
+               "packed operator: for tableaus of %d stages, %d with the dense output", kPackStep,
+               kPackExtra);
+    A.pk_code = (const unsigned short *)op->code;
+    A.pk_diag = op->diag;
+    A.pk_tab = op->table;
+    A.pk_width = op->width;
+    A.pk_cbits = op->cbits;
+    A.pk_ntab = op->ntab;
+    A.pk_imag = op->imag;
+    return QA_OK;
+}
+
 int qa_mc_run(int d, int ntraj, int ntimes, const double *times_dev, const void *psi0_dev,
               int h_width, const int *h_col, const void *h_vals, int nchan,
               const int *c_rowptr, const int *c_col, const void *c_vals, int neops,
@@ -1334,8 +1466,26 @@ int qa_mc_run(int d, int ntraj, int ntimes, const double *times_dev, const void 
               double norm_min_step, double mc_corr_eps, int fp32, void *expect_out_dev,
               double *col_times_dev, int *col_which_dev, int max_jumps, int *info_dev,
               int grid, void *stream) {
-    QA_REQUIRE(d >= 1 && d <= 2 * kMcThreads, "qa_mc_run: 1 <= d <= %d (rows held per thread)",
-               2 * kMcThreads);
+    return qa_mc_run_packed(nullptr, d, ntraj, ntimes, times_dev, psi0_dev, h_width, h_col, h_vals,
+                            nchan, c_rowptr, c_col, c_vals, neops, e_rowptr, e_col, e_vals,
+                            tableau_dev, draws_dev, max_draws, rtol, atol, nsteps, first_step,
+                            min_step, max_step, norm_steps, norm_t_tol, norm_tol, norm_min_step,
+                            mc_corr_eps, fp32, expect_out_dev, col_times_dev, col_which_dev,
+                            max_jumps, info_dev, grid, stream);
+}
+
+int qa_mc_run_packed(const qa_packed_op *packed, int d, int ntraj, int ntimes,
+              const double *times_dev, const void *psi0_dev, int h_width, const int *h_col, const void *h_vals, int nchan,
+              const int *c_rowptr, const int *c_col, const void *c_vals, int neops,
+              const int *e_rowptr, const int *e_col, const void *e_vals,
+              const void *tableau_dev, const double *draws_dev, int max_draws,
+              double rtol, double atol, int nsteps, double first_step, double min_step,
+              double max_step, int norm_steps, double norm_t_tol, double norm_tol,
+              double norm_min_step, double mc_corr_eps, int fp32, void *expect_out_dev,
+              double *col_times_dev, int *col_which_dev, int max_jumps, int *info_dev,
+              int grid, void *stream) {
+    QA_REQUIRE(d >= 1 && d <= kMcThreads, "qa_mc_run: 1 <= d <= %d (rows held per thread)",
+               kMcThreads);
     QA_REQUIRE(ntraj >= 0 && ntimes >= 1, "qa_mc_run: need ntimes >= 1");
     QA_REQUIRE(nchan >= 1 && nchan <= kMcMaxChan, "qa_mc_run: 1 <= nchan <= %d", kMcMaxChan);
     QA_REQUIRE(neops >= 0 && neops <= kMcMaxEops, "qa_mc_run: neops <= %d", kMcMaxEops);
@@ -1349,7 +1499,9 @@ int qa_mc_run(int d, int ntraj, int ntimes, const double *times_dev, const void 
                "qa_mc_run: null pointer");
     if (ntraj == 0) return QA_OK;
     McArgs A;
+    memset(&A, 0, sizeof(A));
     A.d = d;
+    QA_CHECK(packed_args(A, packed));
     A.ntraj = ntraj;
     A.ntimes = ntimes;
     A.nchan = nchan;
@@ -1399,7 +1551,20 @@ int qa_rk_small_run(int n, int nsys, double t0, int ntimes, const double *times_
                     double rtol, double atol, int nsteps, double first_step, double min_step,
                     double max_step, int fp32, void *fun_out_dev, void *y_final_dev,
                     int *info_dev, int grid, void *stream) {
-    QA_REQUIRE(n >= 1 && n <= 2 * kMcThreads, "qa_rk_small_run: 1 <= n <= %d", 2 * kMcThreads);
+    return qa_rk_small_run_packed(nullptr, n, nsys, t0, ntimes, times_dev, y0_dev, h_width, h_col,
+                                  h_vals, h_stride, nfun, fkind, fptr, frows, fcols, fw,
+                                  tableau_dev, rtol, atol, nsteps, first_step, min_step, max_step,
+                                  fp32, fun_out_dev, y_final_dev, info_dev, grid, stream);
+}
+
+int qa_rk_small_run_packed(const qa_packed_op *packed, int n, int nsys, double t0, int ntimes,
+                    const double *times_dev, const void *y0_dev, int h_width, const int *h_col, const void *h_vals,
+                    long long h_stride, int nfun, const int *fkind, const int *fptr,
+                    const int *frows, const int *fcols, const void *fw, const void *tableau_dev,
+                    double rtol, double atol, int nsteps, double first_step, double min_step,
+                    double max_step, int fp32, void *fun_out_dev, void *y_final_dev,
+                    int *info_dev, int grid, void *stream) {
+    QA_REQUIRE(n >= 1 && n <= kMcThreads, "qa_rk_small_run: 1 <= n <= %d", kMcThreads);
     QA_REQUIRE(nsys >= 0 && ntimes >= 0 && nfun >= 0, "qa_rk_small_run: negative size");
     QA_REQUIRE(h_width >= 0 && h_width % 4 == 0 && h_width <= n + 3 && h_stride >= 0,
                "qa_rk_small_run: h_width must be a multiple of 4, at most n + 3");
@@ -1412,6 +1577,8 @@ int qa_rk_small_run(int n, int nsys, double t0, int ntimes, const double *times_
     McArgs A;
     memset(&A, 0, sizeof(A));
     A.d = n;
+    QA_REQUIRE(!packed || h_stride == 0, "qa_rk_small_run_packed: one operator for every system");
+    QA_CHECK(packed_args(A, packed));
     A.ntraj = nsys;
     A.ntimes = ntimes;
     A.h_width = h_width;

@@ -214,6 +214,82 @@ def _ell_block(A, d, fp32):
             _data.DeviceBuffer.from_array(np.ascontiguousarray(val)))
 
 
+PACK_WIDTH = 16   # off-diagonal entries a row (kMcPack)
+PACK_VALUES = 256  # distinct off-diagonal values (kMcPackTab)
+PACK_STAGES = (10, 16)  # stages of the tableau, without and with the dense output
+
+
+class _PackedOp(C.Structure):
+    """qa_packed_op of the C ABI."""
+    _fields_ = [("code", C.c_void_p), ("diag", C.c_void_p), ("table", C.c_void_p),
+                ("width", C.c_int), ("cbits", C.c_int), ("ntab", C.c_int), ("imag", C.c_int),
+                ("rk_step", C.c_int), ("rk_extra", C.c_int)]
+
+
+def _packed_host(A, d, fp32):
+    """The packed form of a d x d operator (qa_packed_op): (codes uint16
+    [width, d], diagonal, table, column bits, imag), or None when a row has
+    more than 16 off-diagonal entries or the values do not fit the codes.
+    A row's entries are ordered by their distance from the diagonal, so the
+    lanes of a wave mostly read one value and shifted runs of the vector."""
+    A = sp.csr_matrix(A, dtype=np.complex64 if fp32 else np.complex128)
+    A = A.copy()
+    A.sum_duplicates()
+    n = np.repeat(np.arange(d), np.diff(A.indptr))
+    diag = np.zeros(d, dtype=A.dtype)
+    on = A.indices == n
+    diag[n[on]] = A.data[on]
+    off = ~on & (A.data != 0)
+    rows, cols, vals = n[off], A.indices[off].astype(np.int64), A.data[off]
+    counts = np.bincount(rows, minlength=d)
+    width = -(-int(counts.max()) // 2) * 2 if len(rows) else 0
+    cbits = max(1, int(d - 1).bit_length())
+    if width > PACK_WIDTH or cbits > 15:
+        return None
+    table, inv = np.unique(np.concatenate([np.zeros(1, A.dtype), vals]), return_inverse=True)
+    zero = int(inv[0])
+    if zero != 0:  # the padding value is entry 0
+        table[[0, zero]] = table[[zero, 0]]
+        inv = np.where(inv == zero, 0, np.where(inv == 0, zero, inv))
+    if len(table) > min(PACK_VALUES, 1 << (16 - cbits)):
+        return None
+    order = np.lexsort((cols - rows, np.abs(cols - rows), rows))
+    rows, cols, idx = rows[order], cols[order], inv[1:].reshape(-1)[order]
+    start = np.concatenate([[0], np.cumsum(counts)[:-1]])
+    slot = np.arange(len(rows)) - start[rows]
+    codes = np.tile(np.arange(d, dtype=np.uint16), (max(width, 1), 1))
+    codes[slot, rows] = (cols | (idx << cbits)).astype(np.uint16)
+    imag = bool((table.real == 0).all())
+    table = np.ascontiguousarray(table.imag if imag else table)
+    return codes[:max(width, 1)], diag, table, width, cbits, imag
+
+
+class PackedOp:
+    """A packed operator on the device (``ref``: the struct for the C ABI)."""
+
+    def __init__(self, host):
+        codes, diag, table, width, cbits, imag = host
+        self._bufs = [_data.DeviceBuffer.from_array(np.ascontiguousarray(a))
+                      for a in (codes, diag, table)]
+        self.struct = _PackedOp(*[b.ptr for b in self._bufs], width, cbits, len(table), int(imag),
+                                *PACK_STAGES)
+
+    @property
+    def ref(self):
+        return C.cast(C.pointer(self.struct), C.c_void_p)
+
+
+def packed_op(A, d, fp32, tab, interpolate):
+    """The packed form of A uploaded, or None: also where the tableau is not
+    one the packed kernels are compiled for (vern7's shape)."""
+    a, b = (np.asarray(tab[k], dtype=np.float64) for k in ("a", "b"))
+    if (tab["e"] is None or not interpolate or (len(b), len(tab["c"])) != PACK_STAGES
+            or np.allclose(a[len(b) - 1, :len(b)], b, rtol=1e-5, atol=1e-14)):
+        return None
+    host = _packed_host(A, d, fp32)
+    return PackedOp(host) if host is not None else None
+
+
 class MCSolver:
     """Monte-Carlo wave-function solver, all trajectories in one persistent
     kernel.  ``options`` keys as qutip's MCSolver.solver_options
@@ -310,7 +386,8 @@ class MCSolver:
                       len(b), len(cc), bi.shape[1], _dp(a), _dp(b), _dp(cc), _dp(e), _dp(bi),
                       int(bool(self.options["interpolate"])))
             tab_dev = _data.DeviceBuffer.from_array(buf)
-            self._dev = (fp32, h, c, tab_dev)
+            packed = packed_op(self.H_eff, self.d, fp32, tab, self.options["interpolate"])
+            self._dev = (fp32, h, c, tab_dev, packed)
         return self._dev
 
     def run_batch(self, psi0, tlist, e_ops, draws, max_jumps=64, fp32=None):
@@ -334,10 +411,11 @@ class MCSolver:
             ntraj, max_draws = draws.shape
             dr = _data.DeviceBuffer.from_array(np.ascontiguousarray(draws))
         ntimes = len(tlist)
-        _, h, c, tab = self._device_ops(fp32)
+        ops = self._device_ops(fp32)
+        _, h, c, tab, packed = ops
         e = _csr_block([O.to_csr() for O in e_ops] or [sp.identity(self.d)], self.d, fp32)
         neops = len(e_ops)
-        H = {"e": e, "dr": dr, "ntraj": ntraj, "ntimes": ntimes, "neops": neops,
+        H = {"ops": ops, "e": e, "dr": dr, "ntraj": ntraj, "ntimes": ntimes, "neops": neops,
              "max_jumps": max_jumps, "stream": stream}
         H["times"] = _data.DeviceBuffer.from_array(np.asarray(tlist, dtype=np.float64))
         H["p0"] = _data.DeviceBuffer.from_array(np.ascontiguousarray(np.asarray(psi0).ravel(),
@@ -347,8 +425,9 @@ class MCSolver:
         H["cw"] = _data.DeviceBuffer(4 * ntraj * max_jumps)
         H["info"] = _data.DeviceBuffer(16 * ntraj)
         L = _lib.lib()
-        rc = L.qa_mc_run(
-            self.d, ntraj, ntimes, _vp(H["times"].ptr), _vp(H["p0"].ptr), int(h[0]),
+        rc = L.qa_mc_run_packed(
+            packed.ref if packed is not None else None, self.d, ntraj, ntimes,
+            _vp(H["times"].ptr), _vp(H["p0"].ptr), int(h[0]),
             _vp(h[1].ptr), _vp(h[2].ptr), len(self.c_ops), _vp(c[0].ptr), _vp(c[1].ptr),
             _vp(c[2].ptr), neops, _vp(e[0].ptr), _vp(e[1].ptr), _vp(e[2].ptr), _vp(tab.ptr),
             _vp(dr.ptr), max_draws, float(o["rtol"]), float(o["atol"]), int(o["nsteps"]),
@@ -357,7 +436,7 @@ class MCSolver:
             float(o["norm_min_step"]), float(o["mc_corr_eps"]), int(fp32), _vp(H["ex"].ptr),
             _vp(H["ct"].ptr), _vp(H["cw"].ptr), max_jumps, _vp(H["info"].ptr), int(o["grid"]),
             stream)
-        _lib.check(rc, "qa_mc_run")
+        _lib.check(rc, "qa_mc_run_packed")
         return H
 
     def collect_async(self, H, with_jumps=False):

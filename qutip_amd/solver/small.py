@@ -17,7 +17,7 @@ import scipy.sparse as sp
 
 from .. import _lib
 from .. import data as _data
-from .mcsolve import _ell_host
+from .mcsolve import _ell_host, packed_op
 from .tableaus import TABLEAUS
 
 __all__ = ["SmallSolve", "MAX_N"]
@@ -70,7 +70,10 @@ class SmallSolve:
         self.stride = max(W, 1) * n if self.nops > 1 else 0
         self._col = _data.DeviceBuffer.from_array(np.ascontiguousarray(np.concatenate(cols)))
         self._val = _data.DeviceBuffer.from_array(np.ascontiguousarray(np.concatenate(vals)))
+        # one operator for every system: its packed form too, where it has one
         self._tab, self.tableau = _pack_tableau(tableau, interpolate)
+        self._packed = (packed_op(ops[0], n, self.fp32, self.tableau, interpolate)
+                        if self.nops == 1 else None)
         self.opts = dict(rtol=float(rtol), atol=float(atol), nsteps=int(nsteps),
                          first_step=float(first_step), min_step=float(min_step),
                          max_step=float(max_step))
@@ -140,14 +143,15 @@ class SmallSolve:
              "yfin": yfin if yfin is not None else _data.DeviceBuffer(16 * nsys * self.n),
              "info": self._scratch("info", 16 * max(nsys, 1), reuse)}
         o = self.opts
-        rc = _lib.lib().qa_rk_small_run(
-            self.n, nsys, float(t0), nt, _vp(H["times"].ptr), _vp(y0buf.ptr), self.width,
+        rc = _lib.lib().qa_rk_small_run_packed(
+            self._packed.ref if self._packed is not None else None, self.n, nsys, float(t0), nt,
+            _vp(H["times"].ptr), _vp(y0buf.ptr), self.width,
             _vp(self._col.ptr), _vp(self._val.ptr), self.stride, self.nfun, _vp(self._fk.ptr),
             _vp(self._fp.ptr), _vp(self._fr.ptr), _vp(self._fc.ptr), _vp(self._fw.ptr),
             _vp(self._tab.ptr), o["rtol"], o["atol"], o["nsteps"], o["first_step"],
             o["min_step"], o["max_step"], int(self.fp32), _vp(H["out"].ptr),
             _vp(H["yfin"].ptr), _vp(H["info"].ptr), int(grid), stream)
-        _lib.check(rc, "qa_rk_small_run")
+        _lib.check(rc, "qa_rk_small_run_packed")
         return H
 
     def collect(self, H):
