@@ -324,6 +324,9 @@ struct DenseOp {
     const float2 *Hm, *Hp, *C, *Cd;  // N x N each; C / Cd: nc blocks
     float2 *T;                        // nc blocks of scratch
     float2 *Xf;                       // the stage input in complex64 (tiled path)
+    float2 *part;                     // [hgroups][upper tiles][kGT^2] partial tiles
+    unsigned *arrived;                // [upper tiles] workgroups that stored theirs
+    int hgroups;  // workgroups that share the products of an upper 32 x 32 tile
 };
 
 __device__ __forceinline__ float2 tof(double2 a) { return make_float2((float)a.x, (float)a.y); }
@@ -581,19 +584,31 @@ __global__ __launch_bounds__(64 * kMaxSplit) void rk_dense_stage_kernel(EpiArgs 
 }
 
 // ---- large N: 32 x 32 workgroup tiles through LDS ------------------------
-// A workgroup of 4 waves owns a 32 x 32 output tile (each wave one 16 x 16
-// MFMA tile).  K goes in chunks of 64: the 256 threads load the A chunk
-// (32 rows x 64 k, one 256-byte column piece per k) and the B chunk (64 k x
-// 32 columns, one 512-byte piece per column) into LDS, the next chunk's loads are issued before the current
-// chunk's MFMAs (one chunk of register prefetch, double-buffered LDS), and
-// every A and B element loaded serves two waves.  All products of a stage
-// run through one flattened chunk loop, so one memory latency is exposed
-// per stage.  Used for N >= kTiledN, where the one-tile-per-workgroup
-// kernels above re-read every operand row and column 32 times from L2.
+// Half a workgroup (4 waves) owns a 32 x 32 output tile (each wave one
+// 16 x 16 MFMA tile).  K goes in chunks of 32: the 256 threads load the A
+// chunk (32 rows x 32 k, one 256-byte column piece per k) and the B chunk
+// (32 k x 32 columns, one 256-byte piece per column) into LDS, the next
+// chunk's loads are issued before the current chunk's MFMAs (one chunk of
+// register prefetch, double-buffered LDS), and every A and B element loaded
+// serves two waves.  All products of a workgroup run through one flattened
+// chunk loop, so one memory latency is exposed per stage.  Chunks of 64 took
+// 137 KB of LDS, one workgroup a CU, whose waves all wait at once; with 32
+// two fit (69 KB): C_c X for N = 512, nc = 3 went from 51 to 29 us.  Used for
+// N >= kTiledN, where the one-tile-per-workgroup kernels above re-read every
+// operand row and column 32 times from L2.
 constexpr int kGT = 32;      // output tile edge per workgroup
-constexpr int kGK = 64;      // K chunk
+constexpr int kGK = 32;      // K chunk
 constexpr int kGP = 2;       // LDS row padding (float2) against bank conflicts
 constexpr int kTiledN = 384;
+constexpr int kTiledStep = 64;  // the tiled path takes multiples of this
+
+// Workgroups that share the products of one upper tile: two workgroups fit a
+// CU, so 512 run at once, and fewer tiles than that leave CUs idle.
+__host__ inline int herm_groups(int N, int nc) {
+    const int tiles = (N / kGT) * (N / kGT + 1) / 2;
+    if (tiles >= 512) return 1;
+    return std::min(2 + nc, (1024 + tiles - 1) / tiles);
+}
 
 struct GemmTile {
     float2 a[2][kGK][kGT + kGP];  // a[buf][k][i]
@@ -703,9 +718,9 @@ struct GemmShared {
     GemmTile L[kGHalves];
 };
 
-// Product p's operands: p < 0 selects the T kernel's single product C_c X.
+// The products p0 .. p0 + np - 1 of a stage, or A0 B0 (the T kernel's C_c X).
 template <typename TB, int NP>
-__device__ __forceinline__ void gt_run(const DenseOp &D, GemmShared &G, int np,
+__device__ __forceinline__ void gt_run(const DenseOp &D, GemmShared &G, int p0, int np,
                                        const float2 *A0, const TB *B0, int i0, int j0,
                                        v4f &re, v4f &im) {
     const int h = threadIdx.x >> 8, tid = threadIdx.x & 255;
@@ -714,7 +729,7 @@ __device__ __forceinline__ void gt_run(const DenseOp &D, GemmShared &G, int np,
     const int trips = (total + kGHalves - 1) / kGHalves;
     GemmTile &L = G.L[h];
     auto operands = [&](int idx, const float2 *&A, const TB *&B, int &k0) {
-        const int p = idx / nch;
+        const int p = p0 + idx / nch;
         k0 = (idx % nch) * kGK;
         if (A0) {
             A = A0;
@@ -776,7 +791,7 @@ __device__ __forceinline__ void dense_t_tiled(const DenseOp &D, const double2 *X
     }
     if (c >= D.nc) return;  // uniform over the workgroup
     v4f re = {0.f, 0.f, 0.f, 0.f}, im = {0.f, 0.f, 0.f, 0.f};
-    gt_run<double2, NP>(D, G, 1, D.C + (size_t)c * NN, X, i0, j0, re, im);
+    gt_run<double2, NP>(D, G, 0, 1, D.C + (size_t)c * NN, X, i0, j0, re, im);
     if ((threadIdx.x >> 8) != 0) return;
     const int lane = threadIdx.x & 63, w = (threadIdx.x & 255) >> 6;
 #pragma unroll
@@ -789,7 +804,7 @@ __device__ __forceinline__ void dense_t_tiled(const DenseOp &D, const double2 *X
 template <int NP>
 __device__ __forceinline__ void dense_k_tiled(const DenseOp &D, GemmShared &G, v4f &re,
                                               v4f &im) {
-    gt_run<float2, NP>(D, G, 2 + D.nc, nullptr, (const float2 *)nullptr, blockIdx.x * kGT,
+    gt_run<float2, NP>(D, G, 0, 2 + D.nc, nullptr, (const float2 *)nullptr, blockIdx.x * kGT,
                    blockIdx.y * kGT, re, im);
 }
 
@@ -1080,14 +1095,95 @@ __global__ __launch_bounds__(512 / IPT) void rk_dense_herm_stage_kernel(EpiArgs 
     }
 }
 
-// The same on the upper 32 x 32 workgroup tiles of the LDS-staged path
-// (N >= kTiledN): 2 E^2 items over 512 threads.
+// The same with the products of a tile shared by up to 16 waves: wave
+// w = u + ns g takes part u of K in products g, g + ng, ...  With few tiles
+// (36 at N = 128) the waves are alone on their SIMDs and each product is a
+// chain of loads and MFMAs.  Whole solves: N = 128, nc = 2: 26.8 -> 25.0 ms,
+// N = 256: 19.0 -> 17.7; what is left there is two launches a stage and the
+// stage vectors' way through few CUs.
+constexpr int kMaxWide = 16;
 template <int NP>
-__global__ __launch_bounds__(256 * kGHalves) void rk_dense_herm_stage_tiled_kernel(EpiArgs P,
+__global__ __launch_bounds__(64 * kMaxWide) void rk_dense_herm_wide_kernel(EpiArgs P, DenseOp D,
+                                                                           int ns) {
+    __shared__ float2 part[kMaxWide][256];
+    __shared__ double smem[kMaxWide];
+    int bi, bj;
+    upper_tile(blockIdx.x, bi, bj);
+    const int i0 = 16 * bi, j0 = 16 * bj;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int g = w / ns, ng = nw / ns;
+    int k0, k1;
+    k_range(D.N, ns, w % ns, k0, k1);
+    const int nb = (k1 - k0) / 32, total = (2 + D.nc - g + ng - 1) / ng * nb;
+    auto load = [&](int s, float2 (&a)[8], float2 (&b)[8]) {
+        const float2 *A, *B;
+        gt_operands(D, g + ng * (s / nb), A, B);
+        step_load(A, B, D.N, i0, j0, lane, k0 + 32 * (s % nb), a, b);
+    };
+    // the first operands are requested with the control block, before it is
+    // known that this stage runs
+    float2 a0[8], b0[8];
+    load(0, a0, b0);
+    RKCtl *ctl = P.ctl;
+    if (ctl->phase != P.run_phase) return;
+    const StageVecs v = stage_vecs(P, ctl);
+    const int nitems = bi == bj ? 256 : 512;
+    const bool own = (int)threadIdx.x < nitems;
+    const HermItem it = herm_item<16>(D.N, i0, j0, threadIdx.x & 511);
+    double2 o, er;
+    if (own) epi_pre(P, v, it.idx, o, er);
+    v4f re = {0.f, 0.f, 0.f, 0.f}, im = {0.f, 0.f, 0.f, 0.f};
+    v4f re2 = {0.f, 0.f, 0.f, 0.f}, im2 = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < total; ++s) {
+        float2 an[8], bn[8];
+        load(min(s + 1, total - 1), an, bn);
+        step_mma<NP>(a0, b0, re, im, re2, im2);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            a0[u] = an[u];
+            b0[u] = bn[u];
+        }
+    }
+    re += re2;
+    im += im2;
+    herm_partial_store(part, w, lane, re, im);
+    __syncthreads();
+    double sum = 0.0;
+    if (own) {
+        const float2 t = herm_partial_sum(part, nw, it.src);
+        sum = epi_post(P, ctl, v, it.idx, herm_value(t, it), o, er);
+    }
+    if (P.epi == EPI_FINAL) {
+        sum = block_sum(sum, smem);
+        if (threadIdx.x == 0) P.partials[blockIdx.x] = sum;
+    }
+}
+
+// Tile sums that workgroups on any XCD hand on: stored and loaded past the L2.
+__device__ __forceinline__ void part_store(float2 *p, float2 v) {
+    __hip_atomic_store((unsigned long long *)p, __builtin_bit_cast(unsigned long long, v),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 part_load(const float2 *p) {
+    return __builtin_bit_cast(float2,
+                              __hip_atomic_load((const unsigned long long *)p, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT));
+}
+
+// The same on the upper 32 x 32 workgroup tiles of the LDS-staged path
+// (N >= kTiledN): 2 E^2 items over 512 threads.  gridDim.y workgroups share a
+// tile: each takes some of its products and stores its sum, and the one that
+// arrives last adds the sums in their order and does the epilogue.  One
+// workgroup a tile left 120 of 256 CUs idle at N = 512 (136 tiles): 78 us a
+// stage, 39 with five (nc = 3); a whole solve 31.7 -> 25.4 ms, at N = 384
+// 18.0 -> 14.2.  Two workgroups a CU need at most 128 registers (FP32).
+template <int NP>
+__global__ __launch_bounds__(256 * kGHalves, NP == 0 ? 4 : 2) void rk_dense_herm_stage_tiled_kernel(EpiArgs P,
                                                                                   DenseOp D) {
     constexpr int IPT = 2 * kGT * kGT / (256 * kGHalves);
     __shared__ GemmShared G;
     __shared__ double smem[256 * kGHalves / QA_WAVE];
+    __shared__ int last;
     RKCtl *ctl = P.ctl;
     if (ctl->phase != P.run_phase) return;
     const StageVecs v = stage_vecs(P, ctl);
@@ -1095,9 +1191,11 @@ __global__ __launch_bounds__(256 * kGHalves) void rk_dense_herm_stage_tiled_kern
     upper_tile(blockIdx.x, bi, bj);
     const int i0 = kGT * bi, j0 = kGT * bj;
     const int nitems = bi == bj ? kGT * kGT : 2 * kGT * kGT;
+    const int np = 2 + D.nc, ng = gridDim.y, g = blockIdx.y;
+    const int p0 = g * np / ng, p1 = (g + 1) * np / ng;
     v4f re = {0.f, 0.f, 0.f, 0.f}, im = {0.f, 0.f, 0.f, 0.f};
-    gt_run<float2, NP>(D, G, 2 + D.nc, nullptr, (const float2 *)nullptr, i0, j0, re, im);
-    // the tile is complete in half 0; it goes through LDS to the items
+    gt_run<float2, NP>(D, G, p0, p1 - p0, nullptr, (const float2 *)nullptr, i0, j0, re, im);
+    // the sum is complete in half 0; it goes through LDS to the items
     __syncthreads();
     float2 *tile = (float2 *)&G.L[0];
     const int h = threadIdx.x >> 8, lane = threadIdx.x & 63, w = (threadIdx.x & 255) >> 6;
@@ -1108,6 +1206,32 @@ __global__ __launch_bounds__(256 * kGHalves) void rk_dense_herm_stage_tiled_kern
                 make_float2(re[q], im[q]);
     }
     __syncthreads();
+    if (ng > 1) {
+        const size_t stride = (size_t)gridDim.x * kGT * kGT;
+        float2 *part = D.part + (size_t)blockIdx.x * kGT * kGT;
+        for (int e = threadIdx.x; e < kGT * kGT; e += blockDim.x)
+            part_store(part + g * stride + e, tile[e]);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // stored before the arrival counts
+        __syncthreads();
+        if (threadIdx.x == 0)
+            last = __hip_atomic_fetch_add(D.arrived + blockIdx.x, 1u, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(ng - 1);
+        __syncthreads();
+        if (!last) return;
+        if (threadIdx.x == 0)
+            __hip_atomic_store(D.arrived + blockIdx.x, 0u, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+        for (int e = threadIdx.x; e < kGT * kGT; e += blockDim.x) {
+            float2 t = part_load(part + e);
+            for (int u = 1; u < ng; ++u) {
+                const float2 x = part_load(part + u * stride + e);
+                t.x += x.x;
+                t.y += x.y;
+            }
+            tile[e] = t;
+        }
+        __syncthreads();
+    }
     // the epilogue's loads follow the products here: issued before them,
     // four items' K terms would not fit the registers beside the LDS pipeline
     double sum = 0.0;
@@ -1762,6 +1886,15 @@ int launch_sparse_stage(qa_rk_solver *S, int i) {
         }                                                                                \
     } while (0)
 
+// Groups of waves that share the np products of an upper 16 x 16 tile (ns
+// waves a group), or 0 for one group: where every tile has a CU of its own.
+// At least eight waves, one for each item of the epilogue.
+int herm_wide_groups(int tiles, int ns, int np) {
+    if (tiles > 256) return 0;
+    const int ng = std::min(kMaxWide / ns, np);
+    return ng > 1 && ns * ng >= 8 ? ng : 0;
+}
+
 // Hermitian stage inputs: the T layer (which also writes Xf), then the
 // upper-tile stage kernel.
 int launch_dense_herm_stage(qa_rk_solver *S, const EpiArgs &P) {
@@ -1771,7 +1904,7 @@ int launch_dense_herm_stage(qa_rk_solver *S, const EpiArgs &P) {
         QA_DENSE_LAUNCH(S->dop.prec, rk_dense_t_tiled_kernel, dim3(nt, nt, nz),
                         dim3(256 * kGHalves), S->stream, P, S->dop);
         QA_CHECK_LAUNCH();
-        QA_DENSE_LAUNCH(S->dop.prec, rk_dense_herm_stage_tiled_kernel, dim3(nt * (nt + 1) / 2),
+        QA_DENSE_LAUNCH(S->dop.prec, rk_dense_herm_stage_tiled_kernel, dim3(nt * (nt + 1) / 2, S->dop.hgroups),
                         dim3(256 * kGHalves), S->stream, P, S->dop);
         QA_CHECK_LAUNCH();
         return QA_OK;
@@ -1782,6 +1915,12 @@ int launch_dense_herm_stage(qa_rk_solver *S, const EpiArgs &P) {
                        S->dop);
     QA_CHECK_LAUNCH();
     const dim3 grid(nt * (nt + 1) / 2), block(64 * ns);
+    if (const int ng = herm_wide_groups(nt * (nt + 1) / 2, ns, 2 + S->dop.nc)) {
+        QA_DENSE_LAUNCH(S->dop.prec, rk_dense_herm_wide_kernel, grid, dim3(64 * ns * ng), S->stream,
+                        P, S->dop, ns);
+        QA_CHECK_LAUNCH();
+        return QA_OK;
+    }
     switch (ns) {
         case 8: hipLaunchKernelGGL(rk_dense_herm_stage_kernel<1>, grid, block, 0, S->stream, P, S->dop); break;
         case 4: hipLaunchKernelGGL(rk_dense_herm_stage_kernel<2>, grid, block, 0, S->stream, P, S->dop); break;
@@ -2419,9 +2558,17 @@ int qa_rk_create_dense(qa_rk_solver **out, int N, int nc, const double *H_nh, co
                 Cs[k * NN + (size_t)j * N + i] = make_float2((float)src[0], (float)src[1]);
                 Cds[k * NN + (size_t)i * N + j] = make_float2((float)src[0], (float)-src[1]);
             }
+    // the partial tiles and the arrival counts follow the matrices
+    const size_t ntile = (size_t)(N / kGT) * (N / kGT + 1) / 2;
+    S->dop.hgroups = N % kTiledStep == 0 ? herm_groups(N, nc) : 1;
+    const size_t npart = S->dop.hgroups > 1 ? S->dop.hgroups * ntile * kGT * kGT : 0;
+    const size_t nmat = (3 + 3 * (size_t)nc) * NN;
     hipError_t he = hipStreamCreateWithFlags(&S->stream, hipStreamNonBlocking);
     if (he == hipSuccess)
-        he = hipMalloc(&S->dense_block, sizeof(float2) * ((3 + 3 * (size_t)nc) * NN + 1));
+        he = hipMalloc(&S->dense_block,
+                       sizeof(float2) * (nmat + npart) + sizeof(unsigned) * (ntile + 1));
+    if (he == hipSuccess)
+        he = hipMemset((float2 *)S->dense_block + nmat + npart, 0, sizeof(unsigned) * (ntile + 1));
     if (he == hipSuccess)
         he = hipMemcpy(S->dense_block, h.data(), sizeof(float2) * h.size(), hipMemcpyHostToDevice);
     if (he != hipSuccess) {
@@ -2447,8 +2594,10 @@ int qa_rk_create_dense(qa_rk_solver **out, int N, int nc, const double *H_nh, co
     S->dop.Cd = d + (2 + (size_t)nc) * NN;
     S->dop.T = d + (2 + 2 * (size_t)nc) * NN;
     S->dop.Xf = d + (2 + 3 * (size_t)nc) * NN;
+    S->dop.part = d + nmat;
+    S->dop.arrived = (unsigned *)(d + nmat + npart);
     S->dop.hsplit = N % 32 == 0 ? herm_split(N) : 1;
-    S->dop.tiled = (N >= kTiledN && N % kGK == 0 && N % kGT == 0) ? 1 : 0;
+    S->dop.tiled = (N >= kTiledN && N % kTiledStep == 0) ? 1 : 0;
     // S->nparts stays (N / 16)^2, the most any tile shape needs (the shape
     // can be changed later, qa_rk_set_dense_shape)
     rc = rk_finish_create(S, order, rk_step, rk_extra, dorder, a, b, c, e, bi, rtol, atol, nsteps,
@@ -2630,8 +2779,8 @@ int qa_rk_set_dense_shape(qa_rk_solver *S, int tiled, int nsplit, int hsplit) {
     const bool pow2 = [](int v) { return v == 1 || v == 2 || v == 4 || v == 8; }(nsplit) &&
                       [](int v) { return v == 1 || v == 2 || v == 4 || v == 8; }(hsplit);
     QA_REQUIRE(pow2, "qa_rk_set_dense_shape: nsplit and hsplit must be 1, 2, 4 or 8");
-    QA_REQUIRE(tiled == 0 || (tiled == 1 && N % kGK == 0 && N % kGT == 0),
-               "qa_rk_set_dense_shape: tiled needs N %% %d == 0", kGK);
+    QA_REQUIRE(tiled == 0 || (tiled == 1 && N % kTiledStep == 0),
+               "qa_rk_set_dense_shape: tiled needs N %% %d == 0", kTiledStep);
     const int kstep = S->dop.prec >= 1 ? 32 : 16;
     QA_REQUIRE(N % (nsplit * kstep) == 0,
                "qa_rk_set_dense_shape: N must be a multiple of %d x nsplit", kstep);
