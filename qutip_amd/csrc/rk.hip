@@ -585,19 +585,23 @@ __global__ __launch_bounds__(64 * kMaxSplit) void rk_dense_stage_kernel(EpiArgs 
 
 // ---- large N: 32 x 32 workgroup tiles through LDS ------------------------
 // Half a workgroup (4 waves) owns a 32 x 32 output tile (each wave one
-// 16 x 16 MFMA tile).  K goes in chunks of 32: the 256 threads load the A
-// chunk (32 rows x 32 k, one 256-byte column piece per k) and the B chunk
-// (32 k x 32 columns, one 256-byte piece per column) into LDS, the next
+// 16 x 16 MFMA tile).  K goes in chunks of 32 or 64: the 256 threads load the
+// A chunk (32 rows x GK k, one 256-byte column piece per k) and the B chunk
+// (GK k x 32 columns, one piece per column) into LDS, the next
 // chunk's loads are issued before the current chunk's MFMAs (one chunk of
 // register prefetch, double-buffered LDS), and every A and B element loaded
 // serves two waves.  All products of a workgroup run through one flattened
-// chunk loop, so one memory latency is exposed per stage.  Chunks of 64 took
+// chunk loop, so one memory latency is exposed per stage.  Chunks of 64 take
 // 137 KB of LDS, one workgroup a CU, whose waves all wait at once; with 32
-// two fit (69 KB): C_c X for N = 512, nc = 3 went from 51 to 29 us.  Used for
+// two fit (69 KB): C_c X in FP32 for N = 512, nc = 3 went from 51 to 29 us.
+// The bf16 splits need more registers than two workgroups a CU leave, and
+// keep 64 (with 32 they were 3 to 5 % slower).  Used for
 // N >= kTiledN, where the one-tile-per-workgroup kernels above re-read every
 // operand row and column 32 times from L2.
 constexpr int kGT = 32;      // output tile edge per workgroup
-constexpr int kGK = 32;      // K chunk
+// K chunk of the FP32 (NP 0) and bf16 kernels
+template <int NP>
+constexpr int kGK = NP == 0 ? 32 : 64;
 constexpr int kGP = 2;       // LDS row padding (float2) against bank conflicts
 constexpr int kTiledN = 384;
 constexpr int kTiledStep = 64;  // the tiled path takes multiples of this
@@ -610,43 +614,47 @@ __host__ inline int herm_groups(int N, int nc) {
     return std::min(2 + nc, (1024 + tiles - 1) / tiles);
 }
 
+template <int NP>
 struct GemmTile {
-    float2 a[2][kGK][kGT + kGP];  // a[buf][k][i]
-    float2 b[2][kGT][kGK + kGP];  // b[buf][j][k]
+    float2 a[2][kGK<NP>][kGT + kGP];  // a[buf][k][i]
+    float2 b[2][kGT][kGK<NP> + kGP];  // b[buf][j][k]
 };
 
-constexpr int kGQ = kGT * kGK / 256;  // chunk elements per thread, per operand
+template <int NP>
+constexpr int kGQ = kGT * kGK<NP> / 256;  // chunk elements per thread, per operand
 
-template <typename TA, typename TB>
+template <int NP, typename TA, typename TB>
 __device__ __forceinline__ void gt_fetch(const TA *__restrict__ A, const TB *__restrict__ B,
                                          int N, int i0, int j0, int k0, int tid,
-                                         float2 (&ra)[kGQ], float2 (&rb)[kGQ]) {
+                                         float2 (&ra)[kGQ<NP>], float2 (&rb)[kGQ<NP>]) {
 #pragma unroll
-    for (int q = 0; q < kGQ; ++q) {
+    for (int q = 0; q < kGQ<NP>; ++q) {
         const int e = tid + 256 * q;
         ra[q] = tof(A[(size_t)(k0 + e / kGT) * N + i0 + e % kGT]);
-        rb[q] = tof(B[(size_t)(j0 + e / kGK) * N + k0 + e % kGK]);
+        rb[q] = tof(B[(size_t)(j0 + e / kGK<NP>) * N + k0 + e % kGK<NP>]);
     }
 }
 
-__device__ __forceinline__ void gt_store(GemmTile &L, int buf, int tid, const float2 (&ra)[kGQ],
-                                         const float2 (&rb)[kGQ]) {
+template <int NP>
+__device__ __forceinline__ void gt_store(GemmTile<NP> &L, int buf, int tid,
+                                         const float2 (&ra)[kGQ<NP>],
+                                         const float2 (&rb)[kGQ<NP>]) {
 #pragma unroll
-    for (int q = 0; q < kGQ; ++q) {
+    for (int q = 0; q < kGQ<NP>; ++q) {
         const int e = tid + 256 * q;
         L.a[buf][e / kGT][e % kGT] = ra[q];
-        L.b[buf][e / kGK][e % kGK] = rb[q];
+        L.b[buf][e / kGK<NP>][e % kGK<NP>] = rb[q];
     }
 }
 
 // The wave's 16 x 16 tile += A_chunk B_chunk from LDS buffer `buf`, with
 // the inputs split into NP bf16 pieces (32-wide K steps).
 template <int NP>
-__device__ __forceinline__ void gt_mma_bf16(const GemmTile &L, int buf, int wi, int wj, int lane,
+__device__ __forceinline__ void gt_mma_bf16(const GemmTile<NP> &L, int buf, int wi, int wj, int lane,
                                             v4f &re, v4f &im, v4f &re2, v4f &im2) {
     const int r = lane & 15, kq = lane >> 4;
 #pragma unroll
-    for (int st = 0; st < kGK / 32; ++st) {
+    for (int st = 0; st < kGK<NP> / 32; ++st) {
         v8bf ar[NP], ai[NP], nai[NP], br[NP], bi[NP];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
@@ -668,7 +676,7 @@ __device__ __forceinline__ void gt_mma_bf16(const GemmTile &L, int buf, int wi, 
 // The wave's 16 x 16 tile += A_chunk B_chunk from LDS buffer `buf`; NP = 0:
 // FP32 MFMA, 2 / 3: the bf16 x3 / x6 splits.
 template <int NP>
-__device__ __forceinline__ void gt_mma(const GemmTile &L, int buf, int wi, int wj, int lane,
+__device__ __forceinline__ void gt_mma(const GemmTile<NP> &L, int buf, int wi, int wj, int lane,
                                        v4f &re, v4f &im) {
     const int r = lane & 15, kq = lane >> 4;
     v4f re2 = {0.f, 0.f, 0.f, 0.f}, im2 = {0.f, 0.f, 0.f, 0.f};
@@ -676,7 +684,7 @@ __device__ __forceinline__ void gt_mma(const GemmTile &L, int buf, int wi, int w
         gt_mma_bf16<NP>(L, buf, wi, wj, lane, re, im, re2, im2);
     } else {
 #pragma unroll
-        for (int st = 0; st < kGK / 4; ++st) {
+        for (int st = 0; st < kGK<NP> / 4; ++st) {
             const float2 a = L.a[buf][4 * st + kq][16 * wi + r];
             const float2 b = L.b[buf][16 * wj + r][4 * st + kq];
             re = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, re, 0, 0, 0);
@@ -714,23 +722,24 @@ __device__ __forceinline__ void gt_operands(const DenseOp &D, int p, const float
 constexpr int kGHalves = 2;
 
 
+template <int NP>
 struct GemmShared {
-    GemmTile L[kGHalves];
+    GemmTile<NP> L[kGHalves];
 };
 
 // The products p0 .. p0 + np - 1 of a stage, or A0 B0 (the T kernel's C_c X).
 template <typename TB, int NP>
-__device__ __forceinline__ void gt_run(const DenseOp &D, GemmShared &G, int p0, int np,
+__device__ __forceinline__ void gt_run(const DenseOp &D, GemmShared<NP> &G, int p0, int np,
                                        const float2 *A0, const TB *B0, int i0, int j0,
                                        v4f &re, v4f &im) {
     const int h = threadIdx.x >> 8, tid = threadIdx.x & 255;
     const int lane = threadIdx.x & 63, w = tid >> 6, wi = w & 1, wj = w >> 1;
-    const int nch = D.N / kGK, total = np * nch;
+    const int nch = D.N / kGK<NP>, total = np * nch;
     const int trips = (total + kGHalves - 1) / kGHalves;
-    GemmTile &L = G.L[h];
+    GemmTile<NP> &L = G.L[h];
     auto operands = [&](int idx, const float2 *&A, const TB *&B, int &k0) {
         const int p = p0 + idx / nch;
-        k0 = (idx % nch) * kGK;
+        k0 = (idx % nch) * kGK<NP>;
         if (A0) {
             A = A0;
             B = B0;
@@ -740,21 +749,21 @@ __device__ __forceinline__ void gt_run(const DenseOp &D, GemmShared &G, int p0, 
             B = (const TB *)Bf;
         }
     };
-    float2 ra[kGQ], rb[kGQ];
+    float2 ra[kGQ<NP>], rb[kGQ<NP>];
     const float2 *A;
     const TB *B;
     int k0;
     operands(min(h, total - 1), A, B, k0);
-    gt_fetch(A, B, D.N, i0, j0, k0, tid, ra, rb);
-    gt_store(L, 0, tid, ra, rb);
+    gt_fetch<NP>(A, B, D.N, i0, j0, k0, tid, ra, rb);
+    gt_store<NP>(L, 0, tid, ra, rb);
     __syncthreads();
     for (int it = 0; it < trips; ++it) {
         const int cur = kGHalves * it + h;
         const int nx = min(cur + kGHalves, total - 1);
         operands(nx, A, B, k0);
-        gt_fetch(A, B, D.N, i0, j0, k0, tid, ra, rb);
+        gt_fetch<NP>(A, B, D.N, i0, j0, k0, tid, ra, rb);
         if (cur < total) gt_mma<NP>(L, it & 1, wi, wj, lane, re, im);
-        gt_store(L, (it + 1) & 1, tid, ra, rb);
+        gt_store<NP>(L, (it + 1) & 1, tid, ra, rb);
         __syncthreads();
     }
     // half 1 hands its partial tile to half 0 through its own LDS tile
@@ -780,7 +789,7 @@ __device__ __forceinline__ void gt_run(const DenseOp &D, GemmShared &G, int p0, 
 // blockIdx.z == 0 workgroups also write Xf = complex64(X) for their tile.
 template <int NP>
 __device__ __forceinline__ void dense_t_tiled(const DenseOp &D, const double2 *X) {
-    __shared__ GemmShared G;
+    __shared__ GemmShared<NP> G;
     const int i0 = blockIdx.x * kGT, j0 = blockIdx.y * kGT, c = blockIdx.z;
     const size_t NN = (size_t)D.N * D.N;
     if (c == 0) {
@@ -802,7 +811,7 @@ __device__ __forceinline__ void dense_t_tiled(const DenseOp &D, const double2 *X
 
 // k tile = Hm Xf + Xf Hp + sum_c T_c Cd_c; complete in half 0.
 template <int NP>
-__device__ __forceinline__ void dense_k_tiled(const DenseOp &D, GemmShared &G, v4f &re,
+__device__ __forceinline__ void dense_k_tiled(const DenseOp &D, GemmShared<NP> &G, v4f &re,
                                               v4f &im) {
     gt_run<float2, NP>(D, G, 0, 2 + D.nc, nullptr, (const float2 *)nullptr, blockIdx.x * kGT,
                    blockIdx.y * kGT, re, im);
@@ -818,7 +827,7 @@ __global__ __launch_bounds__(256 * kGHalves) void rk_dense_t_tiled_kernel(EpiArg
 template <int NP>
 __global__ __launch_bounds__(256 * kGHalves) void rk_dense_stage_tiled_kernel(EpiArgs P,
                                                                              DenseOp D) {
-    __shared__ GemmShared G;
+    __shared__ GemmShared<NP> G;
     __shared__ double smem[256 * kGHalves / QA_WAVE];
     RKCtl *ctl = P.ctl;
     if (ctl->phase != P.run_phase) return;
@@ -1181,7 +1190,7 @@ template <int NP>
 __global__ __launch_bounds__(256 * kGHalves, NP == 0 ? 4 : 2) void rk_dense_herm_stage_tiled_kernel(EpiArgs P,
                                                                                   DenseOp D) {
     constexpr int IPT = 2 * kGT * kGT / (256 * kGHalves);
-    __shared__ GemmShared G;
+    __shared__ GemmShared<NP> G;
     __shared__ double smem[256 * kGHalves / QA_WAVE];
     __shared__ int last;
     RKCtl *ctl = P.ctl;
@@ -1260,7 +1269,7 @@ __global__ __launch_bounds__(256 * kGHalves) void dense_t_tiled_kernel(DenseOp D
 template <int NP>
 __global__ __launch_bounds__(256 * kGHalves) void dense_rhs_tiled_kernel(DenseOp D,
                                                                         double2 *out) {
-    __shared__ GemmShared G;
+    __shared__ GemmShared<NP> G;
     v4f re = {0.f, 0.f, 0.f, 0.f}, im = {0.f, 0.f, 0.f, 0.f};
     dense_k_tiled<NP>(D, G, re, im);
     if ((threadIdx.x >> 8) != 0) return;
