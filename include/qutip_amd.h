@@ -418,7 +418,9 @@ int qa_mc_run(int d, int ntraj, int ntimes, const double *times_dev, const void 
  * `width` (even, at most 16) off-diagonal entries a row as 16-bit codes,
  * entry u of row r at code[u d + r]: the column in the low cbits bits, an
  * index into `table` above them.  table[0] is 0; shorter rows are filled
- * with their own row and index 0.  ntab <= min(256, 2^(16 - cbits)).  imag != 0:
+ * with their own row and index 0.  complex64: the entries in the order of
+ * their columns, and one more row of codes, code[width d + r]: the number of
+ * entries of row r before its diagonal.  ntab <= min(256, 2^(16 - cbits)).  imag != 0:
  * every off-diagonal value is purely imaginary and `table` holds the ntab
  * imaginary parts (real numbers), else ntab complex ones.  Values are
  * complex64 / float when the run's fp32 is set.  The kernels that read it

@@ -37,8 +37,8 @@
 // with 16 waves a CU the instructions and the LDS bytes of the gathers.
 // Measured against the ELL form with two rows a thread and a run-time
 // tableau, Ising chains with vern7, kernel time: L = 10, 2048 trajectories:
-// complex128 140 -> 53 ms, complex64 104 -> 52; L = 8, 500 of them: 4.2 ->
-// 1.9 ms and 3.8 -> 1.9; L = 8, 8192: 62 -> 16 ms; whole solve of a 400-row
+// complex128 140 -> 51 ms, complex64 104 -> 69; L = 8, 500 of them: 4.2 ->
+// 1.9 ms and 3.8 -> 2.4; L = 8, 8192: 62 -> 15 ms and 41 -> 21; whole solve of a 400-row
 // Liouvillian: 5.5 -> 2.9 ms.  What gave it, for L = 10: no ELL in the
 // stages, one row a thread and stages in registers (the spills gone from the
 // stage loop) 140 -> 104, compile-time stage loops with step and dense output
@@ -247,7 +247,8 @@ struct Ctx {
     const int *hcol;    // this system's H_eff ELL
     const void *hval;
     unsigned pk[FM == OP_ELL ? 1 : kMcPack / 2];  // this thread's codes, two a word
-    C2<R> dg;                                     // and diagonal entries
+    C2<R> dg;                                     // and diagonal entry
+    int dpos;  // complex64: the slot before which the diagonal is added
     int n_step, n_extra, is_fsal, is_adaptive, is_interp;  // of the tableau, uniform
     const __attribute__((address_space(4))) McTableau *tab;
     // Packed operators come with a tableau of vern7's shape (packed_args), so
@@ -367,7 +368,7 @@ __device__ __forceinline__ void ell_chunk(Ctx<R, NT, FM> &c, int u0, C2<R> &acc)
 // M packed entries u0 .. u0 + M - 1 of this thread's rows: the gathers and
 // the values (LDS, no other memory) together, then the multiply-adds.
 template <int M, int U0, typename R, int NT, int FM>
-__device__ __forceinline__ void packed_chunk(Ctx<R, NT, FM> &c, C2<R> &acc) {
+__device__ __forceinline__ void packed_chunk(Ctx<R, NT, FM> &c, const C2<R> &x, C2<R> &acc) {
     const unsigned cm = (1u << c.A.pk_cbits) - 1u;
     C2<R> xv[M], vv[M];
 #pragma unroll
@@ -381,6 +382,7 @@ __device__ __forceinline__ void packed_chunk(Ctx<R, NT, FM> &c, C2<R> &acc) {
     }
 #pragma unroll
     for (int w = 0; w < M; ++w) {
+        if (sizeof(R) == 4 && c.dpos == U0 + w) cfmaR<R>(acc, c.dg, x);
         if constexpr (FM == OP_PACKED_IM) {
             acc.x = fma(-vv[w].y, xv[w].y, acc.x);
             acc.y = fma(vv[w].y, xv[w].x, acc.y);
@@ -391,24 +393,24 @@ __device__ __forceinline__ void packed_chunk(Ctx<R, NT, FM> &c, C2<R> &acc) {
 }
 
 template <int K, int U0, typename R, int NT, int FM>
-__device__ __forceinline__ void packed_from(Ctx<R, NT, FM> &c, C2<R> &acc) {
+__device__ __forceinline__ void packed_from(Ctx<R, NT, FM> &c, const C2<R> &x, C2<R> &acc) {
     if constexpr (U0 < kMcPack) {
         const int left = c.A.pk_width - U0;  // uniform, even
         if constexpr (K >= 8 && U0 + 8 <= kMcPack) {
             if (left >= 8) {
-                packed_chunk<8, U0>(c, acc);
-                packed_from<K, U0 + 8>(c, acc);
+                packed_chunk<8, U0>(c, x, acc);
+                packed_from<K, U0 + 8>(c, x, acc);
                 return;
             }
         }
         if constexpr (U0 + 4 <= kMcPack) {
             if (left >= 4) {
-                packed_chunk<4, U0>(c, acc);
-                packed_from<4, U0 + 4>(c, acc);
+                packed_chunk<4, U0>(c, x, acc);
+                packed_from<4, U0 + 4>(c, x, acc);
                 return;
             }
         }
-        if (left == 2) packed_chunk<2, U0>(c, acc);
+        if (left == 2) packed_chunk<2, U0>(c, x, acc);
     }
 }
 
@@ -416,7 +418,10 @@ __device__ __forceinline__ void packed_from(Ctx<R, NT, FM> &c, C2<R> &acc) {
 // width is a multiple of 4 (the host pads it), so entries go in chunks of 8
 // (4 in 1024 threads with complex128 stages in registers, which leaves room
 // for those) and at most one chunk of 4; no load is predicated.
-// Packed: the diagonal, then the entries in eights or fours and a last two.
+// Packed: the entries in eights or fours and a last two, after the diagonal;
+// complex64 adds the diagonal in its column's place, as the ELL form does: in
+// another order the sums differ by 1e-7, and now and then a trajectory of
+// 500 takes another jump (it costs 1.94 -> 2.37 ms for 500 of L = 8).
 template <typename R, int NT, int FM>
 __device__ __forceinline__ C2<R> rhs(Ctx<R, NT, FM> &c, const C2<R> &x) {
     stage_in(c, x);
@@ -432,8 +437,9 @@ __device__ __forceinline__ C2<R> rhs(Ctx<R, NT, FM> &c, const C2<R> &x) {
         // registers for the whole kernel
 #pragma unroll
         for (int w = 0; w < kMcPack / 2; ++w) asm volatile("" : "+v"(c.pk[w]));
-        cfmaR<R>(acc, c.dg, x);
-        packed_from<K, 0>(c, acc);
+        if (sizeof(R) == 8) cfmaR<R>(acc, c.dg, x);
+        packed_from<K, 0>(c, x, acc);
+        if (sizeof(R) == 4 && c.dpos >= c.A.pk_width) cfmaR<R>(acc, c.dg, x);
     }
     if constexpr (FM == OP_ELL) {
         if (!c.act) acc = mk<R>(0, 0);  // padding rows stay zero
@@ -870,6 +876,7 @@ __device__ __forceinline__ void ctx_rows(Ctx<R, NT, FM> &c, const int *hcol, con
     c.rowc = c.act ? row : 0;
     if constexpr (FM != OP_ELL) {
         // padding rows: a zero diagonal and value 0 in every slot
+        c.dpos = sizeof(R) == 4 && c.act ? c.A.pk_code[(size_t)c.A.pk_width * c.A.d + c.rowc] : 0;
         c.dg = c.act ? ((const C2<R> *)c.A.pk_diag)[c.rowc] : mk<R>(0, 0);
 #pragma unroll
         for (int u = 0; u < kMcPack; ++u) {

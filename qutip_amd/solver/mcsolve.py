@@ -231,7 +231,9 @@ def _packed_host(A, d, fp32):
     [width, d], diagonal, table, column bits, imag), or None when a row has
     more than 16 off-diagonal entries or the values do not fit the codes.
     A row's entries are ordered by their distance from the diagonal, so the
-    lanes of a wave mostly read one value and shifted runs of the vector."""
+    lanes of a wave mostly read one value and shifted runs of the vector; in
+    complex64 by their columns, with the number of them before the diagonal
+    in one more row of codes, so that the sums round as the ELL form's do."""
     A = sp.csr_matrix(A, dtype=np.complex64 if fp32 else np.complex128)
     A = A.copy()
     A.sum_duplicates()
@@ -253,7 +255,8 @@ def _packed_host(A, d, fp32):
         inv = np.where(inv == zero, 0, np.where(inv == 0, zero, inv))
     if len(table) > min(PACK_VALUES, 1 << (16 - cbits)):
         return None
-    order = np.lexsort((cols - rows, np.abs(cols - rows), rows))
+    order = (np.lexsort((cols, rows)) if fp32
+             else np.lexsort((cols - rows, np.abs(cols - rows), rows)))
     rows, cols, idx = rows[order], cols[order], inv[1:].reshape(-1)[order]
     start = np.concatenate([[0], np.cumsum(counts)[:-1]])
     slot = np.arange(len(rows)) - start[rows]
@@ -261,7 +264,11 @@ def _packed_host(A, d, fp32):
     codes[slot, rows] = (cols | (idx << cbits)).astype(np.uint16)
     imag = bool((table.real == 0).all())
     table = np.ascontiguousarray(table.imag if imag else table)
-    return codes[:max(width, 1)], diag, table, width, cbits, imag
+    codes = codes[:max(width, 1)]
+    if fp32:
+        before = np.bincount(rows[cols < rows], minlength=d).astype(np.uint16)
+        codes = np.vstack([codes[:width], before[None, :]])
+    return codes, diag, table, width, cbits, imag
 
 
 class PackedOp:

@@ -9,8 +9,8 @@ sum to at most 4 in absolute value, that is below 10^4 eps an attempt, and
 the flow does not amplify it: tol = 10^4 eps attempts.  Sizes at the edges of
 waves and of the two kernel forms (at most 512 rows and at most 256 systems,
 or else), widths 0 to 16, imaginary and complex values.  In complex64 the
-error norms of the two differ by their rounding, so the steps do: each run
-then stays within its own local errors, atol sqrt(n) + rtol an attempt."""
+order is the same, so the bits are: there rounding alone could send a
+trajectory to another jump."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -68,6 +68,20 @@ def test_packed_host_refuses():
     assert M.packed_op(ok, 20, False, tab, False) is None
 
 
+def test_packed_host_complex64_keeps_the_order():
+    A = _op(300, 8, False)
+    codes, diag, table, w, cbits, im = M._packed_host(A, 300, True)
+    E = sp.csr_matrix(A, dtype=np.complex64)
+    E.sort_indices()
+    assert codes.shape == (w + 1, 300)
+    for r in range(300):
+        row = [(codes[u, r] & 511, table[codes[u, r] >> cbits]) for u in range(w)
+               if codes[u, r] >> cbits]
+        row.insert(int(codes[w, r]), (r, diag[r]))
+        assert [c for c, _ in row] == list(E.indices[E.indptr[r]:E.indptr[r + 1]])
+        assert [v for _, v in row] == list(E.data[E.indptr[r]:E.indptr[r + 1]])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,width,imag,nsys", [
     (1, 0, True, 1), (2, 1, False, 1), (63, 2, True, 3), (64, 3, False, 1), (65, 16, True, 300),
@@ -91,16 +105,16 @@ def test_small_packed_against_ell(n, width, imag, nsys, fp32):
     S._packed = None
     ref, yr, ir = S.run(0.0, y0, times)
     assert (ig[:, 0] == ir[:, 0]).all() and (ig[:, 0] >= 0).all()
-    if not fp32:
-        assert (ig[:, 3] == ir[:, 3]).all()  # attempts
+    assert (ig[:, 3] == ir[:, 3]).all()  # attempts
     eps = np.finfo(np.float32 if fp32 else np.float64).eps
-    step = 1e4 * eps + (2 * (rtol + np.sqrt(n) * atol) if fp32 else 0.0)
-    tol = step * max(ir[:, 3].max(), ig[:, 3].max())
+    tol = 0.0 if fp32 else 1e4 * eps * ir[:, 3].max()
     a, b = (np.empty((nsys, n), np.complex128) for _ in range(2))
     yg.download(a)
     yr.download(b)
     assert np.linalg.norm(a - b, axis=1).max() <= tol
     assert np.abs(got - ref).max() <= 2 * np.sqrt(n) * tol
+    if fp32:
+        assert np.array_equal(got, ref)
 
 
 @pytest.mark.gpu
