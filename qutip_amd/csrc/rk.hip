@@ -2770,6 +2770,16 @@ int qa_functionals_check(int n, int nfun, const int *kinds, const int *fptr, con
     return QA_OK;
 }
 
+int qa_rk_set_resident(qa_rk_solver *S, int on) {
+    QA_REQUIRE(S != nullptr, "qa_rk_set_resident: null solver");
+    QA_REQUIRE(S->res_dev < 0, "qa_rk_set_resident: a run is in progress");
+    if (!on)
+        S->res = 0;
+    else if (S->res == 0 && S->use_graph)
+        S->res = -1;
+    return QA_OK;
+}
+
 int qa_rk_set_hermitian(qa_rk_solver *S, int on) {
     QA_REQUIRE(S != nullptr, "qa_rk_set_hermitian: null solver");
     // the upper-tile kernels split K in 32-wide steps

@@ -246,6 +246,10 @@ class RKEngine:
                   _ip(rows), _ip(cols), _dp(w))
         self.nfun = len(kinds)
 
+    def set_resident(self, on):
+        """Whether runs may take the resident step loop (same bits)."""
+        _lib.call("qa_rk_set_resident", self.handle, int(bool(on)))
+
     def set_hermitian(self, on, tune=True):
         """Hermitian states on the dense engine (assume_hermitian_state):
         the upper tiles and their mirror; no effect on the other engines.
