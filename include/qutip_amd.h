@@ -349,6 +349,10 @@ int qa_rk_get_state(qa_rk_solver *s, double *t, void *y_out);
  * the two of the first-step estimate, graph launches, status, output index,
  * phase. */
 int qa_rk_stats(qa_rk_solver *s, int64_t *stats);
+/* stats[0..1] since the last qa_rk_set_state: launches of the resident step
+ * loop whose results stand, and launches that gave up (the launched loop then
+ * went on from the state before).  No reference counterpart. */
+int qa_rk_resident_stats(qa_rk_solver *s, int64_t *stats);
 
 /* Average duration (ms, HIP events on the engine stream, `reps` launches) of
  * each stage kernel into ms_per_stage[0 .. rk_extra-1] (rk_step entries when

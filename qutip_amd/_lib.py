@@ -92,6 +92,7 @@ SIGNATURES = {
     "qa_rk_finish": [vp, P_f64, P_i32, P_f64],
     "qa_rk_get_state": [vp, P_f64, vp],
     "qa_rk_stats": [vp, P_i64],
+    "qa_rk_resident_stats": [vp, P_i64],
     "qa_rk_iterate": [vp, i32],
     "qa_rk_profile_stages": [vp, i32, P_f64],
     "qa_rk_profile_sequence": [vp, i32, P_f64, P_f64],

@@ -1768,6 +1768,7 @@ struct qa_rk_solver {
     // res_dev: the device whose resident slot this engine holds while a
     // launch is in flight, or -1.
     int res = -1, res_form = 0, res_dev = -1;
+    long long res_done = 0, res_gave_up = 0;  // launches since the last set_state
     ResArgs rp = {};
     void *res_block = nullptr;
     // the rows the functionals read, and the entries by their slots
@@ -2914,6 +2915,7 @@ int qa_rk_set_state(qa_rk_solver *S, double t0, const void *y0_dev) {
     double dt = S->first_step;
     S->setup_rhs = 0;
     S->graph_launches = 0;
+    S->res_done = S->res_gave_up = 0;
     if (dt == 0.0 && S->adaptive) {
         double norm2 = 0.0, kn2 = 0.0;
         rc = qa_norm2_z(S->n, S->y1, &norm2, s);
@@ -3287,9 +3289,10 @@ int qa_rk_advance(qa_rk_solver *S, int *done) {
             // its workgroups did not all become resident: the state is as it
             // was, and the launched loop takes over for good
             S->res = 0;
+            ++S->res_gave_up;
         } else if (resident) {
             S->run_iters += h.n_attempts - std::max(S->last_attempts, 0LL);
-            S->graph_launches += h.n_attempts - std::max(S->last_attempts, 0LL);
+            ++S->res_done;
         }
         out_base = h.out_idx;
         if (h.phase == PH_DONE || h.phase == PH_IDLE) {
@@ -3432,6 +3435,13 @@ int qa_rk_stats(qa_rk_solver *S, int64_t *stats) {
     stats[5] = h.status;
     stats[6] = h.out_idx;
     stats[7] = h.phase;
+    return QA_OK;
+}
+
+int qa_rk_resident_stats(qa_rk_solver *S, int64_t *stats) {
+    QA_REQUIRE(S != nullptr && stats != nullptr, "qa_rk_resident_stats: null argument");
+    stats[0] = S->res_done;
+    stats[1] = S->res_gave_up;
     return QA_OK;
 }
 

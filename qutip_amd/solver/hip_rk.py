@@ -313,7 +313,10 @@ class RKEngine:
         _lib.call("qa_rk_stats", self.handle, s)
         keys = ["attempts", "accepted", "dense_preps", "rhs_evals", "graph_launches",
                 "status", "out_idx", "phase"]
-        return dict(zip(keys, [int(x) for x in s]))
+        out = dict(zip(keys, [int(x) for x in s]))
+        _lib.call("qa_rk_resident_stats", self.handle, s)
+        out["resident_launches"], out["resident_giveups"] = int(s[0]), int(s[1])
+        return out
 
     def iterate(self, count):
         self.t_set = None

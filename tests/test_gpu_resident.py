@@ -4,7 +4,8 @@ launched loop.
 Both take the same products, combines, sums and step control in the same
 order, so everything must be the same bits: functionals, stored states, the
 final state, the counts.  QUTIP_AMD_RESIDENT=0 (read when an engine is
-created) keeps the launched loop.  Sizes at the edges of the resident shapes:
+created) keeps the launched loop; the counts of committed resident launches
+say which of the two ran.  Sizes at the edges of the resident shapes:
 one workgroup, a part of one, a ring that wraps, one XCD full, one row more
 (every XCD), two rows of workgroups.  Bar: bit-identical."""
 import numpy as np
@@ -44,16 +45,22 @@ def _run(eng, y0, tl, fun, store):
     more, _, _ = eng.run([tl[-1] + 0.05])  # goes on from the state at hand
     stats = eng.stats()
     return (vals, t, y.to_array(), more, buf.to_array() if store else None,
-            {k: stats[k] for k in STATS})
+            {k: stats[k] for k in STATS}, _launches(stats))
+
+
+def _launches(stats):
+    return stats["resident_launches"], stats["resident_giveups"], stats["graph_launches"]
 
 
 def _compare(monkeypatch, make, y0, tl, fun, store=False):
     monkeypatch.setenv("QUTIP_AMD_RESIDENT", "0")
     a = _run(make(), y0, tl, fun, store)
     monkeypatch.delenv("QUTIP_AMD_RESIDENT")
+    assert a[6][:2] == (0, 0) and a[6][2] > 0
     eng = make()
     for rep in range(2):
         b = _run(eng, y0, tl, fun, store)
+        assert b[6][0] >= 2 and b[6][1:] == (0, 0)  # both runs, no launched iteration
         assert a[5] == b[5]
         assert a[1] == b[1]
         for x, y in ((a[0], b[0]), (a[2], b[2]), (a[3], b[3])):
@@ -129,6 +136,7 @@ def test_resident_tableaus(monkeypatch, tableau, interpolate):
                     got = eng.run(tl[1:])[0]
                 except qa.IntegratorException as e:
                     got = str(e)
+                assert _launches(eng.stats())[0] >= 1
         assert np.array_equal(ref, got)
         return
     _compare(monkeypatch, make, _state(n, rng), tl, _fun(n, rng), store=True)
@@ -152,6 +160,7 @@ def test_resident_rejections_and_limits(monkeypatch):
         with pytest.raises(qa.IntegratorException) as e:
             eng.run([50.0])
         seen.append((str(e.value), eng.stats()["attempts"]))
+        assert (_launches(eng.stats())[0] > 0) == (env == "1")
     assert seen[0] == seen[1]
 
 
@@ -178,6 +187,7 @@ def test_resident_banded_matrix_form(monkeypatch, N):
             "store_final_state": True, "nsteps": 100000})
         res = solver.run(s["psi0"], tl, e_ops=s["e_ops"])
         st = solver._integrator.stats()
+        assert (_launches(st)[0] > 0) == (env == "1")
         out.append((np.array(res.expect), res.final_state.full(), {k: st[k] for k in STATS}))
     assert out[0][2] == out[1][2]
     assert np.array_equal(out[0][0], out[1][0])
