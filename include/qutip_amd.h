@@ -246,9 +246,12 @@ int qa_rk_create_dense(qa_rk_solver **out, int N, int nc, const double *H_nh, co
  * reference's A + A^dag (:175-189) is; off (the default), the full RHS.
  * No effect on the other engines; get reports what the engine runs. */
 int qa_rk_set_hermitian(qa_rk_solver *s, int on);
-/* The resident step loop of an engine between runs: 0 keeps the launched
- * loop (same bits), for callers that run many engines at once: a resident
- * grid waits for free CUs and holds them.  No reference counterpart. */
+/* Whether the engine's next runs may take the resident step loop (the
+ * default): 0 keeps the launched loop (same bits), for callers that run many
+ * engines at once: a resident grid waits for free CUs and holds them.  Has no
+ * effect where the environment keeps the launched loop.  1 also lets an
+ * engine try again whose last resident launch gave up.  No reference
+ * counterpart. */
 int qa_rk_set_resident(qa_rk_solver *s, int on);
 int qa_rk_get_hermitian(qa_rk_solver *s, int *on);
 /* Tile shape of the dense engine's MFMA kernels (the autotuner measures

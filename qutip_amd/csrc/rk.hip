@@ -1764,10 +1764,13 @@ struct qa_rk_solver {
     std::vector<double> times_host;
     bool run_single = false;
     // the resident loop (rk_resident.hip): -1 not planned yet, 0 not for this
-    // engine (QUTIP_AMD_RESIDENT=0, or a shape it does not take), 1 planned.
-    // res_dev: the device whose resident slot this engine holds while a
-    // launch is in flight, or -1.
+    // engine (a shape it does not take, or a launch that gave up), 1 planned.
+    // Runs take it where the environment (QUTIP_AMD_RESIDENT, QUTIP_AMD_GRAPH
+    // when the engine is created) and the caller (qa_rk_set_resident) let
+    // them.  res_dev: the device whose resident slot this engine holds while
+    // a launch is in flight, or -1.
     int res = -1, res_form = 0, res_dev = -1;
+    bool res_env = true, res_on = true;
     long long res_done = 0, res_gave_up = 0;  // launches since the last set_state
     ResArgs rp = {};
     void *res_block = nullptr;
@@ -1784,6 +1787,7 @@ namespace {
 
 void res_give(qa_rk_solver *S);
 int res_prepare(qa_rk_solver *S);
+bool res_wanted(const qa_rk_solver *S) { return S->res_env && S->res_on; }
 
 void fill_epi(EpiArgs &P, qa_rk_solver *S, int i) {
     P.nrows = S->n;
@@ -2242,7 +2246,7 @@ int rk_finish_create(qa_rk_solver *S, int order, int rk_step, int rk_extra, int 
         const char *so = getenv("QUTIP_AMD_STEP_ONLY");
         S->step_only = !(so && so[0] == '0');
         const char *rs = getenv("QUTIP_AMD_RESIDENT");
-        if (!S->use_graph || (rs && rs[0] == '0')) S->res = 0;
+        S->res_env = S->use_graph && !(rs && rs[0] == '0');
     }
     if (bi) S->bi.assign(bi, bi + (size_t)rk_extra * dorder);
     S->rtol = rtol;
@@ -2711,11 +2715,9 @@ int qa_rk_set_coefficients(qa_rk_solver *S, int ncoef, const int *start, const i
     S->td = T;
     S->td_on = 1;
     S->graph_dirty = true;
-    if (S->res == 1) {  // planned for the generator before
-        S->retired.push_back(S->res_block);
-        S->res_block = nullptr;
-        S->res = -1;
-    }
+    if (S->res_block) S->retired.push_back(S->res_block);
+    S->res_block = nullptr;  // planned for the generator before
+    S->res = -1;
     return QA_OK;
 }
 
@@ -2774,10 +2776,8 @@ int qa_functionals_check(int n, int nfun, const int *kinds, const int *fptr, con
 int qa_rk_set_resident(qa_rk_solver *S, int on) {
     QA_REQUIRE(S != nullptr, "qa_rk_set_resident: null solver");
     QA_REQUIRE(S->res_dev < 0, "qa_rk_set_resident: a run is in progress");
-    if (!on)
-        S->res = 0;
-    else if (S->res == 0 && S->use_graph)
-        S->res = -1;
+    S->res_on = on != 0;
+    if (on && S->res == 0 && S->res_block) S->res = 1;  // after a launch that gave up
     return QA_OK;
 }
 
@@ -2873,8 +2873,8 @@ int qa_rk_set_functionals(qa_rk_solver *S, int nfun, const int *kinds, const int
         QA_HIP(hipMemcpy(S->fcol_dev, cols, sizeof(int) * nnz, hipMemcpyHostToDevice));
         QA_HIP(hipMemcpy(S->fw_dev, w, sizeof(double2) * nnz, hipMemcpyHostToDevice));
     }
-    if (nnz > 0 && S->res != 0 && S->kind != 1) {
-        // the slots of the rows the entries read, in row order
+    if (nnz > 0 && S->res_env && S->kind != 1) {
+        // whatever the plan is now (it can change before the next run): the slots of the rows the entries read, in row order
         std::vector<int> need((size_t)S->npad, -1), slot(2 * (size_t)nnz, 0);
         for (int f = 0; f < nfun; ++f)
             for (int p = fptr[f]; p < fptr[f + 1]; ++p) {
@@ -2974,7 +2974,7 @@ int qa_rk_begin(qa_rk_solver *S, int ntimes, const double *times, int single_ste
     // the previous run may still be draining its last chunk
     QA_HIP(hipStreamSynchronize(s));
     res_give(S);
-    if (S->res < 0) QA_CHECK(res_prepare(S));
+    if (res_wanted(S) && S->res < 0) QA_CHECK(res_prepare(S));
     if (ntimes > S->times_cap) {
         if (S->times_dev) S->retired.push_back(S->times_dev);
         QA_CHECK(release_retired(S));
@@ -3008,7 +3008,7 @@ int qa_rk_begin(qa_rk_solver *S, int ntimes, const double *times, int single_ste
     S->run_store = states_out != nullptr;
     // an engine with a resident loop captures its graphs when it first needs
     // them (qa_rk_advance)
-    if (S->use_graph && (S->res != 1 || single_step) &&
+    if (S->use_graph && (!res_wanted(S) || S->res != 1 || single_step) &&
         (S->graph_dirty || S->graph_store != S->run_store)) {
         int rc = rebuild_graph(S);
         if (rc) return rc;
@@ -3163,6 +3163,7 @@ int res_prepare(qa_rk_solver *S) {
 // outputs it reaches; false when it cannot run now.
 int res_chunk(qa_rk_solver *S, int out_base, bool *ran) {
     *ran = false;
+    if (S->fnnz > 0 && !S->fslot_dev) return QA_OK;  // no slots for the functionals' entries
     const int left = S->run_ntimes - out_base;
     int64_t cap = left;
     if (S->nneed > 0)
@@ -3328,7 +3329,7 @@ int qa_rk_advance(qa_rk_solver *S, int *done) {
         S->last_front = h.t_front;
         idle = true;
     }
-    if (S->res == 1 && !S->run_single) {
+    if (res_wanted(S) && S->res == 1 && !S->run_single) {
         bool ran = false;
         QA_CHECK(res_chunk(S, out_base, &ran));
         if (ran) {

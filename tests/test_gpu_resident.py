@@ -8,6 +8,8 @@ created) keeps the launched loop; the counts of committed resident launches
 say which of the two ran.  Sizes at the edges of the resident shapes:
 one workgroup, a part of one, a ring that wraps, one XCD full, one row more
 (every XCD), two rows of workgroups.  Bar: bit-identical."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -15,6 +17,7 @@ import scipy.sparse as sp
 pytestmark = pytest.mark.gpu
 
 import qutip_amd as qa  # noqa: E402
+from qutip_amd import _lib  # noqa: E402
 from qutip_amd.solver.hip_rk import RKEngine, time_dependent_operator  # noqa: E402
 from tests import systems  # noqa: E402
 
@@ -208,3 +211,47 @@ def test_resident_time_dependent(monkeypatch, L):
     for lanes in (1, 4):
         _compare(monkeypatch, lambda: RKEngine(None, "vern7", 1e-8, 1e-10, td=td, lanes=lanes),
                  _state(n, rng), np.linspace(0.0, 2.0, 9), _fun(n, rng))
+
+
+def test_resident_switched_off_and_on(monkeypatch):
+    """qa_rk_set_resident between runs, in every order with the functionals:
+    the loop that is asked for runs, with the same results; no memory is
+    taken by switching; the environment's choice stands."""
+    print("resident switched off and on", flush=True)
+    n = 40000  # a ring of 20 MB
+    rng = np.random.default_rng(11)
+    A = _banded(n)
+    y0, fun, other = _state(n, rng), _fun(n, rng), _fun(n, rng)
+    tl = np.array([0.0, 0.4, 0.6])
+
+    def run(eng, f):
+        eng.set_functionals(*f)
+        eng.set_state(0.0, y0)
+        vals = eng.run(tl[1:])[0]
+        return vals, eng.get_state()[1].to_array(), _launches(eng.stats())
+
+    monkeypatch.setenv("QUTIP_AMD_RESIDENT", "0")
+    eng = RKEngine(A, "vern7", 1e-8, 1e-10, lanes=1)
+    eng.set_resident(True)
+    ref = {0: run(eng, fun), 1: run(eng, other)}
+    assert ref[0][2][0] == ref[1][2][0] == 0
+    monkeypatch.delenv("QUTIP_AMD_RESIDENT")
+    eng = RKEngine(A, "vern7", 1e-8, 1e-10, lanes=1)
+    for on, which in ((False, 0), (True, 0), (True, 1), (False, 1), (False, 0), (True, 0),
+                      (True, 1), (False, 0), (True, 1)):
+        eng.set_resident(on)
+        vals, y, launches = run(eng, (fun, other)[which])
+        assert (launches[0] > 0) == on and launches[1] == 0
+        assert np.array_equal(vals, ref[which][0]) and np.array_equal(y, ref[which][1])
+
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        _lib.call("qa_mem_info", C.byref(free), C.byref(total))
+        return free.value
+
+    free = free_bytes()
+    for _ in range(10):  # a plan each would take 200 MB
+        eng.set_resident(False)
+        eng.set_resident(True)
+        assert run(eng, other)[2][0] > 0
+    assert free_bytes() > free - (50 << 20)
