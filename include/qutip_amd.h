@@ -253,6 +253,10 @@ int qa_rk_set_hermitian(qa_rk_solver *s, int on);
  * engine try again whose last resident launch gave up.  No reference
  * counterpart. */
 int qa_rk_set_resident(qa_rk_solver *s, int on);
+/* How long a resident launch waits for its grid: polls of 0.4 us or more, at
+ * most (and by default) 2^20; 0 makes every launch give up at once.  No
+ * reference counterpart. */
+int qa_rk_set_resident_polls(qa_rk_solver *s, int polls);
 int qa_rk_get_hermitian(qa_rk_solver *s, int *on);
 /* Tile shape of the dense engine's MFMA kernels (the autotuner measures
  * and picks it; no counterpart in the reference, whose zgemm picks its own

@@ -75,6 +75,7 @@ SIGNATURES = {
                            P_f64, P_f64, P_f64, P_f64, P_f64, f64, f64, i32, f64, f64, f64, i32],
     "qa_rk_set_hermitian": [vp, i32],
     "qa_rk_set_resident": [vp, i32],
+    "qa_rk_set_resident_polls": [vp, i32],
     "qa_rk_get_hermitian": [vp, P_i32],
     "qa_rk_set_dense_shape": [vp, i32, i32, i32],
     "qa_rk_get_dense_shape": [vp, P_i32, P_i32, P_i32],

@@ -1771,6 +1771,7 @@ struct qa_rk_solver {
     // a launch is in flight, or -1.
     int res = -1, res_form = 0, res_dev = -1;
     bool res_env = true, res_on = true;
+    int res_polls = kResPolls;
     long long res_done = 0, res_gave_up = 0;  // launches since the last set_state
     ResArgs rp = {};
     void *res_block = nullptr;
@@ -2781,6 +2782,14 @@ int qa_rk_set_resident(qa_rk_solver *S, int on) {
     return QA_OK;
 }
 
+int qa_rk_set_resident_polls(qa_rk_solver *S, int polls) {
+    QA_REQUIRE(S != nullptr, "qa_rk_set_resident_polls: null solver");
+    QA_REQUIRE(polls >= 0 && polls <= kResPolls,
+               "qa_rk_set_resident_polls: 0 <= polls <= %d", kResPolls);
+    S->res_polls = polls;
+    return QA_OK;
+}
+
 int qa_rk_set_hermitian(qa_rk_solver *S, int on) {
     QA_REQUIRE(S != nullptr, "qa_rk_set_hermitian: null solver");
     // the upper-tile kernels split K in 32-wide steps
@@ -3185,6 +3194,7 @@ int res_chunk(qa_rk_solver *S, int out_base, bool *ran) {
     P.need = S->nneed > 0 ? S->need_dev : nullptr;
     P.yout = S->yout_dev;
     P.nneed = S->nneed;
+    P.polls = S->res_polls;
     P.out_base = out_base;
     P.out_cap = (int)std::max<int64_t>(cap, kMaxPending);
     int rc = res_launch(S->res_form, P, S->dia, S->stream);

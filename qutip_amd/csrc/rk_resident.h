@@ -11,6 +11,7 @@ namespace qa {
 constexpr int kResRing = 32;        // slots of the stage-input ring
 constexpr int kResKept = 16;        // entries a lane keeps
 constexpr int kResSyncWords = 2048; // control words of one launch (see rk_resident.hip)
+constexpr int kResPolls = 1 << 20;  // polls of a wait, unless an engine sets them
 
 // The combine lists of the tableau: x_{i+1} (or y_front, for the last step
 // stage) = y_prev + sum_t dt tc[i][t] k_{tj[i][t]} + dt cs[i] k_i; the error
@@ -54,6 +55,7 @@ struct ResArgs {
     double2 *yout;
     int nneed, out_base, out_cap;
     int max_attempts;
+    int polls;  // bound of every wait, in polls of 0.4 us or more
 };
 
 // RES_KEPT: at most kResKept entries a lane, kept in registers; the others

@@ -56,7 +56,6 @@ namespace qa {
 namespace {
 
 constexpr int kResThreads = 512;      // at most; two waves per SIMD
-constexpr int kResPoll = 1 << 20;     // polls of a wait (0.4 us or more each)
 constexpr int kResChunk = 12;         // entries of a longer plain row in flight (registers)
 constexpr int kResTimes = 256;        // output times kept in LDS
 constexpr size_t kResLdsMax = 160 * 1024 - 8 * 1024;  // beside the static part
@@ -104,19 +103,20 @@ struct ResShared {
     alignas(16) int koff[kMaxStages + 1][kMaxStages];  // byte offsets of the lists' k
     int nt[kMaxStages + 1];
     int front[kMaxPending], okq[kMaxPending];
-    int wg, xcc, lidx, nloc, xccs, ok;
+    int wg, xcc, lidx, nloc, xccs, ok, commit;
 };
 
 struct Where {  // this workgroup's place in the barrier
     int wg, nwg, multi, xcc, lidx, nloc;
     unsigned xccs;  // XCDs that take part
     unsigned *sync;
+    int polls;      // polls of a wait
 };
 
 // Lanes 0 .. of wave 0 wait until every word (lane < cnt, at p + stride lane)
 // has reached g.
-__device__ __forceinline__ bool poll_words(const unsigned *p, bool mine, unsigned g) {
-    for (int k = 0; k < kResPoll; ++k) {
+__device__ __forceinline__ bool poll_words(const unsigned *p, bool mine, unsigned g, int polls) {
+    for (int k = 0; k < polls; ++k) {
         const bool ok = !mine || (int)(ld_agent(p) - g) >= 0;
         if (__all(ok)) return true;
     }
@@ -135,13 +135,14 @@ __device__ __forceinline__ void arrive(const Where &W, unsigned g) {
 __device__ __forceinline__ bool wait_all(const Where &W, unsigned g) {
     const int lane = threadIdx.x;
     unsigned *y = W.sync;
-    if (!W.multi) return poll_words(y + kSyFlags + (lane & 31), lane < W.nwg, g);
+    if (!W.multi) return poll_words(y + kSyFlags + (lane & 31), lane < W.nwg, g, W.polls);
     const bool part = lane < 16 && ((W.xccs >> (lane & 15)) & 1u);
     if (W.lidx == 0) {
-        if (!poll_words(y + kSyLocal + 32 * W.xcc + (lane & 31), lane < W.nloc, g)) return false;
+        if (!poll_words(y + kSyLocal + 32 * W.xcc + (lane & 31), lane < W.nloc, g, W.polls))
+            return false;
         if (part) st_agent(y + kSyGlobal + 32 * lane + W.xcc, g);
     }
-    return poll_words(y + kSyGlobal + 32 * W.xcc + (lane & 15), part, g);
+    return poll_words(y + kSyGlobal + 32 * W.xcc + (lane & 15), part, g, W.polls);
 }
 
 // x[r] = v, seen by every workgroup after the next barrier.
@@ -282,13 +283,14 @@ __global__ __launch_bounds__(kResThreads) void rk_resident_kernel(ResArgs P, Dia
     W.nloc = 0;
     W.xccs = 0;
     W.sync = P.sync;
+    W.polls = P.polls;
     if (P.multi) {
         // every workgroup has registered: the XCDs' counts are final
         if (tid == 0) {
             wait_stores();
             atomicAdd(P.sync + kSyRegister, 1u);
             int ok = 0;
-            for (int k = 0; k < kResPoll && !ok; ++k)
+            for (int k = 0; k < P.polls && !ok; ++k)
                 ok = ld_agent(P.sync + kSyRegister) >= (unsigned)P.nwg;
             unsigned m = 0;
             for (int i = 0; i < 16; ++i) {
@@ -650,7 +652,7 @@ __global__ __launch_bounds__(kResThreads) void rk_resident_kernel(ResArgs P, Dia
         unsigned d;
         d = 0;
         if (alive && W.wg != 0)
-            for (int k = 0; k < 4 * kResPoll && d == 0; ++k) d = ld_agent(P.sync + kSyCommit);
+            for (int k = 0; k / 4 < P.polls && d == 0; ++k) d = ld_agent(P.sync + kSyCommit);
         if (d == 0) {
             // workgroup 0 past the last barrier, or a wait that ran out: the
             // first to set the word decides for all.  (Write back can only
@@ -659,10 +661,12 @@ __global__ __launch_bounds__(kResThreads) void rk_resident_kernel(ResArgs P, Dia
             const unsigned old = atomicCAS(P.sync + kSyCommit, 0u, want);
             d = old ? old : want;
         }
-        S.ok = (int)d;
+        // a word of its own: a wave may still have to read S.ok of the wait
+        // that ended the loop
+        S.commit = (int)d;
     }
     __syncthreads();
-    if (S.ok != 1) return;
+    if (S.commit != 1) return;
     if (owner) {
         (cur ? P.y1 : P.y0)[r] = yprev;
         (cur ? P.y0 : P.y1)[r] = yfront;

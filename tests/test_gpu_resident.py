@@ -255,3 +255,51 @@ def test_resident_switched_off_and_on(monkeypatch):
         eng.set_resident(True)
         assert run(eng, other)[2][0] > 0
     assert free_bytes() > free - (50 << 20)
+
+
+@pytest.mark.parametrize("n,lanes,form", [
+    (64, 1, "uniform"), (2116, 4, "uniform"), (8192, 1, "sell"),  # one XCD
+    (8193, 1, "uniform"), (16385, 2, "sell"), (65536, 1, "uniform")])  # every XCD
+@pytest.mark.parametrize("polls", [0, 1, 4, 16, 64])
+def test_resident_gives_up(n, lanes, form, polls):
+    """Waits that end before the grid has come together (no polls at all, or
+    so few that some workgroups pass a barrier and others do not): the kernels
+    end, nothing is written back, and the launched loop goes on from the
+    state as it was; asked again, the engine's next launch goes through."""
+    print(f"resident give-up: n={n} lanes={lanes} {form} polls={polls}", flush=True)
+    rng = np.random.default_rng(n + 1)
+    A = _banded(n, n, few=form == "uniform")
+    kw = dict(lanes=lanes, coded=form == "uniform")
+    y0, fun = _state(n, rng), _fun(n, rng)
+    tl = np.array([0.0, 0.3, 0.31, 1.0, 3.0])
+    eng = RKEngine(A, "vern7", 1e-8, 1e-10, **kw)
+    eng.set_functionals(*fun)
+
+    def run(times):
+        vals, _, t = eng.run(times)
+        st = eng.stats()
+        return vals, t, eng.get_state()[1].to_array(), {k: st[k] for k in STATS}, _launches(st)
+
+    def same(a, b):
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[2], b[2])
+        assert a[1] == b[1] and a[3] == b[3]
+
+    eng.set_resident(False)
+    eng.set_state(0.0, y0)
+    ref = [run(tl[1:]), run([3.5, 4.0])]
+    assert ref[1][4][0] == 0
+    # from the state that was set, and from a resident launch's
+    for first in (polls, 1 << 20):
+        eng.set_resident(True)
+        _lib.call("qa_rk_set_resident_polls", eng.handle, first)
+        eng.set_state(0.0, y0)
+        got = run(tl[1:])
+        same(got, ref[0])
+        if first == 1 << 20:
+            assert got[4][0] >= 1 and got[4][1] == 0
+        _lib.call("qa_rk_set_resident_polls", eng.handle, polls)
+        eng.set_resident(True)
+        got = run([3.5, 4.0])
+        same(got, ref[1])
+        if polls == 0:
+            assert got[4][:2] == ((0, 2) if first == 0 else (1, 1))
