@@ -103,24 +103,25 @@ struct ResShared {
     alignas(16) int koff[kMaxStages + 1][kMaxStages];  // byte offsets of the lists' k
     int nt[kMaxStages + 1];
     int front[kMaxPending], okq[kMaxPending];
-    int wg, xcc, lidx, nloc, xccs, ok, commit;
+    int wg, xcc, lidx, nloc, xccs, ok, commit, polls;
 };
 
 struct Where {  // this workgroup's place in the barrier
     int wg, nwg, multi, xcc, lidx, nloc;
     unsigned xccs;  // XCDs that take part
     unsigned *sync;
-    int polls;      // polls of a wait
+    const int *polls;  // of a wait, at least one
 };
 
 // Lanes 0 .. of wave 0 wait until every word (lane < cnt, at p + stride lane)
 // has reached g.
-__device__ __forceinline__ bool poll_words(const unsigned *p, bool mine, unsigned g, int polls) {
-    for (int k = 0; k < polls; ++k) {
+__device__ __forceinline__ bool poll_words(const unsigned *p, bool mine, unsigned g,
+                                           const int *polls) {
+    for (int k = 1;; ++k) {
         const bool ok = !mine || (int)(ld_agent(p) - g) >= 0;
         if (__all(ok)) return true;
+        if (k >= *polls) return false;  // in LDS: read while the next poll would wait anyway
     }
-    return false;
 }
 
 // Wave 0, lane 0: this workgroup has arrived at barrier g.
@@ -269,11 +270,12 @@ __global__ __launch_bounds__(kResThreads) void rk_resident_kernel(ResArgs P, Dia
         } else {
             S.lidx = (int)atomicAdd(P.sync + kSyCount + x, 1u);
         }
+        S.polls = P.polls;
         S.wg = wg;
         S.xcc = (int)x;
     }
     __syncthreads();
-    if (S.wg < 0) return;  // another XCD's, or one too many: uniform
+    if (S.wg < 0 || P.polls < 1) return;  // another XCD's, or one too many: uniform
     Where W;
     W.wg = S.wg;
     W.nwg = P.nwg;
@@ -283,7 +285,7 @@ __global__ __launch_bounds__(kResThreads) void rk_resident_kernel(ResArgs P, Dia
     W.nloc = 0;
     W.xccs = 0;
     W.sync = P.sync;
-    W.polls = P.polls;
+    W.polls = &S.polls;
     if (P.multi) {
         // every workgroup has registered: the XCDs' counts are final
         if (tid == 0) {
