@@ -403,3 +403,13 @@ def test_operator_layouts_leave_the_matrix_as_it_is():
     for e, M in enumerate(mats):
         part = sp.csr_matrix((np.where(elem == e, A.data, 0), A.indices, A.indptr), A.shape)
         assert np.allclose(part @ x, M @ x, atol=1e-14)
+
+
+def test_no_kernel_is_launched_cooperatively():
+    """The first cooperative launch of a process opens a queue that stays, and
+    kernels of different streams overlap less from then on (the solve server
+    lost a fifth of its rate): grids that wait for each other are launched
+    like any other and bound their waits."""
+    import pathlib
+    for f in (pathlib.Path(qa.__file__).parent / "csrc").iterdir():
+        assert "CooperativeKernel" not in f.read_text(), f.name
