@@ -254,8 +254,8 @@ int qa_rk_set_hermitian(qa_rk_solver *s, int on);
  * counterpart. */
 int qa_rk_set_resident(qa_rk_solver *s, int on);
 /* How long a resident launch waits for its grid: polls of 0.4 us or more, at
- * most (and by default) 2^20; 0 makes every launch give up at once.  No
- * reference counterpart. */
+ * most (and by default) 2^20; 0 makes every launch give up at once, -1 is as
+ * if the runtime refused every launch.  No reference counterpart. */
 int qa_rk_set_resident_polls(qa_rk_solver *s, int polls);
 int qa_rk_get_hermitian(qa_rk_solver *s, int *on);
 /* Tile shape of the dense engine's MFMA kernels (the autotuner measures

@@ -2784,8 +2784,8 @@ int qa_rk_set_resident(qa_rk_solver *S, int on) {
 
 int qa_rk_set_resident_polls(qa_rk_solver *S, int polls) {
     QA_REQUIRE(S != nullptr, "qa_rk_set_resident_polls: null solver");
-    QA_REQUIRE(polls >= 0 && polls <= kResPolls,
-               "qa_rk_set_resident_polls: 0 <= polls <= %d", kResPolls);
+    QA_REQUIRE(polls >= -1 && polls <= kResPolls,
+               "qa_rk_set_resident_polls: -1 <= polls <= %d", kResPolls);
     S->res_polls = polls;
     return QA_OK;
 }
@@ -3198,10 +3198,11 @@ int res_chunk(qa_rk_solver *S, int out_base, bool *ran) {
     P.out_base = out_base;
     P.out_cap = (int)std::max<int64_t>(cap, kMaxPending);
     int rc = res_launch(S->res_form, P, S->dia, S->stream);
-    if (rc) {
+    if (rc) {  // refused: the state is as it was, and the launched loop needs less
+        (void)hipGetLastError();
         res_give(S);
         S->res = 0;
-        return rc;
+        return QA_OK;
     }
     ResFunArgs A;
     A.ctl = S->ctl;

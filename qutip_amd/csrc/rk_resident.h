@@ -70,7 +70,8 @@ size_t res_lds_bytes(int form, int lanes, int threads, int nk, int vbits);
 // Threads and workgroups for `lanes_total` lanes; false when the shape does
 // not fit this device (compute units, XCDs, LDS).
 bool res_plan(int form, int lanes, int64_t lanes_total, int nk, int vbits, ResArgs *P);
-// Clears the control words and launches the loop on s.
+// Clears the control words and launches the loop on s.  On an error the
+// state is as it was (at most the control words are cleared).
 int res_launch(int form, const ResArgs &P, const DiaOp &D, hipStream_t s);
 
 // The functionals of the outputs of a launch, from yout.

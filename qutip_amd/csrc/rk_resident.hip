@@ -805,6 +805,7 @@ bool res_plan(int form, int lanes, int64_t lanes_total, int nk, int vbits, ResAr
 int res_launch(int form, const ResArgs &P, const DiaOp &D, hipStream_t s) {
     const void *fn = res_kernel(form);
     QA_REQUIRE(fn != nullptr, "resident loop: no kernel for this operator");
+    QA_REQUIRE(P.polls >= 0, "resident loop: not launched");
     const size_t lds = res_lds_bytes(form, P.lanes, P.threads, P.nk, P.vbits);
     QA_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(res_prepare_kernel, dim3(1), dim3(256), 0, s, P.sync, P.ctl);

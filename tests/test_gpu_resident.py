@@ -260,12 +260,12 @@ def test_resident_switched_off_and_on(monkeypatch):
 @pytest.mark.parametrize("n,lanes,form", [
     (64, 1, "uniform"), (2116, 4, "uniform"), (8192, 1, "sell"),  # one XCD
     (8193, 1, "uniform"), (16385, 2, "sell"), (65536, 1, "uniform")])  # every XCD
-@pytest.mark.parametrize("polls", [0, 1, 4, 16, 64])
+@pytest.mark.parametrize("polls", [-1, 0, 1, 4, 16, 64])
 def test_resident_gives_up(n, lanes, form, polls):
     """Waits that end before the grid has come together (no polls at all, or
     so few that some workgroups pass a barrier and others do not): the kernels
     end, nothing is written back, and the launched loop goes on from the
-    state as it was; asked again, the engine's next launch goes through."""
+    state as it was, as it does where the launch is refused (-1); asked again, the engine's next launch goes through."""
     print(f"resident give-up: n={n} lanes={lanes} {form} polls={polls}", flush=True)
     rng = np.random.default_rng(n + 1)
     A = _banded(n, n, few=form == "uniform")
@@ -301,5 +301,6 @@ def test_resident_gives_up(n, lanes, form, polls):
         eng.set_resident(True)
         got = run([3.5, 4.0])
         same(got, ref[1])
-        if polls == 0:
-            assert got[4][:2] == ((0, 2) if first == 0 else (1, 1))
+        if polls <= 0:
+            gave_up = (0 if polls < 0 else 1) * (2 if first == polls else 1)
+            assert got[4][:2] == (0 if first == polls else 1, gave_up)
