@@ -58,7 +58,6 @@ namespace {
 constexpr int kResThreads = 512;      // at most; two waves per SIMD
 constexpr int kResChunk = 12;         // entries of a longer plain row in flight (registers)
 constexpr int kResTimes = 256;        // output times kept in LDS
-constexpr size_t kResLdsMax = 160 * 1024 - 8 * 1024;  // beside the static part
 
 // control words, a line (32 words) or more apart
 constexpr int kSyElected = 0;    // XCD + 1 of the first workgroup to arrive
@@ -105,6 +104,11 @@ struct ResShared {
     int front[kMaxPending], okq[kMaxPending];
     int wg, xcc, lidx, nloc, xccs, ok, commit, polls;
 };
+
+// Dynamic LDS beside it.
+constexpr size_t kResLdsMax = 160 * 1024 - (sizeof(ResShared) + 255) / 256 * 256;
+static_assert(sizeof(double2) * kMaxStages * kResThreads <= kResLdsMax,
+              "16 stages of one row a thread fit");
 
 struct Where {  // this workgroup's place in the barrier
     int wg, nwg, multi, xcc, lidx, nloc;
