@@ -253,6 +253,10 @@ int qa_rk_set_hermitian(qa_rk_solver *s, int on);
  * engine try again whose last resident launch gave up.  No reference
  * counterpart. */
 int qa_rk_set_resident(qa_rk_solver *s, int on);
+/* *planned: whether the engine's runs (other than single steps) take the
+ * resident step loop, planned now if it was not yet.  No reference
+ * counterpart. */
+int qa_rk_plan_resident(qa_rk_solver *s, int *planned);
 /* How long a resident launch waits for its grid: polls of 0.4 us or more, at
  * most (and by default) 2^20; 0 makes every launch give up at once, -1 is as
  * if the runtime refused every launch.  No reference counterpart. */

@@ -1,7 +1,7 @@
 """Autotuners: the SELL-C spmv of the RK stage kernels and the tile shape of
 the matrix-form MFMA kernels.
 
-Operators that the resident step loop takes get their lane count from a rule
+Engines that take the resident step loop get their lane count from a rule
 instead (resident_lanes).
 
 The tile shape is the number of lanes per row L (1, 2, 4, 8; C = 64 / L
@@ -109,11 +109,9 @@ def resident_lanes(A, coded=False):
 
 
 def lanes_for(A, fp32=False, coded=False):
+    """Lanes per row for the launched loop."""
     n = A.shape[0]
     nnz_row = A.nnz / max(n, 1)
-    L = resident_lanes(A, coded)
-    if L is not None:
-        return L
     if n < MIN_TUNE_ROWS or os.environ.get("QUTIP_AMD_NO_TUNE"):
         return heuristic_lanes(nnz_row)
     if not _CACHE:

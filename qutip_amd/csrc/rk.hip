@@ -2782,6 +2782,13 @@ int qa_rk_set_resident(qa_rk_solver *S, int on) {
     return QA_OK;
 }
 
+int qa_rk_plan_resident(qa_rk_solver *S, int *planned) {
+    QA_REQUIRE(S != nullptr && planned != nullptr, "qa_rk_plan_resident: null argument");
+    if (res_wanted(S) && S->res < 0) QA_CHECK(res_prepare(S));
+    *planned = res_wanted(S) && S->res == 1;
+    return QA_OK;
+}
+
 int qa_rk_set_resident_polls(qa_rk_solver *S, int polls) {
     QA_REQUIRE(S != nullptr, "qa_rk_set_resident_polls: null solver");
     QA_REQUIRE(polls >= -1 && polls <= kResPolls,

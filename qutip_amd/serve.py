@@ -123,9 +123,10 @@ class _Running:
         elif req.kind in ("se", "me"):
             if req.kind == "se":
                 A = -1j * req.H.to_csr()
-                self.eng = RKEngine(A, "vern7", o["rtol"], o["atol"], o["nsteps"])
-                # a resident grid would wait for the CUs the other requests use
-                self.eng.set_resident(False)
+                # the launched loop: a resident grid would wait for the CUs
+                # that other requests hold, and a process runs one at a time
+                self.eng = RKEngine(A, "vern7", o["rtol"], o["atol"], o["nsteps"],
+                                    resident=False)
                 psi = req.psi0.full().ravel()
                 kinds, fptr, rows, cols, w = self._quadratic(req, psi.size)
                 y0 = psi

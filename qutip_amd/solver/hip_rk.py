@@ -101,7 +101,8 @@ class RKEngine:
 
     def __init__(self, op, tableau="vern7", rtol=1e-6, atol=1e-8, nsteps=1000, first_step=0.0,
                  min_step=0.0, max_step=0.0, interpolate=True, fp32=False, lanes=None,
-                 dense=None, dense_precision="fp32", coded="auto", uniform="auto", td=None):
+                 dense=None, dense_precision="fp32", coded="auto", uniform="auto", td=None,
+                 resident=True):
         """``op``: the sparse generator A (dy/dt = A y), or None with
         ``dense=(H_nh, [c_ops])`` (numpy arrays) for the matrix-form
         Lindblad right-hand side: on MFMA (``dense_precision`` 'fp32',
@@ -115,7 +116,11 @@ class RKEngine:
         DeviceProgram of c_e), ...]) with ``op`` None: the elements go into
         one coded operator whose value table is split by element, and the
         stage kernels evaluate the programs at every stage time
-        (ValueError when the stacked operator has no coded form)."""
+        (ValueError when the stacked operator has no coded form).
+        ``lanes``: lanes per row, by default the resident step loop's where
+        this engine takes that loop, else the tuner's (the sums of a row go
+        by lanes, so results of other lane counts round differently).
+        ``resident``: False keeps the launched loop (set_resident)."""
         tab = TABLEAUS[tableau] if isinstance(tableau, str) else tableau
         self.tableau = tab
         self._a = np.ascontiguousarray(tab["a"], dtype=np.float64)
@@ -169,24 +174,25 @@ class RKEngine:
                 raise ValueError(f"1 to {MAX_COEF} time-dependent elements")
             A, elem = _data.stacked_elements([A0] + [M for M, _ in parts])
             self.n = A.shape[0]
-            if lanes is None:
-                lanes = autotune.lanes_for(A, False, True)
-            self.lanes = lanes
             self.coded = True
-            self.sell = _data.SellMatrix(A, lanes=lanes, uniform=uniform, elem=elem)
-            sptr, cols, vals = self.sell.ptrs
-            rc = L.qa_rk_create_coded(
-                C.byref(h), self.n, lanes, self.sell.nslices, C.c_void_p(sptr),
-                C.c_void_p(cols), C.c_void_p(vals), C.c_void_p(self.sell.otab_ptr),
-                self.sell.vbits, *tab_args)
-            _lib.check(rc, "qa_rk_create_coded")
-            self.handle = h
             progs = DeviceProgram.concat([p for _, p in parts])
             start, code, consts = progs.arrays()
-            vstart = np.ascontiguousarray(self.sell.vstart[1:], dtype=np.int32)
-            self._td_host = (start, vstart, code, consts)
-            _lib.call("qa_rk_set_coefficients", h, len(parts), _ip(start), _ip(vstart),
-                      len(code), _ip(code), len(consts), _dp(consts.view(np.float64)))
+
+            def create(lanes):
+                self.sell = _data.SellMatrix(A, lanes=lanes, uniform=uniform, elem=elem)
+                sptr, cols, vals = self.sell.ptrs
+                rc = L.qa_rk_create_coded(
+                    C.byref(h), self.n, lanes, self.sell.nslices, C.c_void_p(sptr),
+                    C.c_void_p(cols), C.c_void_p(vals), C.c_void_p(self.sell.otab_ptr),
+                    self.sell.vbits, *tab_args)
+                _lib.check(rc, "qa_rk_create_coded")
+                self.handle = h
+                vstart = np.ascontiguousarray(self.sell.vstart[1:], dtype=np.int32)
+                self._td_host = (start, vstart, code, consts)
+                _lib.call("qa_rk_set_coefficients", h, len(parts), _ip(start), _ip(vstart),
+                          len(code), _ip(code), len(consts), _dp(consts.view(np.float64)))
+
+            self.lanes = self._create_lanes(create, h, A, False, True, lanes, resident)
         else:
             if isinstance(op, _data.HipCSR):
                 A = op.to_scipy()
@@ -198,24 +204,29 @@ class RKEngine:
             if coded == "auto":
                 coded = _data.sell_coded_arrays(A, 1, fp32) is not None
             coded = bool(coded)
-            if lanes is None:
-                lanes = autotune.lanes_for(A, fp32, coded)
-            self.lanes = lanes
             self.coded = coded
-            self.sell = _data.SellMatrix(A, fp32=fp32, lanes=lanes, coded=coded, uniform=uniform)
-            sptr, cols, vals = self.sell.ptrs
-            if coded:
-                rc = L.qa_rk_create_coded(
-                    C.byref(h), self.n, lanes, self.sell.nslices, C.c_void_p(sptr),
-                    C.c_void_p(cols), C.c_void_p(vals), C.c_void_p(self.sell.otab_ptr),
-                    self.sell.vbits, *tab_args)
-                _lib.check(rc, "qa_rk_create_coded")
-            else:
-                rc = L.qa_rk_create(
-                    C.byref(h), self.n, lanes, self.sell.nslices, C.c_void_p(sptr),
-                    C.c_void_p(cols), C.c_void_p(vals), int(fp32), *tab_args)
-                _lib.check(rc, "qa_rk_create")
+
+            def create(lanes):
+                self.sell = _data.SellMatrix(A, fp32=fp32, lanes=lanes, coded=coded,
+                                             uniform=uniform)
+                sptr, cols, vals = self.sell.ptrs
+                if coded:
+                    rc = L.qa_rk_create_coded(
+                        C.byref(h), self.n, lanes, self.sell.nslices, C.c_void_p(sptr),
+                        C.c_void_p(cols), C.c_void_p(vals), C.c_void_p(self.sell.otab_ptr),
+                        self.sell.vbits, *tab_args)
+                    _lib.check(rc, "qa_rk_create_coded")
+                else:
+                    rc = L.qa_rk_create(
+                        C.byref(h), self.n, lanes, self.sell.nslices, C.c_void_p(sptr),
+                        C.c_void_p(cols), C.c_void_p(vals), int(fp32), *tab_args)
+                    _lib.check(rc, "qa_rk_create")
+                self.handle = h
+
+            self.lanes = self._create_lanes(create, h, A, fp32, coded, lanes, resident)
         self.handle = h
+        if not resident:
+            self.set_resident(False)
         self.nfun = 0
         # entries between consecutive states in a states_out buffer
         self.npad = self.sell.nslices * (64 // self.lanes) if self.sell is not None else self.n
@@ -227,6 +238,26 @@ class RKEngine:
             if not _data._defer("engine", h):
                 _lib._lib.qa_rk_destroy(h)
             self.handle = None
+
+    @staticmethod
+    def _create_lanes(create, h, A, fp32, coded, lanes, resident):
+        """create(lanes) and the lane count: the resident step loop's only
+        where the engine then plans that loop (tableau, LDS, device), else the
+        tuner's for the launched loop."""
+        if lanes is None and resident:
+            lanes = autotune.resident_lanes(A, coded)
+            if lanes is not None:
+                create(lanes)
+                planned = C.c_int(0)
+                _lib.call("qa_rk_plan_resident", h, C.byref(planned))
+                if planned.value:
+                    return lanes
+                _lib.call("qa_rk_destroy", h)
+                h.value = lanes = None
+        if lanes is None:
+            lanes = autotune.lanes_for(A, fp32, coded)
+        create(lanes)
+        return lanes
 
     def set_functionals(self, kinds, fptr, rows, cols, w):
         """Linear / quadratic functionals of the state evaluated at every
@@ -247,7 +278,8 @@ class RKEngine:
         self.nfun = len(kinds)
 
     def set_resident(self, on):
-        """Whether runs may take the resident step loop (same bits)."""
+        """Whether runs may take the resident step loop (same bits: the lane
+        count stays)."""
         _lib.call("qa_rk_set_resident", self.handle, int(bool(on)))
 
     def set_hermitian(self, on, tune=True):

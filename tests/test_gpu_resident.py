@@ -17,8 +17,9 @@ import scipy.sparse as sp
 pytestmark = pytest.mark.gpu
 
 import qutip_amd as qa  # noqa: E402
-from qutip_amd import _lib  # noqa: E402
+from qutip_amd import _lib, autotune  # noqa: E402
 from qutip_amd.solver.hip_rk import RKEngine, time_dependent_operator  # noqa: E402
+from qutip_amd.solver.tableaus import TABLEAUS  # noqa: E402
 from tests import systems  # noqa: E402
 
 STATS = ("attempts", "accepted", "dense_preps", "rhs_evals", "status", "out_idx")
@@ -304,3 +305,47 @@ def test_resident_gives_up(n, lanes, form, polls):
         if polls <= 0:
             gave_up = (0 if polls < 0 else 1) * (2 if first == polls else 1)
             assert got[4][:2] == (0 if first == polls else 1, gave_up)
+
+
+def test_resident_lanes_only_for_its_engines(monkeypatch):
+    """The resident loop's lane count goes to engines that take that loop: not
+    to one kept on the launched loop, nor to a tableau it refuses (here one
+    whose first stage is not at the step's start)."""
+    print("resident lanes", flush=True)
+    monkeypatch.setenv("QUTIP_AMD_NO_TUNE", "1")
+    A = _banded(5000, offs=(0, 1, -1, 3, -3, 7, -7, 9, -9, 20, -20, 30, -30), few=False)
+    launched, ruled = autotune.lanes_for(A), autotune.resident_lanes(A)
+    assert launched != ruled
+    off = dict(TABLEAUS["tsit5"], c=np.asarray(TABLEAUS["tsit5"]["c"]) + 0.01)
+    for kw, lanes in (({}, ruled), ({"resident": False}, launched), ({"tableau": off}, launched),
+                      ({"lanes": 8}, 8)):
+        eng = RKEngine(A, rtol=1e-6, atol=1e-8, coded=False, **kw)
+        assert eng.lanes == eng.sell.lanes == lanes
+        if "tableau" not in kw:
+            eng.set_state(0.0, _state(5000, np.random.default_rng(2)))
+            eng.run([0.01])
+            assert (eng.stats()["resident_launches"] > 0) == (kw != {"resident": False})
+    m = systems.ising(3, 0.1)
+    H = qa.QobjEvo([m["H"], [m["e_ops"][0], "cos(t)"]])
+    td = time_dependent_operator(qa.MESolver(H, m["c_ops"]).rhs.matmul_data)
+    for kw in ({}, {"resident": False}):
+        eng = RKEngine(None, rtol=1e-6, atol=1e-8, td=td, **kw)
+        eng.set_state(0.0, _state(64, np.random.default_rng(2)))
+        eng.run([0.01])
+        assert (eng.stats()["resident_launches"] > 0) == (not kw)
+
+
+def test_served_requests_keep_the_launched_loop():
+    print("served sesolve of 1200 rows", flush=True)
+    from qutip_amd.serve import SolveRequest, _Running
+    d = 1200
+    rng = np.random.default_rng(8)
+    H = qa.Qobj(sp.csr_matrix(sp.diags([rng.uniform(size=d - 1), rng.uniform(size=d),
+                                        np.zeros(d - 1)], [-1, 0, 1]), dtype=complex))
+    H = H + H.dag()
+    req = SolveRequest("se", H, qa.basis(d, 0), np.linspace(0, 0.5, 3), e_ops=[qa.num(d)])
+    run = _Running(req)
+    while not run.poll():
+        pass
+    st = run.eng.stats()
+    assert req.error is None and st["resident_launches"] == 0 and st["graph_launches"] > 0
