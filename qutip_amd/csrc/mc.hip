@@ -1322,7 +1322,9 @@ int launch_mc_cfg(const McArgs &A0, int threads, int blocks, hipStream_t s) {
     const bool hl = P.hl;
     const int fm = !P.pk ? OP_ELL : A.pk_imag ? OP_PACKED_IM : OP_PACKED;
     const void *fn;
-    if constexpr (!SMALL)
+    if constexpr (!SMALL && NT < kMcThreads)
+        fn = (const void *)mc_traj_kernel<R, NT, OP_ELL>;  // not for packed operators (launch_mc)
+    else if constexpr (!SMALL)
         fn = fm == OP_PACKED_IM ? (const void *)mc_traj_kernel<R, NT, OP_PACKED_IM>
              : fm == OP_PACKED  ? (const void *)mc_traj_kernel<R, NT, OP_PACKED>
                                 : (const void *)mc_traj_kernel<R, NT, OP_ELL>;
@@ -1348,11 +1350,17 @@ bool shape_mc(int d, int *threads) {
 }
 
 // The kernels are compiled for up to 1024 threads (128 vector registers each,
-// so 16 waves a CU), and the whole-solve kernel also for up to 512 (256
-// registers, 8 waves a CU, nothing spilled): that form is the faster one
-// where no CU gets a second workgroup (400 rows, one system: 2.96 ms against
-// 3.23).  Trajectories come in numbers: 512 of 512 rows 3.3 ms with 1024, 4.2
-// with 512, and 8192 of 256 rows 16 against 24 ms; 500 of them are equal.
+// so 16 waves a CU), and some also for up to 512 (256 registers, 8 waves a CU,
+// nothing spilled).  The whole-solve kernel takes that form where no CU gets a
+// second workgroup (400 rows, one system: 2.96 ms against 3.23).
+// Trajectories of a packed operator come in numbers: 512 of 512 rows 3.3 ms
+// with 1024, 4.2 with 512, and 8192 of 256 rows 16 against 24 ms; 500 of them
+// are equal.  Those of an ELL operator in complex128 load eight entries at a
+// time with 256 registers and four with 128, and wide rows are bound by those
+// loads: with 512 while the 8 waves a CU then holds are enough for every
+// trajectory at once (ms with 512 / 1024, width = rows: 64 of 512 rows 41.9 /
+// 50.9, 512 of 256 15.7 / 16.4, 256 of 128 4.2 / 4.9; beyond it 1500 of 128
+// 11.0 / 9.1, and with 16 to 20 entries a row 500 of 300 8.9 / 6.1).
 template <typename R, bool SMALL = false>
 int launch_mc(const McArgs &A, int blocks, hipStream_t s) {
     int threads;
@@ -1360,8 +1368,11 @@ int launch_mc(const McArgs &A, int blocks, hipStream_t s) {
         qa::set_error("qa_mc_run: d = %d does not fit the trajectory kernel", A.d);
         return QA_ERR_ARG;
     }
-    if constexpr (SMALL)
-        if (threads <= kMcThreads / 2 && blocks <= kChipCUs)
+    constexpr int kWaves = kMcThreads / 2 / QA_WAVE;  // a CU's with 256 registers
+    if constexpr (SMALL || sizeof(R) == 8)
+        if (threads <= kMcThreads / 2 &&
+            (SMALL ? blocks <= kChipCUs
+                   : !A.pk_code && blocks <= kChipCUs * (kWaves / (threads / QA_WAVE))))
             return launch_mc_cfg<R, kMcThreads / 2, SMALL>(A, threads, blocks, s);
     return launch_mc_cfg<R, kMcThreads, SMALL>(A, threads, blocks, s);
 }

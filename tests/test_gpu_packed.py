@@ -147,3 +147,28 @@ def test_trajectories_packed_against_ell(N, fp32):
     hit = np.arange(tr.shape[1])[None, :] < ir[:, 1:2]
     assert (wg[hit] == wr[hit]).all()
     assert np.abs(tg[hit] - tr[hit]).max(initial=0.0) <= 4 * tol + (1e-6 if fp32 else 1e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,fit", [(20, 2048), (64, 2048), (65, 1024), (129, 512), (300, 256),
+                                   (512, 256)])
+def test_ell_trajectories_of_both_forms(d, fit):
+    """An operator that does not pack: `fit` trajectories are the most that
+    take the kernel with 256 registers (eight entries a load), one more takes
+    the other (four).  Same sums in the same order: the same bits."""
+    print(f"ELL trajectories d={d} fit={fit}", flush=True)
+    H = qa.rand_herm(d, density=min(1.0, 30.0 / d), seed=d)
+    S = qa.MCSolver(H, [0.3 * qa.destroy(d)])
+    psi = np.ones(d, dtype=complex) / np.sqrt(d)
+    tl = np.linspace(0, 0.5, 4)
+    one = M.draws_for(np.random.SeedSequence(5).spawn(7), 64)
+    assert S._device_ops(False)[4] is None
+    out = []
+    for nt in (fit, fit + 1):
+        e, info, _, _ = S.run_batch(psi, tl, [qa.num(d)], np.resize(one, (nt, 64)))
+        assert (info[:, 0] == 0).all()
+        # every seventh trajectory is the same one
+        assert (info == np.resize(info[:7], info.shape)).all()
+        assert np.array_equal(e, np.resize(e[:7], e.shape))
+        out.append((e[:7], info[:7]))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
