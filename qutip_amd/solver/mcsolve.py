@@ -234,7 +234,18 @@ def _packed_host(A, d, fp32):
     lanes of a wave mostly read one value and shifted runs of the vector; in
     complex64 by their columns, with the number of them before the diagonal
     in one more row of codes, so that the sums round as the ELL form's do."""
-    A = sp.csr_matrix(A, dtype=np.complex64 if fp32 else np.complex128)
+    A = sp.csr_matrix(A)
+    dtype = np.complex64 if fp32 else np.complex128
+    # the fullest row alone refuses most operators that do not pack (for 512
+    # dense rows in 0.1 ms instead of 13)
+    r = int(np.argmax(np.diff(A.indptr)))
+    s = slice(A.indptr[r], A.indptr[r + 1])
+    row = sp.csr_matrix((A.data[s].astype(dtype), A.indices[s].copy(), [0, s.stop - s.start]),
+                        shape=(1, d))
+    row.sum_duplicates()
+    if ((row.data != 0) & (row.indices != r)).sum() > PACK_WIDTH:
+        return None
+    A = sp.csr_matrix(A, dtype=dtype)
     A = A.copy()
     A.sum_duplicates()
     n = np.repeat(np.arange(d), np.diff(A.indptr))

@@ -56,13 +56,25 @@ def test_packed_host_holds_the_operator(n, width, imag):
     assert (B == A.toarray()).all()
 
 
-def test_packed_host_refuses():
+def test_packed_host_refuses(monkeypatch):
     tab = TABLEAUS["vern7"]
     assert M._packed_host(_op(200, 17, True), 200, False) is None  # too many entries a row
     A = sp.csr_matrix(np.diag(np.arange(1.0, 300), 1) * 1j)  # 299 distinct values
     assert M._packed_host(A, 300, False) is None
     A = _op(1024, 4, True) + sp.diags(1j * (np.arange(1.0, 1024) % 70), 1)
     assert M._packed_host(A, 1024, False) is None  # more than 6 bits of values
+    # stored zeros do not count
+    B = _op(200, 16, True).tocoo()
+    z = np.arange(30)
+    B = sp.csr_matrix((np.concatenate([B.data, 0.0 * z]),
+                       (np.concatenate([B.row, 0 * z + 7]),
+                        np.concatenate([B.col, 100 + z]))), shape=(200, 200))
+    assert np.diff(B.indptr).max() > 17 and M._packed_host(B, 200, False) is not None
+    assert M._packed_host(sp.csr_matrix((3, 3), dtype=complex), 3, False) is not None
+    dense = sp.csr_matrix(np.random.default_rng(0).normal(size=(512, 512)) + 0j)
+    monkeypatch.setattr(sp.csr_matrix, "copy", None)  # refused before any work on the whole
+    assert M._packed_host(dense, 512, False) is None
+    monkeypatch.undo()
     ok = _op(20, 4, True)
     assert M.packed_op(ok, 20, False, TABLEAUS["tsit5"], True) is None
     assert M.packed_op(ok, 20, False, tab, False) is None
