@@ -671,10 +671,12 @@ __device__ __forceinline__ void recompute_safe_step(Ctx<R, NT, FM> &c, Traj<R> &
     if (err == 0.0) {
         f = 10.0;
     } else {
-        // three square roots for vern7's eighth root: pow, which every wave
-        // computes, took 3800 clocks of a step in one wave and 13000 in 16
-        f = c.tab->order == 7 ? 0.9 / sqrt(sqrt(sqrt(err)))
-                              : 0.9 * pow(err, -1.0 / (c.tab->order + 1));
+        // square and cube roots for vern7's eighth root and tsit5's sixth: pow,
+        // which every wave computes, took 3800 clocks of a step in one wave
+        // and 13000 in 16 (600 tsit5 solves of 1024 rows 3.8 -> 3.25 ms)
+        f = c.tab->order == 7   ? 0.9 / sqrt(sqrt(sqrt(err)))
+            : c.tab->order == 5 ? 0.9 / sqrt(cbrt(err))
+                                : 0.9 * pow(err, -1.0 / (c.tab->order + 1));
         f = fmin(10.0, f);
         f = fmax(0.2, f);
     }

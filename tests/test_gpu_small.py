@@ -201,3 +201,25 @@ def test_sesolve_initial_point_from_the_kernel():
         got = np.asarray(r.expect[k])
         assert abs(got[0] - want) < 1e-14, (k, got[0], want)
         assert np.abs(got - ref[k]).max() < 1e-6, k
+
+
+@pytest.mark.parametrize("N", [4, 14])
+def test_tsit5_step_sequence(N):
+    """The step factor of an order 5 method (a sixth root) on 64 and 784 rows:
+    the oracle's attempts, and <O>(t) within the tolerance of the method."""
+    print(f"small: tsit5, JC N={N}", flush=True)
+    m = models.jaynes_cummings(N=N)
+    Lm = models.liouvillian(m["H"], m["c_ops"])
+    d = m["H"].shape[0]
+    tl = np.linspace(0.0, 3.0, 13)
+    ss = SmallSolve(Lm, "tsit5", **OPTS)
+    fun = _functionals(m["e_ops"], d)
+    ss.set_functionals(*fun)
+    rho0 = models.vec(models.ket2dm(m["psi0"]))
+    vals, _, info = ss.run(tl[0], rho0, tl[1:])
+    _, _, ost = cbind.rk_solve(Lm, rho0, tl, tableaus.tsit5,
+                               cbind.functionals_from_ops(m["e_ops"], d), **OPTS)
+    print(f"  attempts {info[0, 3]}, oracle {ost['n_attempts']}", flush=True)
+    assert info[0, 0] >= 0 and info[0, 3] == ost["n_attempts"]
+    ref = exact.mesolve_expect(m["H"], m["c_ops"], m["psi0"], tl, m["e_ops"])
+    assert np.abs(_expect(vals[0]).T - ref[:, 1:]).max() < 1e-6
