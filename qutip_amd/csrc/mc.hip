@@ -987,7 +987,7 @@ __global__ __launch_bounds__(NT) void mc_traj_kernel(McArgs A) {
         s.y = mk<R>((R)p0.x, (R)p0.y);
         if (!draw(g, target)) s.status = MC_DRAWS_EXHAUSTED;
         int k = 0;          // the next output
-        int guard = 0;      // advances since the last output
+        int guard = 0;      // steps since the last output
         bool start = true, search = false;
         int tries = 0;
         Uni t_out = A.times[0];  // output k
@@ -1004,7 +1004,7 @@ __global__ __launch_bounds__(NT) void mc_traj_kernel(McArgs A) {
                 t_old = s.t;
                 norm_old = 1.0;  // after a jump (an output below sets it again)
             } else {
-                if (++guard > 100000) {
+                if (!search && ++guard > 100000) {  // a search has its own bound
                     s.status = MC_NO_PROGRESS;
                     break;
                 }

@@ -112,3 +112,21 @@ def test_plain_drop_in_loop_matches_batched_kernel():
     assert (info[:, 0] == 0).all()
     assert jumps.tolist() == info[:, 1].tolist()
     assert np.abs(runs - ex).max() < 1e-5
+
+
+def test_many_jumps_between_two_outputs():
+    """Some 50000 jumps between two output times, in 75000 steps and as many
+    searches: the limit of 100000 steps without an output counts steps, not
+    the searches' advances; twice the steps reach it (MC_NO_PROGRESS, -12)."""
+    print("mcsolve: 50000 jumps between two outputs", flush=True)
+    draws = np.random.default_rng(1).uniform(size=(1, 60000))
+    for opts, status in (({}, 0), ({"rtol": 1e-9, "atol": 1e-11}, -12)):
+        S = qa.MCSolver(0.05 * qa.sigmaz(), [qa.sigmax()], options=opts)
+        _, info, tj, _ = S.run_batch(np.array([1.0, 0.0], dtype=complex),
+                                     np.array([0.0, 50000.0]), [qa.sigmaz()], draws,
+                                     max_jumps=60000)
+        print(f"  status {info[0, 0]}, {info[0, 1]} jumps, {info[0, 3]} attempts", flush=True)
+        assert info[0, 0] == status
+        # the waiting times are exponential with rate 1
+        gaps = np.diff(tj[0, :info[0, 1]])
+        assert len(gaps) > 30000 and abs(gaps.mean() - 1.0) < 5 / np.sqrt(len(gaps))
