@@ -17,6 +17,12 @@ from qutip_amd.solver.hip_rk import RKEngine  # noqa: E402
 from oracle import cbind, models  # noqa: E402
 
 
+@pytest.fixture(autouse=True)
+def _launched_loop(monkeypatch):
+    """These engines would take the resident step loop otherwise."""
+    monkeypatch.setenv("QUTIP_AMD_RESIDENT", "0")
+
+
 def _solve(eng, y0, tl, fun):
     fptr, fidx, fw = fun
     eng.set_functionals(np.zeros(len(fptr) - 1, np.int32), fptr.astype(np.int32),
@@ -38,9 +44,11 @@ def _engines(monkeypatch, make):
 
 def _check_replays(eager, graph, y0, tl, fun, other_work):
     ref = _solve(eager, y0, tl, fun)
+    assert eager.stats()["graph_launches"] > 0
     for rep in range(3):
         got = _solve(graph, y0, tl, fun)
         assert got[2] == ref[2], rep
+        assert graph.stats()["resident_launches"] == 0
         assert np.array_equal(got[0], ref[0]), rep
         assert np.array_equal(got[1], ref[1]), rep
         other_work()

@@ -23,6 +23,12 @@ from qutip_amd.solver.hip_rk import RKEngine  # noqa: E402
 from oracle import cbind, models  # noqa: E402
 
 
+@pytest.fixture(autouse=True)
+def _launched_loop(monkeypatch):
+    """These engines would take the resident step loop otherwise."""
+    monkeypatch.setenv("QUTIP_AMD_RESIDENT", "0")
+
+
 def _padded(fun, n, extra, quad):
     """fun plus one functional of `extra` entries (more than 16: every
     functional is then summed from partial sums)."""
@@ -42,7 +48,9 @@ def _run(eng, fun, y0, tl):
     eng.set_state(tl[0], y0)
     vals, st, _ = eng.run(tl[1:])
     assert st >= 0
-    return vals, eng.stats()
+    stats = eng.stats()
+    assert stats["resident_launches"] == 0
+    return vals, stats
 
 
 def _linear(ops, d):

@@ -22,6 +22,12 @@ from tests import systems  # noqa: E402
 STATS = ("attempts", "accepted", "dense_preps", "rhs_evals", "status", "out_idx")
 
 
+@pytest.fixture(autouse=True)
+def _launched_loop(monkeypatch):
+    """These engines would take the resident step loop otherwise."""
+    monkeypatch.setenv("QUTIP_AMD_RESIDENT", "0")
+
+
 def _pair(monkeypatch, make):
     """(full iterations only, step-only iterations allowed)."""
     monkeypatch.setenv("QUTIP_AMD_STEP_ONLY", "0")
@@ -41,6 +47,7 @@ def _solve(eng, y0, tl, fun, store):
     assert st >= 0
     t, y = eng.get_state()
     stats = eng.stats()
+    assert stats["resident_launches"] == 0
     return (vals, t, y.to_array().ravel(), buf.to_array() if store else None,
             {k: stats[k] for k in STATS}, stats["graph_launches"])
 
