@@ -120,11 +120,10 @@ def bench_mcsolve(qa, systems, log, ntraj=2048, reps=3, cpu=True):
             mean, sig = v.mean(0), v.std(0) / np.sqrt(ntraj)
             dev = np.abs(mean - golden["expect"][k])
             worst_sigma = max(worst_sigma, float((dev[1:] / sig[1:]).max()))
-        # operator bytes the trajectories read from L2: at least 10 RHS per
-        # attempt, each reading the whole ELL (width x d columns and values)
-        width = solver._device_ops(prec == "fp32")[1][0]
+        # whether the kernel has the operator packed (codes in registers,
+        # values in LDS) or reads its ELL from L2 in every stage
+        packed = solver._device_ops(prec == "fp32")[4] is not None
         vb = 8 if prec == "fp32" else 16
-        op_bytes = 10 * float(info[:, 3].sum()) * width * s["H"].shape[0] * (vb + 4)
         # the algorithmic bytes of a batched RHS: every trajectory's state
         # read and its derivative written (2 d 16 B, complex128; 2 d 8 B for
         # complex64) plus the operator once per batch of ntraj; at least 10
@@ -137,8 +136,7 @@ def bench_mcsolve(qa, systems, log, ntraj=2048, reps=3, cpu=True):
                      "all_ok": ok, "jumps": int(info[:, 1].sum()),
                      "rk_attempts": int(info[:, 3].sum()),
                      "max_dev_over_sigma_vs_mesolve": round(worst_sigma, 3),
-                     "ell_width": int(width),
-                     "operator_l2_read_gbs_lower_bound": round(op_bytes / best / 1e9, 1),
+                     "operator_form": "packed" if packed else "ELL",
                      "roofline": {
                          "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                          "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
@@ -414,6 +412,7 @@ def bench_serving(systems, log, nreq=2040, warm=40, policy="sjf", cpu=True, cpu_
 
 COPY_BYTES = 64 << 20
 TRAFFIC_FILE = ROOT / "profiles" / "rk_stage_kernel_ising8_traffic.txt"
+RESIDENT_TRAFFIC_FILE = ROOT / "profiles" / "rk_resident_kernel_ising8_traffic.txt"
 
 
 def pmc_workload():
@@ -423,7 +422,8 @@ def pmc_workload():
     that many bytes), then, for the plain and then the coded operator form
     and each SELL shape (1, 2, 4, 8 lanes per row), 3 launches of each of
     the 16 stage kernels of the L=8 Ising solve in solve order (direct
-    launches, no graph)."""
+    launches, no graph); last, three runs of that solve on the resident step
+    loop."""
     from qutip_amd import _lib, data as qd
     from qutip_amd.solver.hip_rk import RKEngine
     from tests import systems
@@ -448,6 +448,12 @@ def pmc_workload():
             _lib.call("qa_device_sync")
     log(f"pmc workload: 3 copies of {COPY_BYTES} B, then 16 x 3 stage launches for each of "
         f"lanes 1, 2, 4, 8, plain then coded (nnz {L.nnz})")
+    solver = qa.MESolver(s["H"], s["c_ops"], options={"rtol": 1e-8, "atol": 1e-10})
+    for _ in range(3):
+        solver.run(s["psi0"], s["tlist"], e_ops=s["e_ops"])
+    st = solver._integrator.stats()
+    log(f"pmc workload: 3 resident solves, lanes {solver._integrator._engine.lanes}, "
+        f"coded {solver._integrator._engine.coded}, {st}")
 
 
 MC_TRAFFIC_FILE = ROOT / "profiles" / "mc_traj_kernel_ising10_traffic.txt"
@@ -537,6 +543,37 @@ def dense_rhs_probe(N, nc, prec="fp32"):
           flush=True)
 
 
+def resident_roofline(solver, psi0, tlist, L, stats, lanes, coded, reps=5):
+    """Roofline entry of the resident step loop: the engine's run alone (state
+    on the device, host clock around qa_rk_run, which waits for the device)
+    over the solve's right-hand sides."""
+    from qutip_amd import data as qd
+    eng = solver._integrator._engine
+    n, nnz = L.shape[0], L.nnz
+    psi = psi0.full().ravel()
+    rho0 = qd.HipDense.from_array(np.outer(psi, psi.conj()).ravel(order="F"))
+    best, launches = float("inf"), 0
+    for _ in range(reps):
+        eng.set_state(tlist[0], rho0)
+        t0 = time.perf_counter()
+        eng.run(tlist[1:])
+        best = min(best, time.perf_counter() - t0)
+        launches = eng.stats()["resident_launches"]
+    us = best * 1e6 / stats["rhs_evals"]
+    rhs_bytes = nnz * 20 + (n + 1) * 4 + 2 * n * 16
+    achieved = rhs_bytes / us * 1e-3
+    log(f"resident step loop (lanes {lanes}): {us:.2f} us per RHS, {launches} launches a solve: "
+        f"{rhs_bytes / 1e6:.2f} MB per RHS -> {achieved:.0f} GB/s")
+    return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": round(achieved / HBM_PEAK_GBS, 4),
+            "traffic": read_traffic(lanes, coded, RESIDENT_TRAFFIC_FILE),
+            "kernel": "rk_resident_kernel", "us_per_rhs": round(us, 3),
+            "launches_per_solve": launches, "run_ms": round(best * 1e3, 3),
+            "algorithmic_bytes_per_rhs": int(rhs_bytes),
+            "algorithmic_unit": "one RHS of the CSR complex128 product: nnz*20 + (n+1)*4 + "
+                                "2*n*16 bytes (the kernel keeps the operator on the chip)"}
+
+
 def stage_roofline(RKEngine, L, stats, lanes, coded, reps=20):
     """Roofline entry of the stage kernel: HIP events on the engine's stream
     around back-to-back rounds of the 16 stage launches in solve order
@@ -607,13 +644,13 @@ def _lib_call(*a):
     _lib.call(*a)
 
 
-def read_traffic(lanes, coded=False):
-    """HBM bytes per stage-kernel launch from the committed counter summary
-    (FETCH_SIZE + WRITE_SIZE scaled by the copy calibration) when it was
-    taken on the same operator form and SELL shape, else None."""
+def read_traffic(lanes, coded=False, path=None):
+    """HBM bytes per launch (the resident loop: per RHS) from the committed
+    counter summary (FETCH_SIZE + WRITE_SIZE scaled by the copy calibration)
+    when it was taken on the same operator form and SELL shape, else None."""
     vals = {}
     try:
-        for line in TRAFFIC_FILE.read_text().splitlines():
+        for line in (path or TRAFFIC_FILE).read_text().splitlines():
             if ":" in line and not line.startswith(("-", "|", "#", "`")):
                 k, v = line.split(":", 1)
                 vals[k.strip()] = v.strip()
@@ -698,7 +735,10 @@ def main():
 
     lanes = solver._integrator._engine.lanes
     coded = solver._integrator._engine.coded
-    roof = stage_roofline(RKEngine, L, stats, lanes, coded)
+    resident = stats["resident_launches"] > 0
+    stage = stage_roofline(RKEngine, L, stats, lanes, coded)
+    roof = (resident_roofline(solver, s["psi0"], tlist, L, stats, lanes, coded) if resident
+            else stage)
 
     out = {
         "metric": METRIC, "value": round(value, 4), "unit": "solves/s", "n_gpus": 1,
@@ -709,13 +749,15 @@ def main():
         "config": {
             "workload": "mesolve dissipative TFIM L=8: Liouvillian 65536^2 CSR, 1245183 nnz, "
                         "complex128; vern7 rtol=1e-8 atol=1e-10; t in [0,10], 200 outputs; "
-                        "2 e_ops; fused hip_rk (device step control, hipGraph replay)",
+                        "2 e_ops; fused hip_rk (device step control, "
+                        + ("resident step loop)" if resident else "hipGraph replay)"),
             "n": n, "nnz": nnz, "rk_attempts": stats["attempts"],
             "rhs_evals": stats["rhs_evals"], "sell_lanes_per_row": lanes,
             "operator_format": "coded SELL-C" if coded else "SELL-C",
             "autotune": autotune.cache()},
         "err_vs_fp64": float(err),
         "roofline": roof,
+        "launched_stage": stage,
     }
     # the plain SELL-C operator (a value and a column per entry) on the same
     # solve: the same result bits, ten times the operator bytes
@@ -756,11 +798,15 @@ def main():
     # instead of replaying the captured graph (the form the stage kernels'
     # traces are taken in); the same result bits as the timed solve where the
     # lane counts agree (the resident loop has a rule of its own for them)
+    graph_env = os.environ.get("QUTIP_AMD_GRAPH")
     os.environ["QUTIP_AMD_GRAPH"] = "0"
     try:
         dsolver = qa.MESolver(s["H"], s["c_ops"], options=opts)
-    finally:
-        del os.environ["QUTIP_AMD_GRAPH"]
+    finally:  # a traced run sets it for every leg
+        if graph_env is None:
+            del os.environ["QUTIP_AMD_GRAPH"]
+        else:
+            os.environ["QUTIP_AMD_GRAPH"] = graph_env
     dres = dsolver.run(s["psi0"], tlist, e_ops=s["e_ops"])
     _lib.call("qa_device_sync")
     t0 = time.perf_counter()
