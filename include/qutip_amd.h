@@ -253,6 +253,10 @@ int qa_rk_set_hermitian(qa_rk_solver *s, int on);
  * engine try again whose last resident launch gave up.  No reference
  * counterpart. */
 int qa_rk_set_resident(qa_rk_solver *s, int on);
+/* Whether the engine is one of many that run at once (0 by default): 1 keeps
+ * it on the launched loop and its dense stages in workgroups that fit beside
+ * others.  No reference counterpart. */
+int qa_rk_set_shared(qa_rk_solver *s, int on);
 /* *planned: whether the engine's runs (other than single steps) take the
  * resident step loop, planned now if it was not yet.  No reference
  * counterpart. */

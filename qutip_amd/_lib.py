@@ -77,6 +77,7 @@ SIGNATURES = {
     "qa_rk_set_resident": [vp, i32],
     "qa_rk_set_resident_polls": [vp, i32],
     "qa_rk_plan_resident": [vp, P_i32],
+    "qa_rk_set_shared": [vp, i32],
     "qa_rk_get_hermitian": [vp, P_i32],
     "qa_rk_set_dense_shape": [vp, i32, i32, i32],
     "qa_rk_get_dense_shape": [vp, P_i32, P_i32, P_i32],

@@ -160,7 +160,7 @@ def dense_candidates(N, fp32_mfma, herm, default):
 def dense_shape_for(eng, reps=4, rounds=3):
     """The measured best shape for the dense engine ``eng`` in its current
     Hermitian mode (None below MIN_DENSE_TUNE_N or with QUTIP_AMD_NO_TUNE);
-    cached per (N, collapse operators, precision, mode)."""
+    cached per (N, collapse operators, precision, mode, shared or not)."""
     import ctypes as C
 
     from . import _lib
@@ -170,6 +170,8 @@ def dense_shape_for(eng, reps=4, rounds=3):
     herm = eng.hermitian
     nc = len(eng._dense_host[1]) // (N * N) if eng._dense_host[1].size > 1 else 0
     k = f"dense-n{N}-c{nc}-{eng.dense_precision}-{'herm' if herm else 'full'}"
+    if eng.shared:  # other kernels
+        k += "-shared"
     if not _CACHE:
         _load_file()
     if k not in _CACHE:

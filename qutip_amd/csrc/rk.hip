@@ -1767,10 +1767,11 @@ struct qa_rk_solver {
     // engine (a shape it does not take, or a launch that gave up), 1 planned.
     // Runs take it where the environment (QUTIP_AMD_RESIDENT, QUTIP_AMD_GRAPH
     // when the engine is created) and the caller (qa_rk_set_resident) let
-    // them.  res_dev: the device whose resident slot this engine holds while
+    // them, on an engine that is not shared.  res_dev: the device whose resident slot this engine holds while
     // a launch is in flight, or -1.
     int res = -1, res_form = 0, res_dev = -1;
     bool res_env = true, res_on = true;
+    bool shared = false;  // qa_rk_set_shared
     int res_polls = kResPolls;
     long long res_done = 0, res_gave_up = 0;  // launches since the last set_state
     ResArgs rp = {};
@@ -1788,7 +1789,7 @@ namespace {
 
 void res_give(qa_rk_solver *S);
 int res_prepare(qa_rk_solver *S);
-bool res_wanted(const qa_rk_solver *S) { return S->res_env && S->res_on; }
+bool res_wanted(const qa_rk_solver *S) { return S->res_env && S->res_on && !S->shared; }
 
 void fill_epi(EpiArgs &P, qa_rk_solver *S, int i) {
     P.nrows = S->n;
@@ -1903,7 +1904,11 @@ int launch_sparse_stage(qa_rk_solver *S, int i) {
 
 // Groups of waves that share the np products of an upper 16 x 16 tile (ns
 // waves a group), or 0 for one group: where every tile has a CU of its own.
-// At least eight waves, one for each item of the epilogue.
+// At least eight waves, one for each item of the epilogue.  Not for an engine
+// that shares the device: sixteen waves of 128 registers fit only an empty
+// CU, and a launch that waits for one holds up the kernels behind it (a solve
+// server of 64 requests: p50 latency 0.52 -> 1.19 s, sesolve p99 service 0.29
+// -> 1.55 s at the same rate).
 int herm_wide_groups(int tiles, int ns, int np) {
     if (tiles > 256) return 0;
     const int ng = std::min(kMaxWide / ns, np);
@@ -1930,7 +1935,7 @@ int launch_dense_herm_stage(qa_rk_solver *S, const EpiArgs &P) {
                        S->dop);
     QA_CHECK_LAUNCH();
     const dim3 grid(nt * (nt + 1) / 2), block(64 * ns);
-    if (const int ng = herm_wide_groups(nt * (nt + 1) / 2, ns, 2 + S->dop.nc)) {
+    if (const int ng = S->shared ? 0 : herm_wide_groups(nt * (nt + 1) / 2, ns, 2 + S->dop.nc)) {
         QA_DENSE_LAUNCH(S->dop.prec, rk_dense_herm_wide_kernel, grid, dim3(64 * ns * ng), S->stream,
                         P, S->dop, ns);
         QA_CHECK_LAUNCH();
@@ -2779,6 +2784,14 @@ int qa_rk_set_resident(qa_rk_solver *S, int on) {
     QA_REQUIRE(S->res_dev < 0, "qa_rk_set_resident: a run is in progress");
     S->res_on = on != 0;
     if (on && S->res == 0 && S->res_block) S->res = 1;  // after a launch that gave up
+    return QA_OK;
+}
+
+int qa_rk_set_shared(qa_rk_solver *S, int on) {
+    QA_REQUIRE(S != nullptr, "qa_rk_set_shared: null solver");
+    QA_REQUIRE(S->res_dev < 0, "qa_rk_set_shared: a run is in progress");
+    if (S->shared != (on != 0)) S->graph_dirty = true;
+    S->shared = on != 0;
     return QA_OK;
 }
 

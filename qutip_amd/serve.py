@@ -123,10 +123,7 @@ class _Running:
         elif req.kind in ("se", "me"):
             if req.kind == "se":
                 A = -1j * req.H.to_csr()
-                # the launched loop: a resident grid would wait for the CUs
-                # that other requests hold, and a process runs one at a time
-                self.eng = RKEngine(A, "vern7", o["rtol"], o["atol"], o["nsteps"],
-                                    resident=False)
+                self.eng = RKEngine(A, "vern7", o["rtol"], o["atol"], o["nsteps"], shared=True)
                 psi = req.psi0.full().ravel()
                 kinds, fptr, rows, cols, w = self._quadratic(req, psi.size)
                 y0 = psi
@@ -134,7 +131,8 @@ class _Running:
                 cs = [c.full() for c in req.c_ops]
                 Hnh = req.H.full() - 0.5j * sum(c.conj().T @ c for c in cs)
                 self.eng = RKEngine(None, "vern7", o["rtol"], o["atol"], o["nsteps"],
-                                    dense=(Hnh, cs), dense_precision=o.get("dense_precision", "fp32"))
+                                    dense=(Hnh, cs), shared=True,
+                                    dense_precision=o.get("dense_precision", "fp32"))
                 # rho0 = |psi0><psi0| is Hermitian: the upper tiles and their
                 # mirror (mesolve's assume_hermitian_state)
                 self.eng.set_hermitian(True)

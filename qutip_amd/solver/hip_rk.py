@@ -102,7 +102,7 @@ class RKEngine:
     def __init__(self, op, tableau="vern7", rtol=1e-6, atol=1e-8, nsteps=1000, first_step=0.0,
                  min_step=0.0, max_step=0.0, interpolate=True, fp32=False, lanes=None,
                  dense=None, dense_precision="fp32", coded="auto", uniform="auto", td=None,
-                 resident=True):
+                 shared=False):
         """``op``: the sparse generator A (dy/dt = A y), or None with
         ``dense=(H_nh, [c_ops])`` (numpy arrays) for the matrix-form
         Lindblad right-hand side: on MFMA (``dense_precision`` 'fp32',
@@ -120,7 +120,8 @@ class RKEngine:
         ``lanes``: lanes per row, by default the resident step loop's where
         this engine takes that loop, else the tuner's (the sums of a row go
         by lanes, so results of other lane counts round differently).
-        ``resident``: False keeps the launched loop (set_resident)."""
+        ``shared``: this engine is one of many that run at once
+        (qa_rk_set_shared)."""
         tab = TABLEAUS[tableau] if isinstance(tableau, str) else tableau
         self.tableau = tab
         self._a = np.ascontiguousarray(tab["a"], dtype=np.float64)
@@ -192,7 +193,7 @@ class RKEngine:
                 _lib.call("qa_rk_set_coefficients", h, len(parts), _ip(start), _ip(vstart),
                           len(code), _ip(code), len(consts), _dp(consts.view(np.float64)))
 
-            self.lanes = self._create_lanes(create, h, A, False, True, lanes, resident)
+            self.lanes = self._create_lanes(create, h, A, False, True, lanes, shared)
         else:
             if isinstance(op, _data.HipCSR):
                 A = op.to_scipy()
@@ -223,10 +224,11 @@ class RKEngine:
                     _lib.check(rc, "qa_rk_create")
                 self.handle = h
 
-            self.lanes = self._create_lanes(create, h, A, fp32, coded, lanes, resident)
+            self.lanes = self._create_lanes(create, h, A, fp32, coded, lanes, shared)
         self.handle = h
-        if not resident:
-            self.set_resident(False)
+        self.shared = bool(shared)
+        if shared:
+            _lib.call("qa_rk_set_shared", h, 1)
         self.nfun = 0
         # entries between consecutive states in a states_out buffer
         self.npad = self.sell.nslices * (64 // self.lanes) if self.sell is not None else self.n
@@ -240,11 +242,11 @@ class RKEngine:
             self.handle = None
 
     @staticmethod
-    def _create_lanes(create, h, A, fp32, coded, lanes, resident):
+    def _create_lanes(create, h, A, fp32, coded, lanes, shared):
         """create(lanes) and the lane count: the resident step loop's only
         where the engine then plans that loop (tableau, LDS, device), else the
         tuner's for the launched loop."""
-        if lanes is None and resident:
+        if lanes is None and not shared:
             lanes = autotune.resident_lanes(A, coded)
             if lanes is not None:
                 create(lanes)

@@ -17,8 +17,9 @@ from qutip_amd.solver.hip_rk import RKEngine  # noqa: E402
 from tests.test_gpu_dense_herm import _system, _trace_functionals  # noqa: E402
 
 
-def _solve(Hnh, cs, rho0, tl, prec, herm, ops, shape):
-    eng = RKEngine(None, "vern7", 1e-6, 1e-8, dense=(Hnh, cs), dense_precision=prec)
+def _solve(Hnh, cs, rho0, tl, prec, herm, ops, shape, shared=False):
+    eng = RKEngine(None, "vern7", 1e-6, 1e-8, dense=(Hnh, cs), dense_precision=prec,
+                   shared=shared)
     eng.set_hermitian(herm)
     if shape is not None:
         eng.dense_shape = (shape[0], eng.dense_shape[1], shape[1])
@@ -39,10 +40,22 @@ def _solve(Hnh, cs, rho0, tl, prec, herm, ops, shape):
 @pytest.mark.parametrize("prec", ["fp32", "bf16x6"])
 def test_shared_products_match_full_rhs(N, nc, tiled, hsplit, prec):
     print(f"dense groups N={N} nc={nc} tiled={tiled} hsplit={hsplit} {prec}", flush=True)
+    _check(N, nc, tiled, hsplit, prec, False)
+
+
+@pytest.mark.parametrize("N,nc,hsplit", [(32, 6, 1), (64, 3, 2), (128, 2, 4), (256, 1, 8),
+                                         (352, 3, 1)])
+@pytest.mark.parametrize("prec", ["fp32", "bf16x6"])
+def test_one_group_of_a_shared_engine_matches_full_rhs(N, nc, hsplit, prec):
+    print(f"dense, shared engine N={N} nc={nc} hsplit={hsplit} {prec}", flush=True)
+    _check(N, nc, 0, hsplit, prec, True)
+
+
+def _check(N, nc, tiled, hsplit, prec, shared):
     H, cs, Hnh, rho0 = _system(N, 3 + N + nc, nc)
     tl = np.linspace(0, 0.1, 3)
     ops = [H, np.diag(np.arange(N) / N).astype(complex)]
-    (vh, yh), (v2, y2) = _solve(Hnh, cs, rho0, tl, prec, True, ops, (tiled, hsplit))
+    (vh, yh), (v2, y2) = _solve(Hnh, cs, rho0, tl, prec, True, ops, (tiled, hsplit), shared)
     (vf, yf), _ = _solve(Hnh, cs, rho0, tl, prec, False, ops, None)
     assert np.array_equal(vh, v2) and np.array_equal(yh, y2)
     assert np.array_equal(yh, yh.conj().T)

@@ -309,7 +309,7 @@ def test_resident_gives_up(n, lanes, form, polls):
 
 def test_resident_lanes_only_for_its_engines(monkeypatch):
     """The resident loop's lane count goes to engines that take that loop: not
-    to one kept on the launched loop, nor to a tableau it refuses (here one
+    to one of many that run at once, nor to a tableau it refuses (here one
     whose first stage is not at the step's start)."""
     print("resident lanes", flush=True)
     monkeypatch.setenv("QUTIP_AMD_NO_TUNE", "1")
@@ -317,18 +317,18 @@ def test_resident_lanes_only_for_its_engines(monkeypatch):
     launched, ruled = autotune.lanes_for(A), autotune.resident_lanes(A)
     assert launched != ruled
     off = dict(TABLEAUS["tsit5"], c=np.asarray(TABLEAUS["tsit5"]["c"]) + 0.01)
-    for kw, lanes in (({}, ruled), ({"resident": False}, launched), ({"tableau": off}, launched),
+    for kw, lanes in (({}, ruled), ({"shared": True}, launched), ({"tableau": off}, launched),
                       ({"lanes": 8}, 8)):
         eng = RKEngine(A, rtol=1e-6, atol=1e-8, coded=False, **kw)
         assert eng.lanes == eng.sell.lanes == lanes
         if "tableau" not in kw:
             eng.set_state(0.0, _state(5000, np.random.default_rng(2)))
             eng.run([0.01])
-            assert (eng.stats()["resident_launches"] > 0) == (kw != {"resident": False})
+            assert (eng.stats()["resident_launches"] > 0) == (kw != {"shared": True})
     m = systems.ising(3, 0.1)
     H = qa.QobjEvo([m["H"], [m["e_ops"][0], "cos(t)"]])
     td = time_dependent_operator(qa.MESolver(H, m["c_ops"]).rhs.matmul_data)
-    for kw in ({}, {"resident": False}):
+    for kw in ({}, {"shared": True}):
         eng = RKEngine(None, rtol=1e-6, atol=1e-8, td=td, **kw)
         eng.set_state(0.0, _state(64, np.random.default_rng(2)))
         eng.run([0.01])
