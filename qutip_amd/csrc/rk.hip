@@ -593,7 +593,7 @@ __global__ __launch_bounds__(64 * kMaxSplit) void rk_dense_stage_kernel(EpiArgs 
 // serves two waves.  All products of a workgroup run through one flattened
 // chunk loop, so one memory latency is exposed per stage.  Chunks of 64 take
 // 137 KB of LDS, one workgroup a CU, whose waves all wait at once; with 32
-// two fit (69 KB): C_c X in FP32 for N = 512, nc = 3 went from 51 to 29 us.
+// two fit (69 KB): C_c X in FP32 for N = 512, nc = 3 went from 51 to 39 us.
 // The bf16 splits need more registers than two workgroups a CU leave, and
 // keep 64 (with 32 they were 3 to 5 % slower).  Used for
 // N >= kTiledN, where the one-tile-per-workgroup kernels above re-read every
@@ -1184,7 +1184,7 @@ __device__ __forceinline__ float2 part_load(const float2 *p) {
 // tile: each takes some of its products and stores its sum, and the one that
 // arrives last adds the sums in their order and does the epilogue.  One
 // workgroup a tile left 120 of 256 CUs idle at N = 512 (136 tiles): 78 us a
-// stage, 39 with five (nc = 3); a whole solve 31.7 -> 25.4 ms, at N = 384
+// stage, 53 with five (nc = 3); a whole solve 31.7 -> 25.4 ms, at N = 384
 // 18.0 -> 14.2.  Two workgroups a CU need at most 128 registers (FP32).
 template <int NP>
 __global__ __launch_bounds__(256 * kGHalves, NP == 0 ? 4 : 2) void rk_dense_herm_stage_tiled_kernel(EpiArgs P,
